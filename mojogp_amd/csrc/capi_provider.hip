@@ -360,7 +360,7 @@ int mgp_direct_matvec(void* h, const float* V, int ncols, float* out) {
     a.square = true;
     a.m = a.n = pv->n;
     a.ncols = ncols;
-    direct_matvec(a, pv->train, pv->train, pv->d, dv, dout, pv->st);
+    direct_matvec(a, pv->train, pv->train, pv->d, dv, dout, pv->ws, pv->st);
     MGP_HIP_CHECK(hipMemcpyAsync(out, dout, tot * sizeof(float), hipMemcpyDeviceToHost, pv->st));
     MGP_HIP_CHECK(hipStreamSynchronize(pv->st));
   });

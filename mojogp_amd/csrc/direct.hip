@@ -1,0 +1,340 @@
+// Kernel-matrix products from per-dimension differences of the scaled
+// coordinates (no Gram form): Matern-1/2, point sets whose norms exceed the
+// Gram bound, and input dimensions beyond the tile path.
+//
+// Reference behaviour (caspbian/mojogp):
+//   fused_forward_matvec_ncols  mojogp/codegen_engine/emit/gpu_kernel.py:151-260
+//   fused_cross_matvec_ncols    mojogp/codegen_engine/emit/gpu_kernel.py:487-565
+//
+// Per pair 2 d + ~5 VALU instructions form the value, which enters the product
+// with the right-hand sides as an operand of the fp32 matrix cores
+// (v_mfma_f32_16x16x4_f32: the values keep their 24 bits, so a product is as
+// accurate as one accumulated on the VALU) or, for up to 4 right-hand sides,
+// VALU FMAs.  Issue bound: at d = 5 the value costs ~62 cycles per 64 pairs
+// and the matrix instruction 32, ~250 us for n = 20011 one-sided; measured 313
+// to 330 us with the reduction (11 right-hand sides, Matern-1/2) against 18.7
+// ms for one row per thread with every product added in fp64 (79 workgroups,
+// run-time dimension loops).  Splitting the values for the 16-bit matrix cores
+// would shorten the matrix part but costs accuracy that these products had.
+#include "kval.h"
+#include "matvec.h"
+
+#include <algorithm>
+#include <vector>
+
+namespace mgp {
+
+namespace {
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+constexpr int kDiffTile = 64;    // column points per LDS tile
+constexpr int kDiffWaves = 4;    // waves per workgroup
+
+// Right-hand sides a kernel form carries: VALU forms 1 and 4, matrix-core
+// forms 16 and 64.
+enum DiffForm { kDiff1 = 0, kDiff4, kDiff16, kDiff64, kDiffForms };
+constexpr int kDiffCols[kDiffForms] = {1, 4, 16, 64};
+
+// 16-row tiles per wave: row coordinates (R x D) and accumulators stay in
+// registers with at least 3 waves per SIMD (n = 30000, 16 right-hand sides:
+// d = 16 1.12 ms with 4, 1.03 ms with 2; d = 5 at n = 20011 332 and 344 us).
+constexpr int diff_rows(int D, int form) {
+  return D > 10 || form == kDiff64 ? 2 : 4;
+}
+
+// os tot + noise v in fp64, rounded once (v = 0 where no noise is added).
+__device__ __forceinline__ float diff_epilogue(double tot, float os, float noise, float v) {
+  return (float)((double)os * tot + (double)noise * (double)v);
+}
+
+// Sums over the columns [y tps 64, (y + 1) tps 64) of split y, for rows
+// i0 + 16 r + lane%16 of each wave.  Step s of a column tile: lane l evaluates
+// the pairs (row 16 r + l%16, column 4 s + l/16), r < R, from one LDS read of
+// the column point; they are the A operand of v_mfma_f32_16x16x4_f32 with
+// B = V[column][l%16], whose result holds rows 16 r + 4 (l/16) + q of
+// right-hand side l%16.  fp32 within a tile (64 columns), fp64 across tiles.
+// part != nullptr: part[(y nc + c) m + i] = the fp64 sums; else (one split)
+// the epilogue out = os sum (+ noise V).
+template <int KIND, int D, int FORM>
+__global__ __launch_bounds__(64 * kDiffWaves) void k_diff_tile(
+    const float* __restrict__ Zr, int64_t m, const float* __restrict__ Zc, int64_t n, int d,
+    const float* __restrict__ V, int nc, int64_t tps, float os, float noise, int add_noise,
+    float lim, double* __restrict__ part, float* __restrict__ out) {
+  constexpr int R = diff_rows(D, FORM);
+  constexpr bool MFMA = FORM >= kDiff16;
+  constexpr int NC = kDiffCols[FORM];
+  constexpr int G = MFMA ? NC / 16 : 1;          // 16-column groups
+  constexpr int DS = D <= 2 ? D : (D + 3) / 4 * 4;  // LDS stride of a column point
+  __shared__ __align__(16) float sx[kDiffTile * DS];
+  __shared__ __align__(16) float sv[kDiffTile * NC];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lm = lane & 15, lq = lane >> 4;
+  const int64_t i0 = ((int64_t)blockIdx.x * kDiffWaves + wave) * (16 * R);
+
+  float xi[R][D];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int64_t i = i0 + 16 * r + lm;
+#pragma unroll
+    for (int k = 0; k < D; ++k) xi[r][k] = (i < m && k < d) ? Zr[i * d + k] : 0.0f;
+  }
+  // fp64 sums: MFMA form [r][g][q], VALU form [r][c] of this lane's columns
+  constexpr int NA = MFMA ? 4 * G : NC;
+  double accd[R][NA];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int a = 0; a < NA; ++a) accd[r][a] = 0.0;
+
+  const int64_t tiles = (n + kDiffTile - 1) / kDiffTile;
+  const int64_t t0 = (int64_t)blockIdx.y * tps, t1 = min(tiles, t0 + tps);
+  for (int64_t t = t0; t < t1; ++t) {
+    const int64_t j0 = t * kDiffTile;
+    const int cnt = (int)min((int64_t)kDiffTile, n - j0);
+    __syncthreads();
+    // columns past n: zero coordinates and zero right-hand sides
+    for (int q = threadIdx.x; q < kDiffTile * D; q += 64 * kDiffWaves) {
+      const int jj = q / D, k = q - jj * D;
+      sx[jj * DS + k] = (jj < cnt && k < d) ? Zc[(j0 + jj) * d + k] : 0.0f;
+    }
+    for (int q = threadIdx.x; q < kDiffTile * NC; q += 64 * kDiffWaves) {
+      const int c = q / kDiffTile, jj = q - c * kDiffTile;
+      sv[jj * NC + c] = (jj < cnt && c < nc) ? V[(int64_t)c * n + j0 + jj] : 0.0f;
+    }
+    __syncthreads();
+    // fp32 within the tile, fp64 across tiles
+    float acc[R][NA];
+    f4 am[R][G];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+#pragma unroll
+      for (int a = 0; a < NA; ++a) acc[r][a] = 0.0f;
+#pragma unroll
+      for (int g = 0; g < G; ++g) am[r][g] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    const int steps = (cnt + 3) / 4;
+#pragma unroll 2
+    for (int s = 0; s < steps; ++s) {
+      const int jj = 4 * s + lq;
+      float xj[DS];
+      if constexpr (D <= 2) {
+#pragma unroll
+        for (int k = 0; k < D; ++k) xj[k] = sx[jj * DS + k];
+      } else {
+#pragma unroll
+        for (int k = 0; k < DS; k += 4) {
+          const f4 x = *reinterpret_cast<const f4*>(&sx[jj * DS + k]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) xj[k + e] = x[e];
+        }
+      }
+      float v[MFMA ? G : NC];
+      if constexpr (MFMA) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) v[g] = sv[jj * NC + 16 * g + lm];
+      } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[c] = sv[jj * NC + c];
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float r2 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+          const float df = xi[r][k] - xj[k];
+          r2 = fmaf(df, df, r2);
+        }
+        const float kv = kval<KIND>(r2, lim);
+        if constexpr (MFMA) {
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+            am[r][g] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv, v[g], am[r][g], 0, 0, 0);
+        } else {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) acc[r][c] = fmaf(kv, v[c], acc[r][c]);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if constexpr (MFMA) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) accd[r][4 * g + q] += (double)am[r][g][q];
+      } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) accd[r][c] += (double)acc[r][c];
+      }
+    }
+  }
+
+  auto put = [&](int c, int64_t i, double tot) __attribute__((always_inline)) {
+    if (c >= nc || i >= m) return;
+    if (part) {
+      part[((int64_t)blockIdx.y * nc + c) * m + i] = tot;
+    } else {
+      out[(int64_t)c * m + i] =
+          diff_epilogue(tot, os, noise, add_noise ? V[(int64_t)c * m + i] : 0.0f);
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if constexpr (MFMA) {
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) put(16 * g + lm, i0 + 16 * r + 4 * lq + q, accd[r][4 * g + q]);
+    } else {
+      // the four lane groups hold the row's columns 4 s + l/16: fold them
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        double tot = accd[r][c];
+        tot += __shfl_xor(tot, 16);
+        tot += __shfl_xor(tot, 32);
+        if (lq == 0) put(c, i0 + 16 * r + lm, tot);
+      }
+    }
+  }
+}
+
+// out[c][i] = os sum_y part[y][c][i] (+ noise V[c][i]), splits in order.
+__global__ void k_diff_reduce(const double* __restrict__ part, int splits, int64_t total,
+                              float os, float noise, int add_noise, const float* __restrict__ V,
+                              float* __restrict__ out) {
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= total) return;
+  double tot = 0.0;
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s) tot += part[(int64_t)s * total + idx];
+  out[idx] = diff_epilogue(tot, os, noise, add_noise ? V[idx] : 0.0f);
+}
+
+using DiffFn = void (*)(const float*, int64_t, const float*, int64_t, int, const float*, int,
+                        int64_t, float, float, int, float, double*, float*);
+
+struct DiffKernel {
+  DiffFn fn;
+  int rows;  // rows per workgroup
+};
+
+// Every dimension up to 6, then the steps at which a padded dimension costs
+// at most a quarter of the value's instructions.
+template <int KIND, int FORM>
+DiffKernel pick_diff_d(int d) {
+#define MGP_DIFF_CASE(DV) \
+  if (d <= DV) return {k_diff_tile<KIND, DV, FORM>, 16 * diff_rows(DV, FORM) * kDiffWaves};
+  MGP_DIFF_CASE(1)
+  MGP_DIFF_CASE(2)
+  MGP_DIFF_CASE(3)
+  MGP_DIFF_CASE(4)
+  MGP_DIFF_CASE(5)
+  MGP_DIFF_CASE(6)
+  MGP_DIFF_CASE(8)
+  MGP_DIFF_CASE(10)
+  MGP_DIFF_CASE(12)
+  MGP_DIFF_CASE(16)
+  MGP_DIFF_CASE(20)
+  MGP_DIFF_CASE(24)
+  MGP_DIFF_CASE(32)
+#undef MGP_DIFF_CASE
+  return {nullptr, 0};
+}
+
+template <int KIND>
+DiffKernel pick_diff_form(int form, int d) {
+  switch (form) {
+    case kDiff1: return pick_diff_d<KIND, kDiff1>(d);
+    case kDiff4: return pick_diff_d<KIND, kDiff4>(d);
+    case kDiff16: return pick_diff_d<KIND, kDiff16>(d);
+    default: return pick_diff_d<KIND, kDiff64>(d);
+  }
+}
+
+DiffKernel pick_diff(int kind, int form, int d) {
+  switch (kind) {
+    case KIND_RBF: return pick_diff_form<KIND_RBF>(form, d);
+    case KIND_MATERN12: return pick_diff_form<KIND_MATERN12>(form, d);
+    case KIND_MATERN32: return pick_diff_form<KIND_MATERN32>(form, d);
+    default: return pick_diff_form<KIND_MATERN52>(form, d);
+  }
+}
+
+// Column splits of a launch of row_blocks workgroups: the chip holds `slots`
+// workgroups at once, so a launch takes ceil(blocks / slots) rounds of
+// (tiles per split + about half a tile of set-up); every split's fp64 partials
+// are written once and read once (about 1/40 of a tile's time per split and
+// slot-filling of rows, which only keeps tiny splits apart).
+int64_t diff_splits(int64_t row_blocks, int64_t tiles, int64_t slots) {
+  int64_t best = 1;
+  double best_cost = 0.0;
+  for (int64_t s = 1; s <= std::min<int64_t>(tiles, 64); ++s) {
+    const int64_t tps = ceil_div(tiles, s);
+    if (s > 1 && ceil_div(tiles, s - 1) == tps) continue;
+    const int64_t real = ceil_div(tiles, tps);
+    const double rounds = (double)ceil_div(row_blocks * real, slots);
+    const double cost =
+        rounds * ((double)tps + 0.5) + 0.025 * (double)real * (double)row_blocks / 64.0;
+    if (s == 1 || cost < best_cost) {
+      best_cost = cost;
+      best = real;
+    }
+  }
+  return best;
+}
+
+}  // namespace
+
+void direct_matvec(const MatvecArgs& a, const PackedPoints& rows, const PackedPoints& cols, int d,
+                   const float* V_dev, float* out_dev, MatvecWorkspace& ws, hipStream_t st) {
+  MGP_REQUIRE(d >= 1 && d <= 32, "direct path supports input dimension <= 32");
+  if (a.m <= 0 || a.ncols <= 0) return;
+  int dev = 0, cus = 0;
+  MGP_HIP_CHECK(hipGetDevice(&dev));
+  MGP_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const int64_t tiles = ceil_div(std::max<int64_t>(a.n, 1), kDiffTile);
+  for (int c0 = 0; c0 < a.ncols;) {
+    // up to 4 columns on the VALU (a value then costs at most 4 FMAs against
+    // the 32 cycles of its matrix instruction), up to 16 in one matrix
+    // group; four groups share the values of a wider product
+    const int left = a.ncols - c0;
+    const int form = left == 1 ? kDiff1 : left <= 4 ? kDiff4 : left <= 16 ? kDiff16 : kDiff64;
+    const int nc = std::min(kDiffCols[form], left);
+    const DiffKernel k = pick_diff(a.kind, form, d);
+    MGP_REQUIRE(k.fn != nullptr, "no difference kernel for this shape");
+    const int64_t row_blocks = ceil_div(a.m, k.rows);
+    int per_cu = 0;
+    MGP_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &per_cu, reinterpret_cast<const void*>(k.fn), 64 * kDiffWaves, 0));
+    int64_t splits =
+        diff_splits(row_blocks, tiles, (int64_t)std::max(cus, 1) * std::max(per_cu, 1));
+    const int64_t total = (int64_t)nc * a.m;
+    double* part = nullptr;
+    if (ws.arena != nullptr) {
+      // fixed arena: as many splits as its bytes hold, unsplit without partials
+      splits = std::min<int64_t>(splits, (int64_t)(ws.arena_bytes / (sizeof(double) * total)));
+      if (splits > 1) part = reinterpret_cast<double*>(ws.arena);
+    } else if (splits > 1) {
+      part = ws.direct_part.ensure((size_t)splits * total);
+    }
+    const int64_t tps = ceil_div(tiles, std::max<int64_t>(splits, 1));
+    splits = ceil_div(tiles, tps);
+    const float* Vc = V_dev + (int64_t)c0 * a.n;
+    float* outc = out_dev + (int64_t)c0 * a.m;
+    const int add = a.square ? 1 : 0;
+    hipLaunchKernelGGL(k.fn, dim3((unsigned)row_blocks, (unsigned)splits), dim3(64 * kDiffWaves),
+                       0, st, rows.z.ptr, a.m, cols.z.ptr, a.n, d, Vc, nc, tps, a.outputscale,
+                       a.noise, add, cols.exp2_limit, part, outc);
+    MGP_HIP_CHECK(hipGetLastError());
+    if (part) {
+      hipLaunchKernelGGL(k_diff_reduce, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st,
+                         part, (int)splits, total, a.outputscale, a.noise, add, Vc, outc);
+      MGP_HIP_CHECK(hipGetLastError());
+    }
+    c0 += nc;
+  }
+}
+
+}  // namespace mgp

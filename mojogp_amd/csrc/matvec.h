@@ -141,6 +141,7 @@ struct MatvecWorkspace {
   DevBuf<uint32_t> colmax_part;  // [64][chunks] row-chunk maxima
   DevBuf<float> partial;  // split-K partial sums
   DevBuf<float> sym_tp;   // transposed partial sums of the symmetric product
+  DevBuf<double> direct_part;  // split partial sums of the difference product
   // Fixed-arena mode (allocation-free callers): when arena is set, every work
   // buffer above is carved from [arena, arena + arena_bytes) instead of being
   // grown with hipMalloc; the split count is capped so the partial sums fit,
@@ -177,11 +178,12 @@ constexpr double kSymMaxBytes = 16e9;
 size_t fused_matvec_min_arena(const PackedPoints& cols, int ncols);
 
 // Reference-form product evaluated per pair from per-dimension differences of
-// the scaled coordinates (no Gram form, no MFMA).  Used as an independent
+// the scaled coordinates (no Gram form; direct.hip).  Used as an independent
 // device cross-check and for dimensions beyond the MFMA tile path.
+// Split partials come from ws (its fixed arena when it has one).
 void direct_matvec(const MatvecArgs& a, const PackedPoints& rows,
                    const PackedPoints& cols, int d, const float* V_dev,
-                   float* out_dev, hipStream_t st);
+                   float* out_dev, MatvecWorkspace& ws, hipStream_t st);
 
 // Dense block of K(rows, cols): out[c*cols.n + i] = os k(row r0 + c, col i),
 // c < nrows, from per-dimension differences of the scaled coordinates

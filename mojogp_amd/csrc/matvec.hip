@@ -19,6 +19,7 @@
 // (512 in the symmetric kernel) so the long N-term sums keep ~1e-7 relative
 // accuracy.
 #include "dense.h"
+#include "kval.h"
 #include "matvec.h"
 #include "sym_common.h"
 
@@ -48,48 +49,12 @@ constexpr int kFlushTiles = 16;     // j tiles between fp64 flushes
 // s_waitcnt immediate for vmcnt(0) with expcnt and lgkmcnt left free (gfx9
 // encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
 constexpr int kWaitVmcnt0 = 0x0F70;
-constexpr float kM52A = 0.69314718055994530942f;                     // ln 2
-constexpr float kM52B = 0.69314718055994530942f * 0.69314718055994530942f / 3.0f;
 
 // kExp2Clamp held in a VGPR (hoisted out of the hot loop by the caller).
 __device__ __forceinline__ float clamp_reg() {
   float c = kExp2Clamp;
   asm volatile("" : "+v"(c));
   return c;
-}
-
-// Kernel value from the scaled squared distance s (see kernel_scale()).
-// clampv = the exponent limit exp2_limit(kind, ard) (kExp2Clamp, from
-// clamp_reg() in hot loops, for the Matern-3/2 and 5/2 kernels; the point
-// set's exp2_limit for Matern-1/2; RBF has none).
-template <int KIND>
-__device__ __forceinline__ float kval(float s, float clampv = kExp2Clamp) {
-  if constexpr (KIND == KIND_RBF) {
-    // os * exp(-0.5 r^2) = os * 2^-max(s, 0) (the max only absorbs Gram-form
-    // rounding below zero; the reference does not clamp the RBF exponent)
-    return __builtin_amdgcn_exp2f(-fmaxf(s, 0.0f));
-  } else if constexpr (KIND == KIND_MATERN12) {
-    // os * exp(-r) (isotropic) or os * exp(max(-r, -20)) (ARD),  u = r log2 e
-    const float u = __builtin_amdgcn_sqrtf(fabsf(s));
-    return __builtin_amdgcn_exp2f(-fminf(u, clampv));
-  } else if constexpr (KIND == KIND_MATERN32) {
-    // os * (1 + sqrt3 r) * exp(max(-sqrt3 r, -20)),  u = sqrt3 r log2 e
-    const float u = __builtin_amdgcn_sqrtf(fabsf(s));
-    return fmaf(u, kLn2, 1.0f) * __builtin_amdgcn_exp2f(-fminf(u, clampv));
-  } else {
-    // os * (1 + sqrt5 r + 5/3 r^2) * exp(max(-sqrt5 r, -20)),  u = sqrt5 r log2 e
-    // sqrt(|s|): s < 0 only from Gram-form rounding of a near-zero distance,
-    // where |s| and max(s, 0) agree to the rounding error (dk/du = 0 at u = 0);
-    // the abs is a free source modifier of v_sqrt_f32.
-    const float u = __builtin_amdgcn_sqrtf(fabsf(s));
-    // min(u, C) kept opaque so that the negation is not rewritten into
-    // max(-u, -C) + v_xor but lands on v_exp_f32 as a source modifier.
-    float m = fminf(u, clampv);
-    asm("" : "+v"(m));
-    const float e = __builtin_amdgcn_exp2f(-m);
-    const float p = fmaf(u, fmaf(u, kM52B, kM52A), 1.0f);
-    return p * e;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1692,56 +1657,6 @@ __global__ void k_reduce_mix4(const float* __restrict__ partial, int splits, int
   }
 }
 
-// ---------------------------------------------------------------------------
-// Direct (per-dimension difference) product: one thread per row, LDS tiles of
-// column points.  Arithmetic follows the reference order: r^2 = sum_d diff^2.
-// ---------------------------------------------------------------------------
-constexpr int kDirectTile = 128;
-constexpr int kDirectMaxCols = 16;
-
-template <int KIND>
-__global__ __launch_bounds__(256) void k_direct(
-    const float* __restrict__ Zr, int64_t m, const float* __restrict__ Zc,
-    int64_t n, int d, const float* __restrict__ V, int ncols, float os,
-    float noise, int add_noise, float lim, float* __restrict__ out) {
-  extern __shared__ float sm[];  // [kDirectTile][d + ncols]
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int w = d + ncols;
-  float xi[32];
-  for (int k = 0; k < d; ++k) xi[k] = (i < m) ? Zr[i * d + k] : 0.0f;
-  double acc[kDirectMaxCols];
-  for (int c = 0; c < kDirectMaxCols; ++c) acc[c] = 0.0;
-  for (int64_t j0 = 0; j0 < n; j0 += kDirectTile) {
-    __syncthreads();
-    for (int t = threadIdx.x; t < kDirectTile * w; t += blockDim.x) {
-      const int jj = t / w, k = t - jj * w;
-      const int64_t j = j0 + jj;
-      float val = 0.0f;
-      if (j < n) val = (k < d) ? Zc[j * d + k] : V[(int64_t)(k - d) * n + j];
-      sm[t] = val;
-    }
-    __syncthreads();
-    const int cnt = (int)min((int64_t)kDirectTile, n - j0);
-    for (int jj = 0; jj < cnt; ++jj) {
-      const float* row = sm + jj * w;
-      float r2 = 0.0f;
-      for (int k = 0; k < d; ++k) {
-        const float df = xi[k] - row[k];
-        r2 = fmaf(df, df, r2);
-      }
-      const float kv = kval<KIND>(r2, lim);
-      for (int c = 0; c < ncols; ++c) acc[c] += (double)(kv * row[d + c]);
-    }
-  }
-  if (i < m) {
-    for (int c = 0; c < ncols; ++c) {
-      float o = os * (float)acc[c];
-      if (add_noise) o = fmaf(noise, V[(int64_t)c * m + i], o);
-      out[(int64_t)c * m + i] = o;
-    }
-  }
-}
-
 // Dense cross-covariance block: out[c*n + i] = os * k(zr[r0 + c], zc[i]) for
 // c < rows, i < n, from per-dimension differences (reference arithmetic).
 template <int KIND>
@@ -2477,25 +2392,6 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
                            a.outputscale, a.noise, a.square ? 1 : 0, Vin, outc);
       MGP_HIP_CHECK(hipGetLastError());
     }
-  }
-}
-
-void direct_matvec(const MatvecArgs& a, const PackedPoints& rows,
-                   const PackedPoints& cols, int d, const float* V_dev,
-                   float* out_dev, hipStream_t st) {
-  MGP_REQUIRE(d >= 1 && d <= 32, "direct path supports input dimension <= 32");
-  for (int c0 = 0; c0 < a.ncols; c0 += kDirectMaxCols) {
-    const int nc = std::min(kDirectMaxCols, a.ncols - c0);
-    const size_t shm = (size_t)kDirectTile * (d + nc) * sizeof(float);
-    const dim3 grid((unsigned)ceil_div(std::max<int64_t>(a.m, 1), 256));
-    auto fn = a.kind == KIND_RBF        ? k_direct<KIND_RBF>
-              : a.kind == KIND_MATERN12 ? k_direct<KIND_MATERN12>
-              : a.kind == KIND_MATERN32 ? k_direct<KIND_MATERN32>
-                                        : k_direct<KIND_MATERN52>;
-    hipLaunchKernelGGL(fn, grid, dim3(256), shm, st, rows.z.ptr, a.m, cols.z.ptr,
-                       a.n, d, V_dev + (int64_t)c0 * a.n, nc, a.outputscale,
-                       a.noise, a.square ? 1 : 0, cols.exp2_limit, out_dev + (int64_t)c0 * a.m);
-    MGP_HIP_CHECK(hipGetLastError());
   }
 }
 

@@ -227,7 +227,7 @@ void Provider::forward_scalar(const float* V, int ncols, float* out, MatvecWorks
     return;
   }
   if (!gram_form_ok(kind, train, train)) {
-    direct_matvec(a, train, train, d, V, out, st);
+    direct_matvec(a, train, train, d, V, out, wsp ? *wsp : ws, st);
     return;
   }
   fused_matvec(a, train, train, V, out, wsp ? *wsp : ws, st);
@@ -275,7 +275,7 @@ void Provider::cross(const PackedPoints& rows, const float* V, int ncols,
   a.n = n;
   a.ncols = ncols;
   if (!gram_form_ok(kind, rows, train)) {
-    direct_matvec(a, rows, train, d, V, out, st);
+    direct_matvec(a, rows, train, d, V, out, ws, st);
     return;
   }
   fused_matvec(a, rows, train, V, out, ws, st);

@@ -1,0 +1,89 @@
+"""Difference products (direct.hip) at the edges of their tiles: 64-column LDS
+tiles, 128- or 256-row workgroups, the 1 / 4 / 16 / 64 right-hand-side forms
+and every padded input dimension, against the float64 oracle; the fixed-arena
+call (splits cut to what the array holds) against the allocating one.
+
+Bound: every product term carries a kernel value within a few fp32 ulps of
+r^2 and of the exponent (u <= 20 log2 e scaled by 2^-24 each), so the normwise
+error stays below 2e-6 for lengthscales of the order of the data."""
+
+import numpy as np
+import pytest
+
+from mojogp_amd._provider import NativeProvider
+from oracle import kernels as ok
+
+pytestmark = pytest.mark.gpu
+
+KINDS = [ok.RBF, ok.MATERN52, ok.MATERN12, ok.MATERN32]
+
+
+def _err(a, b):
+    b = np.asarray(b, np.float64)
+    return float(np.linalg.norm(np.asarray(a, np.float64) - b) / max(np.linalg.norm(b), 1e-30))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n,d,t", [(1, 1, 1), (63, 2, 4), (64, 3, 5), (65, 4, 16), (257, 7, 17),
+                                   (300, 9, 64), (511, 11, 65), (640, 17, 3), (1000, 31, 11),
+                                   (1025, 32, 33)])
+def test_edges(kind, n, d, t):
+    rng = np.random.default_rng(1000 * kind + n + d)
+    X = rng.normal(size=(n, d)).astype(np.float32)
+    Xs = rng.normal(size=(max(1, n // 3), d)).astype(np.float32)
+    V = rng.normal(size=(t, n)).astype(np.float32)
+    params = np.concatenate([rng.uniform(0.7, 1.4, d) * np.sqrt(d), [1.2]]).astype(np.float32)
+    print(f"kind={kind} n={n} d={d} t={t}", flush=True)
+    p = NativeProvider(kind, True, X, params, 0.1)
+    try:
+        got = p.direct_matvec(V)
+        cross = p.cross_matvec(Xs, V) if kind == ok.MATERN12 else None
+    finally:
+        p.close()
+    assert _err(got, ok.forward_matvec(kind, X, V, params, 0.1, True)) <= 2e-6
+    if cross is not None:
+        assert _err(cross, ok.cross_matvec(kind, Xs, X, V, params, True)) <= 2e-6
+
+
+def test_columns_are_independent():
+    """A right-hand side's result does not depend on the others' values."""
+    rng = np.random.default_rng(3)
+    n = 700
+    X = rng.normal(size=(n, 3)).astype(np.float32)
+    V = rng.normal(size=(6, n)).astype(np.float32)
+    W = V.copy()
+    W[3] = np.inf
+    p = NativeProvider(ok.MATERN12, False, X, np.array([1.0, 1.0], np.float32), 0.1)
+    try:
+        a, b = p.forward_matvec(V), p.forward_matvec(W)
+    finally:
+        p.close()
+    keep = [0, 1, 2, 4, 5]
+    assert np.array_equal(a[keep], b[keep])
+    assert not np.isfinite(b[3]).any()
+
+
+@pytest.mark.parametrize("n,t", [(2000, 11), (300001, 16)])
+def test_fixed_arena(n, t):
+    """mgp_forward_matvec_device_noalloc on the difference route: split
+    partials inside the fixed array, none where not even two splits fit
+    (300001 x 16 fp64 sums)."""
+    from mojogp_amd import _lib
+    from test_zz_no_alloc import _Dev, _hip
+    hip = _hip()
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(n, 1)).astype(np.float32)
+    V = rng.normal(size=(t, n)).astype(np.float32)
+    src, dst = _Dev(hip, V.nbytes), _Dev(hip, V.nbytes)
+    src.put(V)
+    p = NativeProvider(ok.MATERN12, False, X, np.array([0.7, 1.0], np.float32), 0.1)
+    try:
+        _lib.call("mgp_forward_matvec_device", p.handle, src.ptr, t, dst.ptr)
+        want = dst.get(V.shape)
+        _lib.call("mgp_forward_matvec_device_noalloc", p.handle, src.ptr, t, dst.ptr)
+        got = dst.get(V.shape)
+    finally:
+        p.close()
+        src.free()
+        dst.free()
+    assert _err(got, want) <= 2e-7  # the same fp64 sums in another order, rounded once
