@@ -366,10 +366,21 @@ __global__ void k_tree_part_sum(const double* __restrict__ part, int64_t nblk, i
   if (lane == 0) acc[q] = accumulate ? acc[q] + s : s;
 }
 
+// Column splits of the interpreted traces: one 64-column LDS tile at least
+// (a pair takes a thread ~6 us, so small models need the blocks: 6.5 -> 0.5
+// ms at n = 1000 against 1024 columns a split).
 int64_t grad_splits(int64_t n) {
   const int64_t rows = ceil_div(n, 256);
-  return std::max<int64_t>(1, std::min<int64_t>(ceil_div(2048, rows), ceil_div(n, 1024)));
+  return std::max<int64_t>(1, std::min<int64_t>(ceil_div(2048, rows), ceil_div(n, 64)));
 }
+
+// Points from which the trace runs on the tree's generated kernel (RBF x
+// periodic + RQ, 11 factor columns: 0.13 ms generated and 0.78 ms interpreted
+// at n = 4096, 0.22 and 7.5 ms at n = 10007, where the interpreted one was
+// measured with the old splits): a model of this size trains for seconds, in
+// which one compilation (~0.5 s per tree and process) is repaid.  Below, and
+// for trees whose leaves share parameter slots, the interpreted kernel.
+constexpr int64_t kTreeGradJitMin = 4096;
 }  // namespace
 
 void tree_cat_grad_tables(const KernelTree& t, const float* p_dev, const float* X, int64_t n,
@@ -397,12 +408,30 @@ void tree_grad_traces(const KernelTree& t, const float* p_dev, const float* X, i
                       const float* Lf, const float* Rf, int ncols, double* g_host,
                       DevBuf<double>& work, hipStream_t st) {
   const int P = t.nparams;
-  const int64_t rows = ceil_div(n, 256), splits = grad_splits(n), nblk = rows * splits;
+  TreeGradJitKernel jk;
+  if (n >= kTreeGradJitMin) jk = tree_grad_jit_kernel(t);
+  int64_t rows = ceil_div(n, 256), splits = grad_splits(n), dps = 0;
+  if (jk.fn) {
+    rows = ceil_div(n, (int64_t)jk.block);
+    const int64_t offsets = jk.symmetric ? rows / 2 + 1 : rows;
+    dps = ceil_div(offsets, std::min(offsets, ceil_div(4096, rows)));
+    splits = ceil_div(offsets, dps);
+  }
+  const int64_t nblk = rows * splits;
   double* part = work.ensure((size_t)nblk * P + P);
   double* acc = part + (size_t)nblk * P;
   for (int c0 = 0; c0 < ncols; c0 += kGradCols) {
-    hipLaunchKernelGGL(k_tree_grad_trace, dim3((unsigned)rows, (unsigned)splits), dim3(256), 0,
-                       st, X, n, t, p_dev, Lf, Rf, ncols, c0, part);
+    if (jk.fn) {
+      long long nn = n, nb = rows, dd = dps;
+      int nc = ncols, cc = c0;
+      void* args[] = {(void*)&X,  &nn, (void*)&p_dev, (void*)&Lf, (void*)&Rf, &nc, &cc,
+                      &nb, &dd, (void*)&part};
+      MGP_HIP_CHECK(hipModuleLaunchKernel(jk.fn, (unsigned)rows, (unsigned)splits, 1, 256, 1, 1, 0,
+                                          st, args, nullptr));
+    } else {
+      hipLaunchKernelGGL(k_tree_grad_trace, dim3((unsigned)rows, (unsigned)splits), dim3(256), 0,
+                         st, X, n, t, p_dev, Lf, Rf, ncols, c0, part);
+    }
     hipLaunchKernelGGL(k_tree_part_sum, dim3((unsigned)P), dim3(64), 0, st, part, nblk, P,
                        c0 > 0 ? 1 : 0, acc);
     MGP_HIP_CHECK(hipGetLastError());

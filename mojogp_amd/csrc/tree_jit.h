@@ -23,4 +23,20 @@ TreeJitKernel tree_jit_kernel(const KernelTree& t, int nc);
 // The generated source (tests and inspection).
 std::string tree_jit_source(const KernelTree& t);
 
+struct TreeGradJitKernel {
+  hipFunction_t fn = nullptr;  // extern "C" k_tree_grad_jit; null: not generated for this tree
+  int block = 0;               // points per block
+  bool symmetric = false;      // column blocks of the cyclic half only
+};
+
+// The straight-line gradient-trace kernel of tree t: arguments (const float*
+// X, long long n, const float* p, const float* Lf, const float* Rf, int
+// ncols, int c0, long long nb, long long dps, double* part), grid (nb =
+// ceil(n / block), splits of dps column-block offsets), 256 threads;
+// part[(y nb + x) P + q] = the block's share of parameter q's trace over the
+// factor columns c0 .. min(c0 + 16, ncols).  Compiled on first use per (tree,
+// device); null for trees whose leaves share parameter slots.
+TreeGradJitKernel tree_grad_jit_kernel(const KernelTree& t);
+std::string tree_grad_jit_source(const KernelTree& t);
+
 }  // namespace mgp

@@ -31,6 +31,7 @@ constexpr int kJitTile = 128;  // column points per LDS tile
 const int kJitCols[] = {1, 2, 4, 8, 16};
 constexpr int kJitMfmaMinCols = 8;   // column counts from here use the MFMA product
 constexpr int kJitMfmaRowTiles = 2;  // 16-row tiles per wave in the MFMA kernel
+constexpr int kTreeGradBlock = 128;  // points per block of the gradient kernel
 
 std::string f(float v) {
   std::ostringstream o;
@@ -39,8 +40,10 @@ std::string f(float v) {
   return o.str();
 }
 
-// Prologue (per-thread constants from p) and pair code (k from xi, xj) of the
-// tree; leaf l's value is v<node>, the tree value the last node's.
+// Prologue (per-thread constants from p) and pair code (from xi, xj) of the
+// tree; leaf l's value is l<l>, node i's n<i>, the tree value the last node's.
+// The per-dimension terms and exponentials keep names of their own for the
+// gradient code below.
 void emit_tree(const KernelTree& t, std::string& pro, std::string& pair) {
   std::ostringstream P, Q;
   for (int l = 0; l < t.nleaves; ++l) {
@@ -66,14 +69,15 @@ void emit_tree(const KernelTree& t, std::string& pro, std::string& pair) {
         P << "  const float " << L << "off = p[" << lf.p0 + nls + 1 << "];\n";
       Q << "  float " << L << "d = 0.0f;\n";
       for (int q = 0; q < lf.ndim; ++q) {
-        const std::string xx = "xi[" + std::to_string(dim(q)) + "] * xj[" +
-                               std::to_string(dim(q)) + "]";
+        const std::string xx = L + "x" + std::to_string(q);
+        Q << "  const float " << xx << " = xi[" << dim(q) << "] * xj[" << dim(q) << "];\n";
         if (lf.ard)
           Q << "  " << L << "d = fmaf(" << L << "w" << q << ", " << xx << ", " << L << "d);\n";
         else
           Q << "  " << L << "d = " << L << "d + " << xx << ";\n";
       }
-      if (!lf.ard) Q << "  " << L << "d *= " << L << "w0;\n";
+      if (!lf.ard)
+        Q << "  const float " << L << "raw = " << L << "d;\n  " << L << "d *= " << L << "w0;\n";
       if (lf.kind == KIND_LINEAR) {
         Q << "  const float " << L << " = " << L << "os * " << L << "d;\n";
       } else {
@@ -92,22 +96,25 @@ void emit_tree(const KernelTree& t, std::string& pro, std::string& pair) {
         << "  const float " << L << "os = p[" << lf.p0 + nls + 1 << "];\n";
       Q << "  float " << L << "s = 0.0f;\n";
       for (int q = 0; q < lf.ndim; ++q)
-        Q << "  { const float sn = __sinf((xi[" << dim(q) << "] - xj[" << dim(q) << "]) * " << L
-          << "ip); " << L << "s = fmaf(sn * sn, " << L << "il" << (lf.ard ? q : 0) << ", " << L
-          << "s); }\n";
+        Q << "  const float " << L << "t" << q << " = (xi[" << dim(q) << "] - xj[" << dim(q)
+          << "]) * " << L << "ip, " << L << "n" << q << " = __sinf(" << L << "t" << q << ");\n  "
+          << L << "s = fmaf(" << L << "n" << q << " * " << L << "n" << q << ", " << L << "il"
+          << (lf.ard ? q : 0) << ", " << L << "s);\n";
       Q << "  const float " << L << " = " << L << "os * __expf(-2.0f * " << L << "s);\n";
       continue;
     }
     Q << "  float " << L << "r2 = 0.0f;\n";
     for (int q = 0; q < lf.ndim; ++q)
-      Q << "  { const float u = (xi[" << dim(q) << "] - xj[" << dim(q) << "]) * " << L << "il"
-        << (lf.ard ? q : 0) << "; " << L << "r2 = fmaf(u, u, " << L << "r2); }\n";
+      Q << "  const float " << L << "u" << q << " = (xi[" << dim(q) << "] - xj[" << dim(q)
+        << "]) * " << L << "il" << (lf.ard ? q : 0) << "; " << L << "r2 = fmaf(" << L << "u" << q
+        << ", " << L << "u" << q << ", " << L << "r2);\n";
     if (lf.kind == KIND_RQ) {
       P << "  const float " << L << "al = p[" << lf.p0 + nls << "];\n"
         << "  const float " << L << "ia = 0.5f / " << L << "al;\n"
         << "  const float " << L << "os = p[" << lf.p0 + nls + 1 << "];\n";
-      Q << "  const float " << L << " = " << L << "os * exp2f(-" << L << "al * __log2f(fmaf("
-        << L << "r2, " << L << "ia, 1.0f)));\n";
+      Q << "  const float " << L << "B = fmaf(" << L << "r2, " << L << "ia, 1.0f), " << L
+        << "lb = __log2f(" << L << "B);\n"
+        << "  const float " << L << " = " << L << "os * exp2f(-" << L << "al * " << L << "lb);\n";
       continue;
     }
     P << "  const float " << L << "os = p[" << lf.p0 + nls << "];\n";
@@ -125,12 +132,13 @@ void emit_tree(const KernelTree& t, std::string& pro, std::string& pair) {
         Q << "  const float " << L << " = " << L << "os * __expf(-" << L << "r);\n";
     } else if (lf.kind == KIND_MATERN32) {
       Q << "  const float " << L << "s3 = 1.7320508075688772f * " << L << "r;\n"
-        << "  const float " << L << " = " << L << "os * (1.0f + " << L << "s3) * __expf(fmaxf(-"
-        << L << "s3, -20.0f));\n";
+        << "  const float " << L << "e = __expf(fmaxf(-" << L << "s3, -20.0f));\n"
+        << "  const float " << L << " = " << L << "os * (1.0f + " << L << "s3) * " << L << "e;\n";
     } else {
       Q << "  const float " << L << "s5 = 2.2360679774997897f * " << L << "r;\n"
+        << "  const float " << L << "e = __expf(fmaxf(-" << L << "s5, -20.0f));\n"
         << "  const float " << L << " = " << L << "os * (1.0f + " << L << "s5 + (5.0f / 3.0f) * "
-        << L << "r2) * __expf(fmaxf(-" << L << "s5, -20.0f));\n";
+        << L << "r2) * " << L << "e;\n";
     }
   }
   for (int i = 0; i < t.nnodes; ++i) {
@@ -147,9 +155,11 @@ void emit_tree(const KernelTree& t, std::string& pro, std::string& pair) {
       Q << "  const float " << N << " = s" << i << " * n" << nd.a << ";\n";
     }
   }
-  Q << "  return n" << t.nnodes - 1 << ";\n";
   pro = P.str();
   pair = Q.str();
+}
+std::string tree_value_return(const KernelTree& t) {
+  return "  return n" + std::to_string(t.nnodes - 1) + ";\n";
 }
 
 // The kernel source: out partials part[y][c][i] = sum over split y of
@@ -158,6 +168,7 @@ void emit_tree(const KernelTree& t, std::string& pro, std::string& pair) {
 std::string tree_source(const KernelTree& t) {
   std::string pro, pair;
   emit_tree(t, pro, pair);
+  pair += tree_value_return(t);
   const int D = t.d, DP = (D + 3) / 4 * 4;
   std::ostringstream s;
   s << "#define D " << D << "\n#define DP " << DP << "\n#define TILE " << kJitTile << "\n"
@@ -309,6 +320,269 @@ std::string tree_source(const KernelTree& t) {
   return s.str();
 }
 
+// Backward pass of one pair and the final factors of its sums: the pair code
+// (after emit_tree's) adds w dK/dtheta_q, less a factor that depends on the
+// parameters only, into g[q]; fin holds that factor per parameter (C
+// expressions of p), applied once per thread.  False when two leaves or
+// scales share a parameter slot (their factors differ).
+bool emit_tree_grad(const KernelTree& t, std::string& pair, std::vector<std::string>& fin) {
+  std::ostringstream Q;
+  fin.assign((size_t)t.nparams, "0.0f");
+  std::vector<char> used((size_t)t.nparams, 0);
+  bool ok = true;
+  auto own = [&](int q, const std::string& factor) {
+    if (q < 0 || q >= t.nparams || used[(size_t)q]) {
+      ok = false;
+      return;
+    }
+    used[(size_t)q] = 1;
+    fin[(size_t)q] = factor;
+  };
+  auto pq = [](int q) { return "p[" + std::to_string(q) + "]"; };
+  for (int i = 0; i < t.nnodes; ++i)
+    Q << "  float a" << i << " = " << (i == t.nnodes - 1 ? "w" : "0.0f") << ";\n";
+  for (int i = t.nnodes - 1; i >= 0; --i) {
+    const TreeNode& nd = t.node[i];
+    const std::string A = "a" + std::to_string(i);
+    if (nd.code == TN_ADD) {
+      Q << "  a" << nd.a << " += " << A << "; a" << nd.b << " += " << A << ";\n";
+      continue;
+    }
+    if (nd.code == TN_MUL) {
+      Q << "  a" << nd.a << " = fmaf(" << A << ", n" << nd.b << ", a" << nd.a << "); a" << nd.b
+        << " = fmaf(" << A << ", n" << nd.a << ", a" << nd.b << ");\n";
+      continue;
+    }
+    if (nd.code == TN_SCALE) {
+      Q << "  a" << nd.a << " = fmaf(" << A << ", s" << i << ", a" << nd.a << ");\n  g[" << nd.b
+        << "] = fmaf(" << A << ", n" << nd.a << ", g[" << nd.b << "]);\n";
+      own(nd.b, "1.0f");
+      continue;
+    }
+    const int l = nd.a;
+    const TreeLeaf& lf = t.leaf[l];
+    if (lf.kind == KIND_CAT) continue;  // tables are learned outside this pass
+    const std::string L = "l" + std::to_string(l);
+    const int nls = lf.ard ? lf.ndim : 1;
+    auto add = [&](int q, const std::string& x, const std::string& y, const std::string& factor) {
+      Q << "  g[" << q << "] = fmaf(" << x << ", " << y << ", g[" << q << "]);\n";
+      own(q, factor);
+    };
+    if (lf.kind == KIND_LINEAR || lf.kind == KIND_POLY) {
+      const bool poly = lf.kind == KIND_POLY;
+      const int ios = lf.p0 + nls + (poly ? 2 : 0);
+      std::string h = A, factor = pq(ios);
+      if (poly) {
+        Q << "  const float " << L << "h = " << A << " * " << L << "bp;\n";
+        h = L + "h";
+        factor = f((float)lf.deg) + " * " + pq(ios);
+        Q << "  g[" << lf.p0 + nls + 1 << "] += " << h << ";\n";
+        own(lf.p0 + nls + 1, factor);
+      }
+      for (int q = 0; q < nls; ++q)
+        add(lf.p0 + q, h, lf.ard ? L + "x" + std::to_string(q) : L + "raw", factor);
+      add(ios, A, L, "1.0f / " + pq(ios));
+      continue;
+    }
+    if (lf.kind == KIND_PERIODIC) {
+      const int ip = lf.p0 + nls, ios = ip + 1;
+      // k = os exp(-2 S), S = sum_q sin^2(t_q) / l_q, t_q = pi dx_q / period
+      Q << "  const float " << L << "h = " << A << " * " << L << ";\n  float " << L
+        << "c = 0.0f;\n";
+      for (int q = 0; q < lf.ndim; ++q) {
+        const std::string n = L + "n" + std::to_string(q), tq = L + "t" + std::to_string(q);
+        Q << "  " << L << "c = fmaf(" << n << " * __cosf(" << tq << "), " << tq << " * " << L
+          << "il" << (lf.ard ? q : 0) << ", " << L << "c);\n";
+        if (lf.ard)
+          add(lf.p0 + q, L + "h * " + n, n,
+              "2.0f / (" + pq(lf.p0 + q) + " * " + pq(lf.p0 + q) + ")");
+      }
+      if (!lf.ard) add(lf.p0, L + "h", L + "s", "2.0f / " + pq(lf.p0));
+      add(ip, L + "h", L + "c", "4.0f / " + pq(ip));
+      Q << "  g[" << ios << "] += " << L << "h;\n";
+      own(ios, "1.0f / " + pq(ios));
+      continue;
+    }
+    // radial / RQ lengthscales: dk/dl_q = h u_q^2 / l_q with u_q = dx_q / l_q
+    int ios = lf.p0 + nls;
+    Q << "  const float " << L << "a = " << A << " * " << L << ";\n  const float " << L << "h = ";
+    if (lf.kind == KIND_RBF) {
+      Q << L << "a;\n";
+    } else if (lf.kind == KIND_MATERN12) {
+      Q << L << "a * __builtin_amdgcn_rcpf(" << L << "r);\n";
+    } else if (lf.kind == KIND_MATERN32) {
+      Q << A << " * (3.0f * " << L << "os) * " << L << "e;\n";
+    } else if (lf.kind == KIND_RQ) {
+      ios += 1;
+      Q << L << "a * __builtin_amdgcn_rcpf(" << L << "B);\n";
+      // dk/dalpha = k (r^2 / (2 alpha B) - ln B)
+      add(lf.p0 + nls, L + "a",
+          "fmaf(" + L + "r2 * " + L + "ia, __builtin_amdgcn_rcpf(" + L + "B), " + f(-kLn2) +
+              " * " + L + "lb)",
+          "1.0f");
+    } else {
+      Q << A << " * (5.0f / 3.0f * " << L << "os) * (1.0f + " << L << "s5) * " << L << "e;\n";
+    }
+    if (lf.ard)
+      for (int q = 0; q < lf.ndim; ++q) {
+        const std::string u = L + "u" + std::to_string(q);
+        add(lf.p0 + q, L + "h * " + u, u, "1.0f / " + pq(lf.p0 + q));
+      }
+    else
+      add(lf.p0, L + "h", L + "r2", "1.0f / " + pq(lf.p0));
+    Q << "  g[" << ios << "] += " << L << "a;\n";
+    own(ios, "1.0f / " + pq(ios));
+  }
+  pair = Q.str();
+  return ok;
+}
+
+// Gradient-trace kernel of the tree: part[(y gx + x) P + q] = the block's
+// share of sum_ab dK_ab/dtheta_q sum_c Lf[c][a] Rf[c][b], c in [c0, ncols).
+//
+// Every evaluator of a pair costs the forward and backward pass of the tree
+// (~100 VALU instructions for two or three leaves), so the kernel is VALU
+// bound and a pair is formed once for both of its orders where the tree is
+// symmetric (no correlation tables; n = 10007, RBF x periodic + RQ, 11 factor
+// columns: 7.54 ms interpreted, 0.22 ms): blocks of 128 points, row block b taking
+// the column blocks (b + delta) mod nb of the cyclic half, its diagonal block
+// with weight 1/2.  Per 16 x 16 tile w_ab + w_ba comes from the fp32 matrix
+// cores (v_mfma_f32_16x16x4_f32 over the factor columns, four at a time), its
+// result w[q] belonging to the pair (column 4 (lane/16) + q, row lane%16), so
+// a lane keeps its rows in registers and reads columns from LDS.  g sums a
+// lane's 8 pairs of a tile column in fp32, then fp64.
+std::string tree_grad_source(const KernelTree& t) {
+  std::string pro, pair, back;
+  std::vector<std::string> fin;
+  emit_tree(t, pro, pair);
+  if (!emit_tree_grad(t, back, fin)) return std::string();
+  const int D = t.d, DP = (D + 3) / 4 * 4, P = t.nparams;
+  const bool sym = t.table_size == 0;
+  std::ostringstream s;
+  s << "#define D " << D << "\n#define DP " << DP << "\n#define P " << P << "\n#define BLK "
+    << kTreeGradBlock << "\n#define SYM " << (sym ? 1 : 0) << "\n"
+    << R"(typedef float f4m __attribute__((ext_vector_type(4)));
+#define R 2
+#define CS (BLK + 16)
+extern "C" __global__ __launch_bounds__(256) void k_tree_grad_jit(
+    const float* __restrict__ X, long long n, const float* __restrict__ p,
+    const float* __restrict__ Lf, const float* __restrict__ Rf, int ncols, int c0, long long nb,
+    long long dps, double* __restrict__ part) {
+  __shared__ __align__(16) float sx[BLK * DP];
+  __shared__ float sl[16 * CS], sr[16 * CS];
+  __shared__ double red[4];
+)" << pro
+    << R"(  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lm = lane & 15, lq = lane >> 4;
+  const int cn = ncols - c0 < 16 ? ncols - c0 : 16;
+  const int csteps = (cn + 3) / 4;
+  const long long b = blockIdx.x;
+  float xi[R][DP], lb[R][4], rb[R][4];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const long long i = b * BLK + (wave * R + r) * 16 + lm;
+#pragma unroll
+    for (int k = 0; k < DP; ++k) xi[r][k] = (i < n && k < D) ? X[i * D + k] : 0.0f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int c = 4 * s + lq;
+      const bool in = i < n && c < cn;
+      lb[r][s] = in ? Lf[(long long)(c0 + c) * n + i] : 0.0f;
+      rb[r][s] = in ? Rf[(long long)(c0 + c) * n + i] : 0.0f;
+    }
+  }
+  double gd[P];
+#pragma unroll
+  for (int q = 0; q < P; ++q) gd[q] = 0.0;
+#if SYM
+  const long long span = (nb & 1) ? (nb - 1) / 2 : (b < nb / 2 ? nb / 2 : nb / 2 - 1);
+#else
+  const long long span = nb - 1;
+#endif
+  const long long d0 = (long long)blockIdx.y * dps;
+  const long long d1 = d0 + dps < span + 1 ? d0 + dps : span + 1;
+  for (long long dl = d0; dl < d1; ++dl) {
+    long long J = b + dl;
+    if (J >= nb) J -= nb;
+    const long long j0 = J * BLK;
+    const int cnt = (int)(n - j0 < BLK ? n - j0 : BLK);
+    __syncthreads();
+    for (int q = threadIdx.x; q < BLK * DP; q += 256) {
+      const int jj = q / DP, k = q - jj * DP;
+      sx[q] = (jj < cnt && k < D) ? X[(j0 + jj) * D + k] : 0.0f;
+    }
+    for (int q = threadIdx.x; q < BLK * 16; q += 256) {
+      const int c = q / BLK, jj = q - c * BLK;
+      const bool in = jj < cnt && c < cn;
+      sr[c * CS + jj] = in ? Rf[(long long)(c0 + c) * n + j0 + jj] : 0.0f;
+#if SYM
+      sl[c * CS + jj] = in ? Lf[(long long)(c0 + c) * n + j0 + jj] : 0.0f;
+#endif
+    }
+    __syncthreads();
+    const float wt = (SYM && dl == 0) ? 0.5f : 1.0f;
+    const int tiles = (cnt + 15) / 16;
+#pragma unroll 1
+    for (int ct = 0; ct < tiles; ++ct) {
+      float g[P];
+#pragma unroll
+      for (int q = 0; q < P; ++q) g[q] = 0.0f;
+      f4m wv[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) wv[r] = f4m{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (s >= csteps) break;
+        const float ar = sr[(4 * s + lq) * CS + 16 * ct + lm];
+#if SYM
+        const float al = sl[(4 * s + lq) * CS + 16 * ct + lm];
+#endif
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          wv[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar, lb[r][s], wv[r], 0, 0, 0);
+#if SYM
+          wv[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(al, rb[r][s], wv[r], 0, 0, 0);
+#endif
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float* xjp = sx + (16 * ct + 4 * lq + e) * DP;
+        float xj[DP];
+#pragma unroll
+        for (int k = 0; k < DP; k += 4) {
+          const f4m x = *reinterpret_cast<const f4m*>(xjp + k);
+          xj[k] = x[0]; xj[k + 1] = x[1]; xj[k + 2] = x[2]; xj[k + 3] = x[3];
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const float w = wt * wv[r][e];
+          auto one = [&](const float* xi) __attribute__((always_inline)) {
+)" << pair << back
+    << R"(          };
+          one(xi[r]);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < P; ++q) gd[q] += (double)g[q];
+    }
+  }
+  double* dst = part + ((long long)blockIdx.y * gridDim.x + blockIdx.x) * P;
+  auto put = [&](int q, double v) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+    __syncthreads();
+    if (lane == 0) red[wave] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) dst[q] = red[0] + red[1] + red[2] + red[3];
+  };
+)";
+  for (int q = 0; q < P; ++q)
+    s << "  put(" << q << ", gd[" << q << "] * (double)(" << fin[(size_t)q] << "));\n";
+  s << "}\n";
+  return s.str();
+}
+
 std::string spec_key(const KernelTree& t) {
   std::ostringstream o;
   o << t.d << ' ' << t.nparams << ' ' << t.nleaves << ' ' << t.nnodes << ' ' << t.table_size;
@@ -348,12 +622,9 @@ std::map<std::pair<std::string, int>, Compiled> g_jit;
     }                                                                                     \
   } while (0)
 
-Compiled compile_tree(const KernelTree& t) {
-  const std::string src = tree_source(t);
+hipModule_t compile_source(const std::string& src, const char* name) {
   hiprtcProgram prog = nullptr;
-  MGP_RTC_CHECK(hiprtcCreateProgram(&prog, src.c_str(), "kernel_tree_jit.hip", 0, nullptr,
-                                    nullptr),
-                prog);
+  MGP_RTC_CHECK(hiprtcCreateProgram(&prog, src.c_str(), name, 0, nullptr, nullptr), prog);
   // packed-FP32 VALU forms are disabled here as for every device file
   const char* opts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang",
                         "-target-feature", "-Xclang", "-packed-fp32-ops"};
@@ -370,8 +641,14 @@ Compiled compile_tree(const KernelTree& t) {
     throw;
   }
   (void)hiprtcDestroyProgram(&prog);
+  hipModule_t mod = nullptr;
+  MGP_HIP_CHECK(hipModuleLoadData(&mod, code.data()));
+  return mod;
+}
+
+Compiled compile_tree(const KernelTree& t) {
   Compiled c;
-  MGP_HIP_CHECK(hipModuleLoadData(&c.mod, code.data()));
+  c.mod = compile_source(tree_source(t), "kernel_tree_jit.hip");
   for (int k = 0; k < 5; ++k) {
     const std::string name = "k_tree_jit_" + std::to_string(kJitCols[k]);
     MGP_HIP_CHECK(hipModuleGetFunction(&c.fn[k], c.mod, name.c_str()));
@@ -379,9 +656,34 @@ Compiled compile_tree(const KernelTree& t) {
   return c;
 }
 
+// Gradient kernels per (tree, device); fn null where the tree has none.
+std::map<std::pair<std::string, int>, hipFunction_t> g_jit_grad;
+
 }  // namespace
 
 std::string tree_jit_source(const KernelTree& t) { return tree_source(t); }
+std::string tree_grad_jit_source(const KernelTree& t) { return tree_grad_source(t); }
+
+TreeGradJitKernel tree_grad_jit_kernel(const KernelTree& t) {
+  int dev = 0;
+  MGP_HIP_CHECK(hipGetDevice(&dev));
+  const auto key = std::make_pair(spec_key(t), dev);
+  std::lock_guard<std::mutex> lk(g_jit_mu);
+  auto it = g_jit_grad.find(key);
+  if (it == g_jit_grad.end()) {
+    hipFunction_t fn = nullptr;
+    const std::string src = tree_grad_source(t);
+    if (!src.empty())
+      MGP_HIP_CHECK(hipModuleGetFunction(&fn, compile_source(src, "kernel_tree_grad_jit.hip"),
+                                         "k_tree_grad_jit"));
+    it = g_jit_grad.emplace(key, fn).first;
+  }
+  TreeGradJitKernel out;
+  out.fn = it->second;
+  out.block = kTreeGradBlock;
+  out.symmetric = t.table_size == 0;
+  return out;
+}
 
 TreeJitKernel tree_jit_kernel(const KernelTree& t, int nc) {
   MGP_REQUIRE(nc >= 1 && nc <= 16, "tree product pass takes 1..16 right-hand sides");

@@ -1,0 +1,83 @@
+"""Gradient traces of kernel trees on their generated kernel (n >= 4096) and
+on the interpreted one just below, against the float64 tree restatement:
+every leaf kind, isotropic and ARD, shared subtrees' adjoints, a categorical
+leaf (tables need not be symmetric, so no pair is folded), ragged last blocks
+and 1 .. 17 factor columns.
+
+Bound: a term w_ab dK_ab / dtheta is formed in fp32 from a handful of
+operations (<= 16 ulps with the hardware exp / sin / log), and fp32 sums run
+over at most 64 terms before fp64, so |error| <= (16 + 64) 2^-24 sum |w dK|."""
+
+import numpy as np
+import pytest
+
+from mojogp_amd import (GD, RBF, RQ, Linear, Matern12, Matern32, Matern52, Periodic, Polynomial,
+                        make_ard_kernel)
+from mojogp_amd._provider import NativeProvider
+from oracle import kernels as ok
+
+pytestmark = pytest.mark.gpu
+
+TREES = {
+    "rbf*per[0]+rq": (lambda: RBF() * Periodic(active_dims=[0]) + RQ(), 3),
+    "ard": (lambda: make_ard_kernel((RQ(ard=True) + Matern52(ard=True))
+                                    * Periodic(period=2.0, ard=True), 2), 2),
+    "2*(m12+m32)*m52": (lambda: 2.0 * (Matern12() + Matern32()) * Matern52(), 5),
+    "poly_ard+lin*m12_ard": (lambda: make_ard_kernel(
+        Polynomial(degree=2.0, ard=True) + Linear() * Matern12(ard=True), 2), 2),
+    "poly+lin_ard": (lambda: make_ard_kernel(Polynomial() + Linear(ard=True), 3), 3),
+}
+
+
+def _check(T, X, params, L, R, got):
+    ref, mag = np.zeros(T.nparams), np.zeros(T.nparams)
+    for i in range(0, len(X), 256):
+        G = T.gradients(X[i:i + 256], X, params)
+        W = L[:, i:i + 256].astype(np.float64).T @ R.astype(np.float64)
+        ref += (G * W).sum(axis=(1, 2))
+        mag += np.abs(G * W).sum(axis=(1, 2))
+    err = np.abs(got - ref)
+    print("  error / bound", np.round(err / np.maximum(80 * 2.0**-24 * mag, 1e-300), 4), flush=True)
+    assert np.all(err <= 80 * 2.0**-24 * mag)
+
+
+@pytest.mark.parametrize("name", list(TREES))
+@pytest.mark.parametrize("n,t", [(700, 17), (4095, 3), (4096, 1), (4227, 17)])
+def test_traces_match_oracle(name, n, t):
+    mk, d = TREES[name]
+    node = mk()
+    rng = np.random.default_rng(n + t)
+    X = rng.uniform(-2, 2, size=(n, d)).astype(np.float32)
+    T = ok.TreeKernel(node.to_dict(), d)
+    params = rng.uniform(0.6, 1.5, T.nparams).astype(np.float32)
+    if "poly" in name:
+        params = node.to_engine_params(node.get_initial_params()).astype(np.float32)
+    L, R = (rng.normal(size=(t, n)).astype(np.float32) for _ in range(2))
+    print(f"tree trace {name} n={n} t={t}", flush=True)
+    p = NativeProvider(None, False, X, params, 0.2, tree_spec=node.to_tree_spec(d))
+    try:
+        got = p.gradient_trace(L, R)
+    finally:
+        p.close()
+    _check(T, X, params, L, R, got)
+
+
+def test_categorical_tree_is_not_folded():
+    import ctypes as C
+    from mojogp_amd import _lib
+    rng = np.random.default_rng(5)
+    n, t, levels = 4100, 6, 4
+    X = np.stack([rng.uniform(-2, 2, n), rng.integers(0, levels, n)], axis=1).astype(np.float32)
+    node = RBF(active_dims=[0]) * GD(levels, active_dims=[1])
+    table = rng.uniform(0.2, 1.0, size=(levels, levels)).astype(np.float32)  # not symmetric
+    T = ok.TreeKernel(node.to_dict(), 2, cat_tables=[table])
+    params = np.array([0.8, 1.3], np.float32)
+    L, R = (rng.normal(size=(t, n)).astype(np.float32) for _ in range(2))
+    p = NativeProvider(None, False, X, params, 0.2, tree_spec=node.to_tree_spec(2))
+    try:
+        flat = np.ascontiguousarray(table.ravel())
+        _lib.call("mgp_set_categorical_tables", p.handle, _lib.fptr(flat), int(flat.size))
+        got = p.gradient_trace(L, R)
+    finally:
+        p.close()
+    _check(T, X, params, L, R, got)
