@@ -637,62 +637,56 @@ __global__ __launch_bounds__(256) void k_fused_tile(
   }
 }
 
-// out[c*m+i] = os * sum_s partial[(s*cpad + c)*mpad + i] (+ noise V)
-__global__ void k_reduce_splits(const float* __restrict__ partial, int splits,
-                                int cpad, int64_t mpad, int64_t m, int ncols,
-                                float os, float noise, int add_noise,
-                                const float* __restrict__ Vin,
-                                float* __restrict__ out) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)ncols * m) return;
-  const int c = (int)(idx / m);
-  const int64_t i = idx - (int64_t)c * m;
-  double tot = 0.0;
-  for (int s = 0; s < splits; ++s) tot += partial[((int64_t)s * cpad + c) * mpad + i];
-  float o = os * (float)tot;
-  if (add_noise) o = fmaf(noise, Vin[idx], o);
-  out[idx] = o;
-}
-
-// k_reduce_splits for four consecutive rows per thread (m and mpad multiples
-// of 4): idx4 indexes quads of out; the splits are loaded four at a time and
-// added in split order, as above.
+// out[c*m+i] = os * sum_s partial[(s*cpad + c)*mpad + i] (+ noise V): four
+// consecutive rows of one column per thread, the splits loaded eight at a time
+// (a small model's reduction is a chain of load latencies) and added in split
+// order in fp64.  vec: out and Vin quads are 16-byte aligned (m a multiple of
+// 4); the partials always are (mpad a multiple of 16).
 __global__ void k_reduce_splits4(const float* __restrict__ partial, int splits, int cpad,
                                  int64_t mpad, int64_t m, int ncols, float os, float noise,
-                                 int add_noise, const float* __restrict__ Vin,
+                                 int add_noise, int vec, const float* __restrict__ Vin,
                                  float* __restrict__ out) {
+  const int64_t mq = (m + 3) / 4;
   const int64_t q4 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q4 >= (int64_t)ncols * (m / 4)) return;
-  const int64_t idx = 4 * q4;
-  const int c = (int)(idx / m);
-  const int64_t i = idx - (int64_t)c * m;
+  if (q4 >= (int64_t)ncols * mq) return;
+  const int c = (int)(q4 / mq);
+  const int64_t i = 4 * (q4 - (int64_t)c * mq);
   const float* pc = partial + (int64_t)c * mpad + i;
   const int64_t sstride = (int64_t)cpad * mpad;
   double tot[4] = {0.0, 0.0, 0.0, 0.0};
-  int s = 0;
-  for (; s + 4 <= splits; s += 4) {
-    f4 v[4];
+  auto batch = [&](int s, auto count) __attribute__((always_inline)) {
+    constexpr int B = decltype(count)::value;
+    f4 v[B];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = *reinterpret_cast<const f4*>(pc + (s + q) * sstride);
+    for (int q = 0; q < B; ++q) v[q] = *reinterpret_cast<const f4*>(pc + (s + q) * sstride);
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < B; ++q)
 #pragma unroll
       for (int e = 0; e < 4; ++e) tot[e] += v[q][e];
+  };
+  int s = 0;
+  for (; s + 8 <= splits; s += 8) batch(s, std::integral_constant<int, 8>{});
+  if (s + 4 <= splits) {
+    batch(s, std::integral_constant<int, 4>{});
+    s += 4;
   }
-  for (; s < splits; ++s) {
-    const f4 v = *reinterpret_cast<const f4*>(pc + s * sstride);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) tot[e] += v[e];
-  }
+  for (; s < splits; ++s) batch(s, std::integral_constant<int, 1>{});
   f4 o;
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = os * (float)tot[e];
-  if (add_noise) {
-    const f4 vin = *reinterpret_cast<const f4*>(Vin + idx);
+  const int64_t idx = (int64_t)c * m + i;
+  if (vec) {
+    if (add_noise) {
+      const f4 vin = *reinterpret_cast<const f4*>(Vin + idx);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = fmaf(noise, vin[e], o[e]);
+      for (int e = 0; e < 4; ++e) o[e] = fmaf(noise, vin[e], o[e]);
+    }
+    *reinterpret_cast<f4*>(out + idx) = o;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (i + e < m) out[idx + e] = add_noise ? fmaf(noise, Vin[idx + e], o[e]) : o[e];
   }
-  *reinterpret_cast<f4*>(out + idx) = o;
 }
 
 // ---------------------------------------------------------------------------
@@ -1873,29 +1867,78 @@ using TileFn = void (*)(const h8*, int64_t, const h8*, const void*, int64_t,
                         int64_t, int64_t, int64_t, int, float, float,
                         const uint32_t*, const float*, float*, float*, int64_t, int);
 
-// Row tiles per wave: 4, or 2 where the register budget needs it (more than 16
-// right-hand sides).
-constexpr int rows_per_wave_tiles(int, int ncg) { return ncg >= 2 ? 2 : 4; }
-
-template <int KIND, int NCG>
+template <int KIND, int NCG, int R>
 TileFn pick_kb(int kb) {
   switch (kb) {
-    case 1: return k_fused_tile<KIND, 1, NCG, rows_per_wave_tiles(1, NCG)>;
-    case 2: return k_fused_tile<KIND, 2, NCG, rows_per_wave_tiles(2, NCG)>;
-    case 3: return k_fused_tile<KIND, 3, NCG, rows_per_wave_tiles(3, NCG)>;
+    case 1: return k_fused_tile<KIND, 1, NCG, R>;
+    case 2: return k_fused_tile<KIND, 2, NCG, R>;
+    case 3: return k_fused_tile<KIND, 3, NCG, R>;
   }
   return nullptr;
 }
 
+// R row tiles per wave: 4 or 2 up to 16 right-hand sides, 2 beyond (registers).
 template <int KIND>
-TileFn pick_tile(int kb, int ncg) {
+TileFn pick_tile(int kb, int ncg, int R) {
   switch (ncg) {
-    case 0: return pick_kb<KIND, 0>(kb);
-    case 1: return pick_kb<KIND, 1>(kb);
-    case 2: return pick_kb<KIND, 2>(kb);
-    case 4: return pick_kb<KIND, 4>(kb);
+    case 0: return R == 4 ? pick_kb<KIND, 0, 4>(kb) : pick_kb<KIND, 0, 2>(kb);
+    case 1: return R == 4 ? pick_kb<KIND, 1, 4>(kb) : pick_kb<KIND, 1, 2>(kb);
+    case 2: return pick_kb<KIND, 2, 2>(kb);
+    case 4: return pick_kb<KIND, 4, 2>(kb);
   }
   return nullptr;
+}
+
+// Row tiles per wave and column splits of one tile launch.
+struct TilePlan {
+  int R;
+  int64_t splits;
+};
+
+// Launches that fill the chip several times over: >= 2048 workgroups (1024
+// with 64 right-hand sides, whose waves carry 4x the work and whose split
+// partials cost 4x the traffic) and >= 32 column tiles a split.  Products too
+// small for that (fewer than kTileFull workgroups under that rule: n below
+// ~12k, cross products of few test points) are bound by the chain of
+// column-tile pairs of one wave, so they take 2 row tiles a wave and the
+// split count that minimises
+//   pairs R (u0 + u1 k) us   k = workgroups on the busiest CU: one wave a
+//                            SIMD forms a tile pair in u0 + u1 (0.15 us, 0.26
+//                            with four column groups), more waves hide part
+//                            or most of its latency
+// + splits max(0.12 us, bytes of its partials, written and read, at 3.2 TB/s)
+// (fitted to a sweep of 1..24 pairs a split at n = 500 .. 20000 and 1, 11 and
+// 40 right-hand sides: products of 1000 / 2000 / 4000 points 31 / 42 / 42 ->
+// 21 / 23 / 26 us with one column, 44 / 59 / 59 -> 29 / 31 / 38 us with 11).
+constexpr int64_t kTileFull = 700;
+TilePlan tile_plan(int64_t row_tiles, int64_t col_pairs, int ncg, int nc) {
+  TilePlan p;
+  p.R = ncg >= 2 ? 2 : 4;
+  p.splits = 1;
+  const int64_t target = ncg >= 4 ? 1024 : 2048;
+  const int64_t blocks = ceil_div(row_tiles, (int64_t)kWaves * p.R);
+  while (blocks * p.splits < target && col_pairs / (p.splits * 2) >= 16 && p.splits < 64)
+    p.splits *= 2;
+  if (blocks * p.splits >= kTileFull) return p;
+  p.R = 2;
+  const int64_t rb = ceil_div(row_tiles, (int64_t)kWaves * p.R);
+  const double u0 = ncg <= 1 ? 0.06 : ncg == 2 ? 0.12 : 0.2;
+  const double u1 = ncg <= 1 ? 0.09 : ncg == 2 ? 0.08 : 0.06;
+  const double split_us =
+      std::max(0.12, (double)row_tiles * 16 * 4 * (std::max(16 * ncg, 1) + nc) / 3.2e6);
+  double best = 0.0;
+  for (int64_t s = 1; s <= std::min<int64_t>(col_pairs, 128); ++s) {
+    const int64_t pairs = ceil_div(col_pairs, s);
+    const int64_t real = ceil_div(col_pairs, pairs);
+    if (real != s) continue;
+    const double k = (double)ceil_div(rb * s, 256);
+    const double cost = (double)pairs * p.R * (u0 + u1 * k) + (double)s * split_us;
+    if (s == 1 || cost < best) {
+      best = cost;
+      p.splits = s;
+    }
+  }
+  return p;
 }
 
 }  // namespace
@@ -2259,7 +2302,6 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
   for (int c0 = 0; c0 < a.ncols; c0 += chunk) {
     const int nc = std::min(chunk, a.ncols - c0);
     const int ncg = nc == 1 ? 0 : (nc <= 16 ? 1 : (nc <= 32 ? 2 : 4));
-    const int R = rows_per_wave_tiles(kb, ncg);
     const int cpad = ncg == 0 ? 1 : 16 * ncg;
     const float* Vc = V_dev + (int64_t)c0 * a.n;
     float* outc = out_dev + (int64_t)c0 * a.m;
@@ -2313,23 +2355,15 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
     }
     MGP_HIP_CHECK(hipGetLastError());
 
-    // Grid: row blocks x j splits.  Aim for >= 2048 workgroups (1024 with 64
-    // right-hand sides, whose waves carry 4x the work and whose split partials
-    // cost 4x the traffic) so 256 CUs see several waves each, while every split
-    // keeps >= 32 j tiles of work.
+    const TilePlan plan = tile_plan(row_tiles, col_pairs, ncg, nc);
+    const int R = plan.R;
     const int64_t row_blocks = ceil_div(row_tiles, (int64_t)kWaves * R);
-    const int64_t target_blocks = ncg >= 4 ? 1024 : 2048;
-    int64_t splits = force_splits > 0 ? force_splits : 1;
-    if (force_splits <= 0) {
-      while (row_blocks * splits < target_blocks && col_pairs / (splits * 2) >= 16 &&
-             splits < 64)
-        splits *= 2;
-    }
+    int64_t splits = force_splits > 0 ? force_splits : plan.splits;
     if (ws.arena != nullptr && splits > 1) {
       // Fixed arena: as many splits as the remaining bytes hold partials for.
       const size_t per_split = (size_t)round_up((int64_t)cpad * mpad * 4, 256);
       const int64_t fit = (int64_t)(buf.left() / per_split);
-      while (splits > 1 && splits > fit) splits /= 2;
+      if (splits > fit) splits = std::max<int64_t>(1, fit);
     }
     const int64_t pairs_per_split = ceil_div(col_pairs, splits);
     splits = ceil_div(col_pairs, pairs_per_split);
@@ -2339,9 +2373,9 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
       partial = buf.take(ws.partial, (size_t)splits * cpad * mpad);
 
     MGP_REQUIRE(a.kind != KIND_MATERN12, "Matern-1/2 has no Gram-form tile path");
-    TileFn fn = a.kind == KIND_RBF        ? pick_tile<KIND_RBF>(kb, ncg)
-                : a.kind == KIND_MATERN32 ? pick_tile<KIND_MATERN32>(kb, ncg)
-                                          : pick_tile<KIND_MATERN52>(kb, ncg);
+    TileFn fn = a.kind == KIND_RBF        ? pick_tile<KIND_RBF>(kb, ncg, R)
+                : a.kind == KIND_MATERN32 ? pick_tile<KIND_MATERN32>(kb, ncg, R)
+                                          : pick_tile<KIND_MATERN52>(kb, ncg, R);
     MGP_REQUIRE(fn != nullptr, "no tile kernel for this shape");
     const int64_t diag_shift = a.square ? 0 : (int64_t)1 << 40;
     if (ws.time_tile) MGP_HIP_CHECK(hipEventRecord(ws.ev0, st));
@@ -2377,19 +2411,12 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
                            a.noise, a.square ? 1 : 0, Vin, a.mix, a.mix_accumulate ? 1 : 0, outc);
       MGP_HIP_CHECK(hipGetLastError());
     } else if (splits > 1) {
-      const int64_t tot = (int64_t)nc * a.m;
-      const bool q4 = a.m % 4 == 0 && mpad % 4 == 0 &&
-                      reinterpret_cast<uintptr_t>(outc) % 16 == 0 &&
-                      reinterpret_cast<uintptr_t>(partial) % 16 == 0 &&
-                      (Vin == nullptr || reinterpret_cast<uintptr_t>(Vin) % 16 == 0);
-      if (q4)
-        hipLaunchKernelGGL(k_reduce_splits4, dim3((unsigned)ceil_div(tot / 4, 256)), dim3(256),
-                           0, st, partial, (int)splits, cpad, mpad, a.m, nc, a.outputscale,
-                           a.noise, a.square ? 1 : 0, Vin, outc);
-      else
-        hipLaunchKernelGGL(k_reduce_splits, dim3((unsigned)ceil_div(tot, 256)), dim3(256),
-                           0, st, partial, (int)splits, cpad, mpad, a.m, nc,
-                           a.outputscale, a.noise, a.square ? 1 : 0, Vin, outc);
+      const int64_t tot = (int64_t)nc * ceil_div(a.m, 4);
+      const bool vec = a.m % 4 == 0 && reinterpret_cast<uintptr_t>(outc) % 16 == 0 &&
+                       (Vin == nullptr || reinterpret_cast<uintptr_t>(Vin) % 16 == 0);
+      hipLaunchKernelGGL(k_reduce_splits4, dim3((unsigned)ceil_div(tot, 256)), dim3(256), 0, st,
+                         partial, (int)splits, cpad, mpad, a.m, nc, a.outputscale, a.noise,
+                         a.square ? 1 : 0, vec ? 1 : 0, Vin, outc);
       MGP_HIP_CHECK(hipGetLastError());
     }
   }
