@@ -71,6 +71,9 @@ struct CGOperator {
   // precond(r, ncols, z, rz_part, nb): z = P^-1 r and, when rz_part is set,
   // the partials rz_part[c*nb + b] of r . z over nb row chunks.
   std::function<void(const float*, int, float*, double*, int)> precond;
+  // small systems without a preconditioner: product and vector updates fused
+  // (precond is then empty); null otherwise
+  SmallCg* small = nullptr;
 };
 
 // Solves A X = rhs for `ncols` columns (device rhs [C][n]) by the reference's

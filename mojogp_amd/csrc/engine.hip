@@ -360,6 +360,20 @@ CGResult batched_cg(Provider& pv, Precond* P, const float* rhs, int C, int max_i
   op.n = pv.n;
   op.st = pv.st;
   op.matvec = [&pv](const float* V, int ncols, float* out) { pv.forward(V, ncols, out); };
+  SmallCg small;
+  if (!(P && P->rank > 0) && pv.fused_route() && small_cg_route(pv.kind, pv.train, C)) {
+    small.a.kind = pv.kind;
+    small.a.outputscale = pv.outputscale();
+    small.a.noise = pv.scalar_noise();
+    small.a.square = true;
+    small.a.m = small.a.n = pv.n;
+    small.a.ncols = C;
+    small.pts = &pv.train;
+    small.noise_vec = pv.has_noise_vec ? pv.noise_vec.ptr : nullptr;
+    small.ws = &pv.ws;
+    small.st = pv.st;
+    op.small = &small;
+  }
   if (P && P->rank > 0) {
     op.precond = [&pv, P](const float* r, int ncols, float* z, double* rz_part, int nb) {
       woodbury_apply(P->L.ptr, pv.n, P->rank, P->Minv.ptr, P->noise, r, ncols, z, P->work, r,
@@ -410,20 +424,25 @@ CGResult batched_cg(const CGOperator& op, const float* rhs, int C, int max_iter,
 
   CGResult res;
   int tridiag_size = 0;
+  if (op.small) op.small->begin(p);
   MGP_HIP_CHECK(hipStreamSynchronize(st));
   const auto t_loop = Clock::now();
   for (int iter = 0; iter < max_iter; ++iter) {
     res.iterations = iter + 1;
-    op.matvec(p, C, Ap);
-    coldot_partial(p, Ap, n, C, nb, pa, st);
-    cg_update(x, r, p, Ap, n, C, nb, pa, s, prr, st);  // alpha from pAp; r.r partials
-    if (pre) op.precond(r, C, z, pb, nb);
-    // beta from the r.z partials (r.r without a preconditioner), p update
-    cg_pupdate(p, z, n, C, nb, pre ? pb : prr, s, iter, max_tridiag, st);
-    std::swap(s.rz_old, s.rz_next);
+    if (op.small) {
+      op.small->step(x, r, p, {s.rz_old, prr, s.hist_alpha, s.hist_beta}, iter, max_tridiag);
+    } else {
+      op.matvec(p, C, Ap);
+      coldot_partial(p, Ap, n, C, nb, pa, st);
+      cg_update(x, r, p, Ap, n, C, nb, pa, s, prr, st);  // alpha from pAp; r.r partials
+      if (pre) op.precond(r, C, z, pb, nb);
+      // beta from the r.z partials (r.r without a preconditioner), p update
+      cg_pupdate(p, z, n, C, nb, pre ? pb : prr, s, iter, max_tridiag, st);
+      std::swap(s.rz_old, s.rz_next);
+    }
     if (iter < max_tridiag) tridiag_size = iter + 1;
     if (iter >= 10 && (((iter + 1) % 10) == 0 || iter == max_iter - 1)) {
-      cg_mean_resnorm(prr, nb, C, w.resn.ptr, st);
+      cg_mean_resnorm(prr, op.small ? 1 : nb, C, w.resn.ptr, st);
       float mean_res = 0.f;
       MGP_HIP_CHECK(hipMemcpyAsync(&mean_res, w.resn.ptr, sizeof(float),
                                    hipMemcpyDeviceToHost, st));

@@ -172,6 +172,36 @@ constexpr int64_t kSymMinBlocks = 48;
 bool symmetric_route_taken(const PackedPoints& pts, int ncols);
 constexpr double kSymMaxBytes = 16e9;
 
+// Unpreconditioned CG iterations of a small square system (up to kSmallCgMax
+// points and 16 columns on the one-sided tile kernel): the tile product and
+// one vector kernel per iteration.
+struct SmallCgScalars {
+  float* rz;          // [C] r.r, updated in place
+  double* rr;         // [C] r.r of the updated residual (fp64)
+  float* hist_alpha;  // [max_tridiag][C]
+  float* hist_beta;
+};
+// From here on a column's traffic through one CU costs more than the launches.
+constexpr int64_t kSmallCgMax = 16384;
+bool small_cg_route(int kind, const PackedPoints& pts, int ncols);
+struct SmallCg {
+  MatvecArgs a;  // square, m = n = pts->n, ncols, outputscale, scalar noise
+  const PackedPoints* pts = nullptr;
+  const float* noise_vec = nullptr;  // optional per-point noise (device [n])
+  MatvecWorkspace* ws = nullptr;     // holds the packed p between the steps
+  hipStream_t st = nullptr;
+  // Packs the first search direction p ([C][n]).
+  void begin(const float* p);
+  // Ap, alpha, x += alpha p, r -= alpha Ap, beta, p = r + beta p, p packed.
+  void step(float* x, float* r, float* p, const SmallCgScalars& s, int iter, int max_tridiag);
+
+ private:
+  int R = 2;
+  int64_t splits = 1, pairs_per_split = 1;
+  void* vp = nullptr;
+  uint32_t* colmax = nullptr;
+};
+
 // Bytes of work buffers one fused_matvec call with ncols right-hand sides
 // over cols needs at the least (no split partials): the arena size below which
 // the fixed-arena mode rejects the call.

@@ -671,21 +671,204 @@ __global__ void k_reduce_splits4(const float* __restrict__ partial, int splits, 
     s += 4;
   }
   for (; s < splits; ++s) batch(s, std::integral_constant<int, 1>{});
+  // os sum + noise V in fp64, rounded once
+  const int64_t idx = (int64_t)c * m + i;
+  f4 vin = f4{0.f, 0.f, 0.f, 0.f};
+  if (add_noise) {
+    if (vec) {
+      vin = *reinterpret_cast<const f4*>(Vin + idx);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i + e < m) vin[e] = Vin[idx + e];
+    }
+  }
   f4 o;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = os * (float)tot[e];
-  const int64_t idx = (int64_t)c * m + i;
+  for (int e = 0; e < 4; ++e) o[e] = (float)((double)os * tot[e] + (double)noise * (double)vin[e]);
   if (vec) {
-    if (add_noise) {
-      const f4 vin = *reinterpret_cast<const f4*>(Vin + idx);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = fmaf(noise, vin[e], o[e]);
-    }
     *reinterpret_cast<f4*>(out + idx) = o;
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (i + e < m) out[idx + e] = add_noise ? fmaf(noise, Vin[idx + e], o[e]) : o[e];
+      if (i + e < m) out[idx + e] = o[e];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// One unpreconditioned CG step of a small system around the tile product
+// (cg_solver.mojo:108-255, the arithmetic of k_reduce_splits4, k_coldot_w,
+// k_cg_update_w and k_cg_pupdate_w): a workgroup per column adds the product's
+// split partials (Ap), forms alpha, updates x and r, forms beta, updates p,
+// and packs the new p as the next product's right-hand side, so an iteration
+// is two launches instead of eight.  At a few thousand points every one of
+// those kernels sits on its launch and latency floor (3 to 5 us each; n =
+// 2000, 11 columns: 25 us beside the tile kernel, now 9.4); a column's traffic
+// through one CU (splits + 7 vectors) costs more than the launches saved
+// from kSmallCgMax on.
+// ---------------------------------------------------------------------------
+constexpr int kSmallCgThreads = 1024;
+
+// Sum over the workgroup, waves added in order; every thread gets it.
+__device__ __forceinline__ double small_cg_sum(double v, double* sm) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = sm[0];
+#pragma unroll
+  for (int w = 1; w < kSmallCgThreads / 64; ++w) t += sm[w];
+  return t;
+}
+
+// NQ quads of consecutive rows per thread (n <= 4096 NQ).  vp: packed
+// right-hand sides (h8 operand of the tile kernel; padded fp32 vector when
+// single), whose columns past ncols and rows past n are already zero.
+template <int NQ>
+__global__ __launch_bounds__(kSmallCgThreads) void k_cg_small(
+    const float* __restrict__ partial, int splits, int cpad, int64_t mpad, int n, float os,
+    float noise, const float* __restrict__ dvec, float* __restrict__ x, float* __restrict__ r,
+    float* __restrict__ p, SmallCgScalars s, int iter, int max_tridiag, int single,
+    uint32_t* __restrict__ colmax, void* __restrict__ vp) {
+  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+  __shared__ double sm[kSmallCgThreads / 64];
+  __shared__ uint32_t smax[kSmallCgThreads / 64];
+  const int c = blockIdx.x, ncols = gridDim.x;
+  const int64_t off = (int64_t)c * n;
+  const float* pc = partial + (int64_t)c * mpad;
+  const int64_t sstride = (int64_t)cpad * mpad;
+  float pv[NQ][4], rv[NQ][4], av[NQ][4], xv[NQ][4];
+  // every load of the launch is issued before the first reduction: the vectors
+  // come from other XCDs' caches or memory (~2 us)
+  const float rz = s.rz[c];
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    const int i = 4 * ((int)threadIdx.x + kSmallCgThreads * k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int j = min(i + e, n - 1);
+      pv[k][e] = p[off + j];
+      rv[k][e] = r[off + j];
+      xv[k][e] = x[off + j];
+    }
+  }
+  double dot = 0.0;
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    const int i = 4 * ((int)threadIdx.x + kSmallCgThreads * k);
+    double tot[4] = {0.0, 0.0, 0.0, 0.0};
+    if (i < n) {
+      int sp = 0;
+      for (; sp + 8 <= splits; sp += 8) {
+        f4 v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = *reinterpret_cast<const f4*>(pc + (sp + q) * sstride + i);
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) tot[e] += v[q][e];
+      }
+      for (; sp < splits; ++sp) {
+        const f4 v = *reinterpret_cast<const f4*>(pc + sp * sstride + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tot[e] += v[e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = i + e < n;
+      if (!in) pv[k][e] = rv[k][e] = 0.0f;
+      float a = (float)((double)os * tot[e] + (double)noise * (double)pv[k][e]);
+      if (dvec) a = fmaf(in ? dvec[i + e] : 0.0f, pv[k][e], a);
+      av[k][e] = in ? a : 0.0f;
+      dot += (double)pv[k][e] * (double)av[k][e];
+    }
+  }
+  // alpha = rz / pAp with the skip rules of k_cg_update_w
+  const float pap = (float)small_cg_sum(dot, sm);
+  const float al = (rz != rz || pap != pap || pap < 1e-10f) ? 0.0f : rz / pap;
+  const bool active = !(al == 0.0f || al != al);
+  double rr = 0.0;
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    const int i = 4 * ((int)threadIdx.x + kSmallCgThreads * k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float pi = pv[k][e], ai = av[k][e];
+      if (i + e < n && active && pi == pi && ai == ai) {
+        x[off + i + e] = xv[k][e] + al * pi;
+        rv[k][e] -= al * ai;
+        r[off + i + e] = rv[k][e];
+      }
+      rr += (double)rv[k][e] * (double)rv[k][e];
+    }
+  }
+  const double rr_sum = small_cg_sum(rr, sm);
+  const float rz_new = (float)rr_sum;
+  float b = 0.0f;
+  if (rz == rz && rz_new == rz_new && rz >= 1e-20f) {
+    b = rz_new / (rz + 1e-20f);
+    if (b < 0.0f || b != b) b = 0.0f;
+  }
+  if (threadIdx.x == 0) {
+    s.rr[c] = rr_sum;
+    s.rz[c] = rz_new != rz_new ? 0.0f : rz_new;
+    if (iter < max_tridiag) {
+      s.hist_alpha[(int64_t)iter * ncols + c] = al;
+      s.hist_beta[(int64_t)iter * ncols + c] = b;
+    }
+  }
+  uint32_t mx = 0;
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    const int i = 4 * ((int)threadIdx.x + kSmallCgThreads * k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float po = pv[k][e], ri = rv[k][e];
+      pv[k][e] = (b == 0.0f || po != po) ? ri : ri + b * po;
+      if (i + e < n) {
+        p[off + i + e] = pv[k][e];
+        mx = max(mx, __float_as_uint(fabsf(pv[k][e])));
+      }
+    }
+  }
+  if (single) {
+    float* out = reinterpret_cast<float*>(vp);
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      const int i = 4 * ((int)threadIdx.x + kSmallCgThreads * k);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i + e < n) out[i + e] = pv[k][e];
+    }
+    return;
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
+  if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  mx = smax[0];
+#pragma unroll
+  for (int w = 1; w < kSmallCgThreads / 64; ++w) mx = max(mx, smax[w]);
+  if (threadIdx.x == 0) colmax[c] = mx;
+  const int shift = col_shift(mx);
+  // rows i .. i + 3 are elements 4 h .. 4 h + 3 of one lane's operand (k_pack_rhs16)
+  h4* out = reinterpret_cast<h4*>(vp);
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    const int i = 4 * ((int)threadIdx.x + kSmallCgThreads * k);
+    if (i >= n) continue;
+    h4 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float v = i + e < n ? ldexpf(pv[k][e], shift) : 0.0f;
+      hi[e] = (_Float16)v;
+      lo[e] = (_Float16)(v - (float)hi[e]);
+    }
+    const int u = i >> 5, h = (i >> 4) & 1, lane = (c & 15) + 16 * ((i >> 2) & 3);
+    out[(((int64_t)u * 2 + 0) * 64 + lane) * 2 + h] = hi;
+    out[(((int64_t)u * 2 + 1) * 64 + lane) * 2 + h] = lo;
   }
 }
 
@@ -2420,6 +2603,68 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
       MGP_HIP_CHECK(hipGetLastError());
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Small CG systems: host side.
+// ---------------------------------------------------------------------------
+bool small_cg_route(int kind, const PackedPoints& pts, int ncols) {
+  if (ncols < 1 || ncols > 16 || pts.n < 1 || pts.n > kSmallCgMax) return false;
+  if (!gram_form_ok(kind, pts, pts)) return false;
+  return !symmetric_route_taken(pts, ncols);
+}
+
+void SmallCg::begin(const float* p) {
+  MGP_REQUIRE(small_cg_route(a.kind, *pts, a.ncols), "not a small CG system");
+  const int64_t col_pairs = pts->ntiles / 2, npad = pts->ntiles * 16;
+  const int ncg = a.ncols == 1 ? 0 : 1, nc = a.ncols;
+  const TilePlan plan = tile_plan(pts->ntiles, col_pairs, ncg, nc);
+  R = plan.R;
+  pairs_per_split = ceil_div(col_pairs, plan.splits);
+  splits = ceil_div(col_pairs, pairs_per_split);
+  ws->partial.ensure((size_t)splits * (ncg ? 16 : 1) * npad);
+  if (ncg == 0) {
+    vp = ws->vpack.ensure((size_t)npad);
+    hipLaunchKernelGGL(k_pad_vec, dim3((unsigned)ceil_div(npad, 256)), dim3(256), 0, st, p, a.n,
+                       npad, ws->vpack.ptr);
+  } else {
+    colmax = ws->colmax.ensure(64);
+    const int chunks = (int)std::min<int64_t>(ceil_div(a.n, 4096), 64);
+    uint32_t* cpart = ws->colmax_part.ensure((size_t)64 * chunks);
+    const int vec4 = (a.n % 4 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0) ? 1 : 0;
+    hipLaunchKernelGGL(k_col_absmax_part, dim3((unsigned)chunks, (unsigned)nc), dim3(256), 0, st,
+                       p, a.n, vec4, cpart);
+    hipLaunchKernelGGL(k_col_absmax_final, dim3((unsigned)nc), dim3(64), 0, st, cpart, chunks,
+                       colmax);
+    const int64_t total = col_pairs * 64;
+    vp = ws->vpack.ensure((size_t)total * 2 * 4);
+    hipLaunchKernelGGL(k_pack_rhs16, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, p,
+                       a.n, nc, 1, col_pairs, colmax, vec4, reinterpret_cast<h8*>(vp));
+  }
+  MGP_HIP_CHECK(hipGetLastError());
+}
+
+void SmallCg::step(float* x, float* r, float* p, const SmallCgScalars& s, int iter,
+                   int max_tridiag) {
+  const int64_t col_pairs = pts->ntiles / 2, mpad = pts->ntiles * 16;
+  const int ncg = a.ncols == 1 ? 0 : 1, cpad = ncg ? 16 : 1;
+  TileFn fn = a.kind == KIND_RBF        ? pick_tile<KIND_RBF>(pts->kb, ncg, R)
+              : a.kind == KIND_MATERN32 ? pick_tile<KIND_MATERN32>(pts->kb, ncg, R)
+                                        : pick_tile<KIND_MATERN52>(pts->kb, ncg, R);
+  MGP_REQUIRE(fn != nullptr, "no tile kernel for this shape");
+  hipLaunchKernelGGL(fn, dim3((unsigned)ceil_div(pts->ntiles, (int64_t)kWaves * R),
+                              (unsigned)splits),
+                     dim3(256), 0, st, reinterpret_cast<const h8*>(pts->B.ptr), pts->ntiles,
+                     reinterpret_cast<const h8*>(pts->A.ptr), (const void*)vp, col_pairs,
+                     pairs_per_split, (int64_t)0, a.m, a.ncols, a.outputscale, a.noise, colmax,
+                     (const float*)nullptr, (float*)nullptr, ws->partial.ptr, mpad, cpad);
+  MGP_HIP_CHECK(hipGetLastError());
+  auto k = a.n <= 4096 ? k_cg_small<1> : a.n <= 8192 ? k_cg_small<2> : k_cg_small<4>;
+  static_assert(kSmallCgMax <= 4 * 4 * kSmallCgThreads, "quads per thread");
+  hipLaunchKernelGGL(k, dim3((unsigned)a.ncols), dim3(kSmallCgThreads), 0, st, ws->partial.ptr,
+                     (int)splits, cpad, mpad, (int)a.n, a.outputscale, a.noise, noise_vec, x, r, p,
+                     s, iter, max_tridiag, ncg == 0 ? 1 : 0, colmax, vp);
+  MGP_HIP_CHECK(hipGetLastError());
 }
 
 void fill_cross(int kind, float outputscale, const PackedPoints& rows, int64_t r0,
