@@ -190,7 +190,7 @@ MGP_API int mgp_gradient_matvec(void* handle, const float* V, int ncols, float* 
 /* out[p] = sum_{a,b} dK_p[a,b] sum_c Lf[c*n+a] Rf[c*n+b] for every kernel
  * parameter p (engine layout), Lf and Rf host [ncols][n], out host [P].  The
  * trace routine of mgp_bbmm_eval's gradient step (the matrix-core trace where
- * its route applies, MGP_GRAD_MFMA as there, else the pair loop) on
+ * its route applies, MGP_GRAD_MFMA as there, else by differences) on
  * caller-given weight columns, in place of the reference's per-parameter
  * fused_gradient_matvec + kernel_dot_*_vs_strided pair
  * (combined_inv_quad_logdet.mojo:715-800).  Internal to the reference (no

@@ -257,14 +257,26 @@ struct GradTraceWorkspace {
 // with W = Lf^T Rf over ncols columns ([ncols][n] device arrays), z the
 // scaled coordinates and h the kernel's lengthscale factor (RBF k/os,
 // Matern-3/2 3 e^{-u}, Matern-5/2 (5/3)(1 + u) e^{-u}), the same sums as the
-// pair-loop trace.  Only the symmetric part of W meets the symmetric h dz^2,
+// difference trace.  Only the symmetric part of W meets the symmetric h dz^2,
 // so each unordered block pair is formed once with (W + W^T).  The
-// environment variable MGP_GRAD_MFMA=0 keeps the pair-loop trace, =1 takes
+// environment variable MGP_GRAD_MFMA=0 keeps the difference trace, =1 takes
 // this one for any n the route allows.
 bool grad_trace_mfma_route(int kind, const PackedPoints& pts, int d);
 void grad_trace_mfma(int kind, const PackedPoints& pts, int d, const float* Lf,
                      const float* Rf, int ncols, double* acc, GradTraceWorkspace& ws,
                      hipStream_t st);
-constexpr int64_t kGradMfmaMinPoints = 4096;
+// Taken where it beats the difference form: per pair it saves ~d instructions,
+// per trace it packs its operands and reads partials back (Matern-5/2 ARD, 11
+// columns, us on the matrix cores / by differences: d = 2 240 / 222 at n =
+// 16000, 406 / 424 at 24000; d = 8 165 / 131 at 8000, 239 / 297 at 16000; d =
+// 16 130 / 103 at 4000, 166 / 171 at 8000).
+constexpr double kGradMfmaMinWork = 1.05e9;  // n^2 (d + 1)
+
+// The same sums from per-dimension differences (grad_pair.hip), for every kind
+// and up to 32 dimensions: acc[q] (q < d for ARD kernels, else one sum over
+// the dimensions), then the k / os sum; at least one column.
+void grad_trace_pairs(int kind, bool ard, const PackedPoints& pts, int d, const float* Lf,
+                      const float* Rf, int ncols, double* acc_host, GradTraceWorkspace& ws,
+                      hipStream_t st);
 
 }  // namespace mgp

@@ -1272,9 +1272,8 @@ __global__ __launch_bounds__(64 * kSymWaves) void k_sym_tile(
 // ---------------------------------------------------------------------------
 // Gradient traces on the matrix cores (Gram-form kernels).
 //
-// The pair-loop trace (solver.hip k_grad_trace) spends ~90 VALU instructions
-// per pair on per-dimension differences, the 16-column dot g_ab = sum_c
-// Lf_ca Rf_cb and the per-dimension accumulation.  Here, per 16x16 tile:
+// The difference trace (grad_pair.hip) spends 4 d + ~10 VALU instructions per
+// pair on the differences, the value and the per-dimension accumulation.  Here, per 16x16 tile:
 //   * the scaled squared distance comes from the Gram-form distance MFMAs of
 //     the product kernels (KB per tile);
 //   * D = W + W^T comes from one K=32 contraction of [Rf'_b | Lf'_b] with
@@ -1391,7 +1390,7 @@ __global__ void k_pack_grad_zz(const float* __restrict__ Z, int64_t n, int d, in
   ZZ[((u * 2 * qg + gr) * 2 + 1) * 64 + lane] = lo;
 }
 
-// kv = k/os and h (the derivative factor of the pair-loop trace) from the
+// kv = k/os and h (the derivative factor of the difference trace) from the
 // scaled squared distance s.
 template <int KIND>
 __device__ __forceinline__ void grad_factors(float s, float clampv, float& kv, float& h) {
@@ -2365,7 +2364,7 @@ bool grad_trace_mfma_route(int kind, const PackedPoints& pts, int d) {
   if (!gram_form_ok(kind, pts, pts)) return false;
   const int64_t nb = ceil_div(std::max<int64_t>(pts.n, 1), kGtRows);
   if (nb * kGtRows > pts.ntiles_alloc * 16) return false;
-  return mode > 0 || pts.n >= kGradMfmaMinPoints;
+  return mode > 0 || (double)pts.n * (double)pts.n * (d + 1) >= kGradMfmaMinWork;
 }
 
 namespace {

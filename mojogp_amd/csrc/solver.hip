@@ -1194,144 +1194,6 @@ __global__ __launch_bounds__(256) void k_low_rank_sample(
   }
 }
 
-// ------------------------------------------------------------- gradients
-// Block: 256 rows a; LDS tiles of 64 column points b.  Per pair the reference
-// derivatives (see oracle/kernels.py for the closed forms) are weighted by
-// g_ab = sum_c Lf[c][a] Rf[c][b] and accumulated; fp32 within a tile, fp64
-// across tiles.  part[block][p] (p: per-dim lengthscale terms, then os term).
-constexpr int kGradTile = 64;
-
-template <int KIND, int DM, bool ARD>
-__global__ __launch_bounds__(256) void k_grad_trace(
-    const float* __restrict__ Z, int d, int64_t n, const float* __restrict__ Lf,
-    const float* __restrict__ Rf, int ncols, int c0, double* __restrict__ part,
-    int nterms) {
-  __shared__ float zb[kGradTile][DM + 1];
-  __shared__ float rb[kGradTile][17];
-  __shared__ double sm[4];
-  const int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool live = a < n;
-  const int cn = min(16, ncols - c0);
-  // column range of this split (whole tiles)
-  const int64_t tiles = (n + kGradTile - 1) / kGradTile;
-  const int64_t tps = (tiles + gridDim.y - 1) / gridDim.y;
-  const int64_t jb = min(n, (int64_t)blockIdx.y * tps * kGradTile);
-  const int64_t je = min(n, jb + tps * kGradTile);
-  float za[DM];
-#pragma unroll
-  for (int k = 0; k < DM; ++k) za[k] = (live && k < d) ? Z[a * d + k] : 0.0f;
-  float la[16];
-#pragma unroll
-  for (int c = 0; c < 16; ++c) la[c] = (live && c < cn) ? Lf[(int64_t)(c0 + c) * n + a] : 0.0f;
-  constexpr int NT = ARD ? DM : 1;
-  double accd[NT + 1];
-#pragma unroll
-  for (int t = 0; t <= NT; ++t) accd[t] = 0.0;
-  for (int64_t b0 = jb; b0 < je; b0 += kGradTile) {
-    __syncthreads();
-    for (int t = threadIdx.x; t < kGradTile * DM; t += blockDim.x) {
-      const int bb = t / DM, k = t - bb * DM;
-      const int64_t b = b0 + bb;
-      zb[bb][k] = (b < je && k < d) ? Z[b * d + k] : 0.0f;
-    }
-    for (int t = threadIdx.x; t < kGradTile * 16; t += blockDim.x) {
-      const int bb = t / 16, c = t - bb * 16;
-      const int64_t b = b0 + bb;
-      rb[bb][c] = (b < je && c < cn) ? Rf[(int64_t)(c0 + c) * n + b] : 0.0f;
-    }
-    __syncthreads();
-    float acc[NT + 1];
-#pragma unroll
-    for (int t = 0; t <= NT; ++t) acc[t] = 0.0f;
-    const int cnt = (int)min((int64_t)kGradTile, je - b0);
-    for (int bb = 0; bb < cnt; ++bb) {
-      float dz2[DM];
-      float r2 = 0.0f;
-#pragma unroll
-      for (int k = 0; k < DM; ++k) {
-        const float df = za[k] - zb[bb][k];
-        dz2[k] = df * df;
-        r2 += dz2[k];
-      }
-      float kv, h;
-      if constexpr (KIND == KIND_RBF) {
-        kv = __builtin_amdgcn_exp2f(-fmaxf(r2, 0.0f));  // not clamped
-        h = kv;
-      } else if constexpr (KIND == KIND_MATERN12) {
-        // h = log2(e) k / r with the reference's floored r = sqrt(r^2 + 1e-20);
-        // the exponent is clamped for ARD only (exp2_limit)
-        const float u = __builtin_amdgcn_sqrtf(fmaxf(r2, 0.0f));
-        kv = __builtin_amdgcn_exp2f(ARD ? -fminf(u, kExp2Clamp) : -u);
-        h = kLog2e * kv / __builtin_amdgcn_sqrtf(fmaxf(r2, 0.0f) + kM12RFloor);
-      } else if constexpr (KIND == KIND_MATERN32) {
-        const float u = __builtin_amdgcn_sqrtf(fmaxf(r2, 0.0f));
-        const float e = __builtin_amdgcn_exp2f(-fminf(u, kExp2Clamp));
-        kv = fmaf(u, kLn2, 1.0f) * e;
-        h = 3.0f * e;
-      } else {
-        const float u = __builtin_amdgcn_sqrtf(fmaxf(r2, 0.0f));
-        const float e = __builtin_amdgcn_exp2f(-fminf(u, kExp2Clamp));
-        kv = fmaf(u, fmaf(u, kLn2 * kLn2 / 3.0f, kLn2), 1.0f) * e;
-        h = (5.0f / 3.0f) * fmaf(u, kLn2, 1.0f) * e;
-      }
-      float g = 0.0f;
-#pragma unroll
-      for (int c = 0; c < 16; ++c) g = fmaf(la[c], rb[bb][c], g);
-      const float hg = h * g;
-      acc[NT] = fmaf(kv, g, acc[NT]);
-      if constexpr (ARD) {
-#pragma unroll
-        for (int k = 0; k < DM; ++k) acc[k] = fmaf(hg, dz2[k], acc[k]);
-      } else {
-        acc[0] = fmaf(hg, r2, acc[0]);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t <= NT; ++t) accd[t] += (double)acc[t];
-  }
-  // Block reduction of each term.
-  for (int t = 0; t < nterms; ++t) {
-    const int src = (t == nterms - 1) ? NT : t;
-    double v = 0.0;
-#pragma unroll
-    for (int q = 0; q <= NT; ++q)
-      if (q == src) v = accd[q];
-    const double tot = block_sum_d(live ? v : 0.0, sm);
-    if (threadIdx.x == 0)
-      part[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * nterms + t] = tot;
-  }
-}
-
-// Column splits of the gradient pair loop: enough blocks to fill the chip
-// (>= 2048 with the row blocks) while every split keeps >= 1024 columns.
-static int grad_splits(int64_t n) {
-  const int64_t rows = ceil_div(n, 256);
-  return (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(2048, rows), ceil_div(n, 1024)));
-}
-
-template <int KIND, bool ARD>
-void launch_grad(int dm, const float* Z, int d, int64_t n, const float* Lf,
-                 const float* Rf, int ncols, int c0, double* part, int nterms,
-                 hipStream_t st) {
-  const dim3 grid((unsigned)ceil_div(n, 256), (unsigned)grad_splits(n));
-  switch (dm) {
-#define MGP_GRAD_CASE(DMV)                                                           \
-  case DMV:                                                                         \
-    hipLaunchKernelGGL((k_grad_trace<KIND, DMV, ARD>), grid, dim3(256), 0, st, Z, d, \
-                       n, Lf, Rf, ncols, c0, part, nterms);                         \
-    break;
-    MGP_GRAD_CASE(1)
-    MGP_GRAD_CASE(2)
-    MGP_GRAD_CASE(4)
-    MGP_GRAD_CASE(8)
-    MGP_GRAD_CASE(16)
-    MGP_GRAD_CASE(32)
-#undef MGP_GRAD_CASE
-    default:
-      throw Error(ST_INVALID, "unsupported gradient dimension bucket");
-  }
-}
-
 // ------------------------------------------------------------- Lanczos
 __global__ void k_multi_dot_part(const float* __restrict__ Q, const float* __restrict__ w,
                                  int64_t n, int nb, double* __restrict__ part) {
@@ -1900,7 +1762,7 @@ void gradient_traces(const Provider& pv, const float* Lf, const float* Rf, int n
   const double os = (double)pv.outputscale();
   const int nls = pv.ard ? d : 1;
   if (grad_trace_mfma_route(pv.kind, pv.train, d)) {
-    // Matrix-core trace: per-dimension sums, then the pair-loop's layout.
+    // Matrix-core trace: per-dimension sums, then the difference trace's layout.
     std::vector<double> acc(d + 1, 0.0);
     grad_trace_mfma(pv.kind, pv.train, d, Lf, Rf, ncols, acc.data(), pv.gtws, st);
     double iso = 0.0;
@@ -1910,33 +1772,10 @@ void gradient_traces(const Provider& pv, const float* Lf, const float* Rf, int n
     g_host[nls] = acc[d];
     return;
   }
-  const int dm = d <= 1 ? 1 : d <= 2 ? 2 : d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : 32;
   const int nterms = pv.ard ? d + 1 : 2;
-  const int64_t nblk = ceil_div(pv.n, 256) * grad_splits(pv.n);
-  DevBuf<double> part;
-  part.ensure((size_t)nblk * nterms);
-  std::vector<double> acc(nterms, 0.0), hpart((size_t)nblk * nterms);
-  for (int c0 = 0; c0 < ncols; c0 += 16) {
-    if (pv.kind == KIND_RBF) {
-      if (pv.ard) launch_grad<KIND_RBF, true>(dm, pv.train.z.ptr, d, pv.n, Lf, Rf, ncols, c0, part.ptr, nterms, st);
-      else launch_grad<KIND_RBF, false>(dm, pv.train.z.ptr, d, pv.n, Lf, Rf, ncols, c0, part.ptr, nterms, st);
-    } else if (pv.kind == KIND_MATERN12) {
-      if (pv.ard) launch_grad<KIND_MATERN12, true>(dm, pv.train.z.ptr, d, pv.n, Lf, Rf, ncols, c0, part.ptr, nterms, st);
-      else launch_grad<KIND_MATERN12, false>(dm, pv.train.z.ptr, d, pv.n, Lf, Rf, ncols, c0, part.ptr, nterms, st);
-    } else if (pv.kind == KIND_MATERN32) {
-      if (pv.ard) launch_grad<KIND_MATERN32, true>(dm, pv.train.z.ptr, d, pv.n, Lf, Rf, ncols, c0, part.ptr, nterms, st);
-      else launch_grad<KIND_MATERN32, false>(dm, pv.train.z.ptr, d, pv.n, Lf, Rf, ncols, c0, part.ptr, nterms, st);
-    } else {
-      if (pv.ard) launch_grad<KIND_MATERN52, true>(dm, pv.train.z.ptr, d, pv.n, Lf, Rf, ncols, c0, part.ptr, nterms, st);
-      else launch_grad<KIND_MATERN52, false>(dm, pv.train.z.ptr, d, pv.n, Lf, Rf, ncols, c0, part.ptr, nterms, st);
-    }
-    MGP_HIP_CHECK(hipGetLastError());
-    MGP_HIP_CHECK(hipMemcpyAsync(hpart.data(), part.ptr, hpart.size() * sizeof(double),
-                                 hipMemcpyDeviceToHost, st));
-    MGP_HIP_CHECK(hipStreamSynchronize(st));
-    for (int64_t b = 0; b < nblk; ++b)
-      for (int t = 0; t < nterms; ++t) acc[t] += hpart[(size_t)b * nterms + t];
-  }
+  std::vector<double> acc(nterms, 0.0);
+  if (ncols > 0)
+    grad_trace_pairs(pv.kind, pv.ard, pv.train, d, Lf, Rf, ncols, acc.data(), pv.gtws, st);
   // Convert pair sums (scaled coordinates z = (x - c) * kernel_scale / ls) to
   // parameter derivatives: dk/dl_d = os h (dx_d)^2 / l_d^3 = os h dz_d^2 / (s^2 l_d).
   for (int q = 0; q < nls; ++q)
