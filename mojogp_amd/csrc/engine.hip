@@ -47,12 +47,26 @@ void part_to_float(const double* part, int nb, int ncols, float* out, hipStream_
 }
 
 // --------------------------------------------------- single right-hand-side CG
-// Scalars: s[0] rr_old, s[1] initial residual norm, s[2] alpha, s[3] beta.
+// Scalars: s[0], s[2] rr (one of them the current, the other the next one),
+// s[1] initial residual norm.  Every workgroup forms alpha and beta itself
+// from the partials (the same fixed-order sum, so the same value); the first
+// one stores what the next launch reads, in the scalar this launch does not
+// read.  `done` may be set by the first workgroup while others of the same
+// launch start: they come to the same decision either way.
+
+// Sum of part[0 .. nb) by one wave's lanes (every lane gets it).
+__device__ __forceinline__ double a1_part_sum(const double* __restrict__ part, int nb) {
+  double s = 0.0;
+#pragma unroll 4
+  for (int b = threadIdx.x & 63; b < nb; b += 64) s += part[b];
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
+  return s;
+}
+
 __global__ void k_a1_init(const double* __restrict__ part, int nb, float* s, int* done) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double acc = 0.0;
-  for (int b = 0; b < nb; ++b) acc += part[b];
-  const float rr = (float)acc;
+  const float rr = (float)a1_part_sum(part, nb);
+  if (threadIdx.x != 0) return;
   float init = sqrtf(rr);
   if (init < 1e-20f) init = 1.0f;
   s[0] = rr;
@@ -60,30 +74,22 @@ __global__ void k_a1_init(const double* __restrict__ part, int nb, float* s, int
   *done = 0;
 }
 
-__global__ void k_a1_alpha(const double* __restrict__ part, int nb, float* s, int* done) {
-  if (threadIdx.x != 0 || blockIdx.x != 0 || *done) return;
-  double acc = 0.0;
-  for (int b = 0; b < nb; ++b) acc += part[b];
-  const float pap = (float)acc;
-  if (pap != pap || pap < 1e-10f) {
-    *done = 1;
-    return;
-  }
-  const float a = s[0] / pap;
-  if (a != a) {
-    *done = 1;
-    return;
-  }
-  s[2] = a;
-}
-
-__global__ void k_a1_update(float* __restrict__ x, float* __restrict__ r,
-                            const float* __restrict__ p, const float* __restrict__ Ap,
-                            int64_t n, int nb, const float* __restrict__ s,
-                            const int* __restrict__ done, double* __restrict__ rr_part) {
+// alpha = rr / p.Ap; x += alpha p, r -= alpha Ap, r.r partials.  One
+// workgroup per chunk of the nb of a1_chunk rows.
+__global__ __launch_bounds__(256) void k_a1_update(float* __restrict__ x, float* __restrict__ r,
+                                                   const float* __restrict__ p,
+                                                   const float* __restrict__ Ap, int64_t n, int nb,
+                                                   const double* __restrict__ pap_part,
+                                                   const float* __restrict__ rr_old, int* done,
+                                                   double* __restrict__ rr_part) {
   __shared__ double sm[4];
   if (*done) return;  // uniform
-  const float a = s[2];
+  const float pap = (float)a1_part_sum(pap_part, nb);
+  const float a = rr_old[0] / pap;
+  if (pap != pap || pap < 1e-10f || a != a) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *done = 1;
+    return;
+  }
   const int64_t chunk = (n + nb - 1) / nb;
   const int64_t i0 = (int64_t)blockIdx.x * chunk, i1 = min(n, i0 + chunk);
   double acc = 0.0;
@@ -104,31 +110,30 @@ __global__ void k_a1_update(float* __restrict__ x, float* __restrict__ r,
   }
 }
 
-__global__ void k_a1_beta(const double* __restrict__ part, int nb, float tol, float* s,
-                          int* done) {
-  if (threadIdx.x != 0 || blockIdx.x != 0 || *done) return;
-  double acc = 0.0;
-  for (int b = 0; b < nb; ++b) acc += part[b];
-  const float rr_new = (float)acc;
-  if (sqrtf(rr_new) / s[1] < tol) {
-    *done = 1;
+// Stop test, beta = rr_new / rr_old, p = r + beta p; rr_new stored for the
+// next iteration.
+__global__ __launch_bounds__(256) void k_a1_pupdate(float* __restrict__ p,
+                                                    const float* __restrict__ r, int64_t n,
+                                                    const double* __restrict__ rr_part, int nb,
+                                                    float tol, const float* __restrict__ rr_old_p,
+                                                    const float* __restrict__ init,
+                                                    float* __restrict__ rr_next, int* done) {
+  if (*done) return;
+  const float rr_new = (float)a1_part_sum(rr_part, nb);
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (sqrtf(rr_new) / init[0] < tol) {
+    if (first) *done = 1;
     return;
   }
-  const float rr_old = s[0];
+  const float rr_old = rr_old_p[0];
   float beta = 0.0f;
   if (rr_old >= 1e-20f) {
     beta = rr_new / (rr_old + 1e-20f);
     if (beta < 0.0f || beta != beta) beta = 0.0f;
   }
-  s[3] = beta;
-  s[0] = rr_new;
-}
-
-__global__ void k_a1_pupdate(float* __restrict__ p, const float* __restrict__ r, int64_t n,
-                             const float* __restrict__ s, const int* __restrict__ done) {
-  if (*done) return;
+  if (first) rr_next[0] = rr_new;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = r[i] + s[3] * p[i];
+  if (i < n) p[i] = r[i] + beta * p[i];
 }
 
 // ---------------------------------------- independent single-RHS CG per column
@@ -232,20 +237,116 @@ __global__ void k_mc_alldone(int C, int* done) {
   done[C] = all;
 }
 
-// Lanczos three-term recurrence: w -= a v (+ b vprev).
-__global__ void k_three_term(float* __restrict__ w, const float* __restrict__ v,
-                             const float* __restrict__ vprev, float a, float b, int64_t n) {
+// ---------------------------------------------------------------- Lanczos
+// One iteration j without a host round trip: the scalars stay on the device
+// (ab[j] = alpha_j, ab[r + j] = beta_j; stop != 0 after a breakdown, from
+// when on every kernel returns).
+
+// a = v.w from the partials; w -= a v (+ beta_{j-1} vprev).
+__global__ __launch_bounds__(256) void k_lz_three_term(
+    float* __restrict__ w, const float* __restrict__ v, const float* __restrict__ vprev,
+    const double* __restrict__ part, int nb, int j, int r, float* __restrict__ ab,
+    const int* __restrict__ stop, int64_t n) {
+  if (*stop) return;
+  const float a = (float)a1_part_sum(part, nb);
+  if (blockIdx.x == 0 && threadIdx.x == 0) ab[j] = a;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   float x = w[i] - a * v[i];
-  if (vprev) x -= b * vprev[i];
+  if (vprev) x -= ab[r + j - 1] * vprev[i];
   w[i] = x;
 }
 
-__global__ void k_scale_into(float* __restrict__ dst, const float* __restrict__ src, float inv,
-                             int64_t n) {
+// The second re-orthogonalisation pass runs only where the first one saw an
+// inner product >= 1e-5 (coef: that pass's products; null: the first pass),
+// or one that is not small against the last beta (bprev, null at j = 0): once
+// the Krylov space is exhausted w is rounding noise of that size, which one
+// pass leaves far from orthogonal and the recurrence then blows up.
+__device__ __forceinline__ bool lz_skip(const double* __restrict__ coef, int nvec,
+                                        const float* __restrict__ bprev,
+                                        const int* __restrict__ stop) {
+  if (*stop) return true;
+  if (!coef) return false;
+  double mx = 0.0;
+  for (int k = threadIdx.x & 63; k < nvec; k += 64) mx = fmax(mx, fabs(coef[k]));
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  return mx < 1e-5 && (!bprev || mx < 1e-2 * (double)bprev[0]);
+}
+
+// part[k nb + b] = Q_k . w over chunk b (grid = (nb, nvec)).
+__global__ __launch_bounds__(256) void k_lz_dots(const float* __restrict__ Q,
+                                                 const float* __restrict__ w, int64_t n, int nb,
+                                                 const double* __restrict__ coef,
+                                                 const float* __restrict__ bprev,
+                                                 const int* __restrict__ stop,
+                                                 double* __restrict__ part) {
+  __shared__ double sm[4];
+  if (lz_skip(coef, gridDim.y, bprev, stop)) return;
+  const int64_t chunk = (n + nb - 1) / nb;
+  const int64_t i0 = (int64_t)blockIdx.x * chunk, i1 = min(n, i0 + chunk);
+  const float* q = Q + (int64_t)blockIdx.y * n;
+  double acc = 0.0;
+#pragma unroll 4
+  for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) acc += (double)q[i] * (double)w[i];
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o);
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) part[(int64_t)blockIdx.y * nb + blockIdx.x] = sm[0] + sm[1] + sm[2] + sm[3];
+}
+
+// coef_k = sum_b part[k nb + b] (one wave per k).
+__global__ __launch_bounds__(64) void k_lz_coefs(const double* __restrict__ part, int nb,
+                                                 const double* __restrict__ coef,
+                                                 const float* __restrict__ bprev,
+                                                 const int* __restrict__ stop,
+                                                 double* __restrict__ out) {
+  if (lz_skip(coef, gridDim.x, bprev, stop)) return;
+  const double s = a1_part_sum(part + (int64_t)blockIdx.x * nb, nb);
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
+}
+
+// w -= sum_k c_k Q_k: four threads per row take a quarter of the vectors each.
+__global__ __launch_bounds__(256) void k_lz_axpy(const float* __restrict__ Q, int nvec,
+                                                 const double* __restrict__ c,
+                                                 const double* __restrict__ coef,
+                                                 const float* __restrict__ bprev,
+                                                 const int* __restrict__ stop,
+                                                 float* __restrict__ w, int64_t n) {
+  __shared__ double sm[4][64];
+  if (lz_skip(coef, nvec, bprev, stop)) return;
+  const int t = threadIdx.x & 63, grp = threadIdx.x >> 6;
+  const int64_t i = (int64_t)blockIdx.x * 64 + t;
+  const int k0 = nvec * grp / 4, k1 = nvec * (grp + 1) / 4;
+  double s = 0.0;
+  if (i < n) {
+#pragma unroll 8
+    for (int k = k0; k < k1; ++k) s += c[k] * (double)Q[(int64_t)k * n + i];
+  }
+  sm[grp][t] = s;
+  __syncthreads();
+  if (grp == 0 && i < n) w[i] = (float)((double)w[i] - (s + sm[1][t] + sm[2][t] + sm[3][t]));
+}
+
+// beta_j = |w| from the partials; Q_{j+1} = w / beta_j (also into vnext when
+// given), or the stop flag on a breakdown.
+__global__ __launch_bounds__(256) void k_lz_next(const float* __restrict__ w,
+                                                 const double* __restrict__ part, int nb, int j,
+                                                 int r, float* __restrict__ ab, int* stop,
+                                                 float* __restrict__ qnext,
+                                                 float* __restrict__ vnext, int64_t n) {
+  if (*stop) return;
+  const float b = sqrtf((float)a1_part_sum(part, nb));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (j < r - 1) ab[r + j] = b;
+    if (b < 1e-10f) *stop = 1;
+  }
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i] / inv;
+  if (i >= n || b < 1e-10f || !qnext) return;
+  const float q = w[i] / b;
+  qnext[i] = q;
+  if (vnext) vnext[i] = q;
 }
 
 __global__ void k_add_scalar(float* __restrict__ y, float s, int64_t n) {
@@ -1009,8 +1110,7 @@ struct AlphaSolve {
 
   AlphaSolve(Provider& pv_, const float* y_host, float mean, int max_iter_, float tol_,
              PredictState& ps, float* p_ext = nullptr, float* Ap_ext = nullptr)
-      : pv(pv_), n(pv_.n), st(pv_.st), nb(reduction_chunks(pv_.n)), max_iter(max_iter_),
-        tol(tol_) {
+      : pv(pv_), n(pv_.n), st(pv_.st), nb(cg_chunks(pv_.n)), max_iter(max_iter_), tol(tol_) {
     x = ps.alpha.ensure(n);
     r.ensure(n);
     p = p_ext ? p_ext : pbuf.ensure(n);
@@ -1027,13 +1127,13 @@ struct AlphaSolve {
     finished = max_iter <= 0;
   }
   void step() {
+    float* rr_old = s.ptr + (it & 1 ? 2 : 0);
+    float* rr_next = s.ptr + (it & 1 ? 0 : 2);
     coldot_partial(p, Ap, n, 1, nb, part.ptr, st);
-    hipLaunchKernelGGL(k_a1_alpha, dim3(1), dim3(64), 0, st, part.ptr, nb, s.ptr, done.ptr);
-    hipLaunchKernelGGL(k_a1_update, dim3(nb), dim3(256), 0, st, x, r.ptr, p, Ap, n, nb, s.ptr,
-                       done.ptr, part.ptr + nb);
-    hipLaunchKernelGGL(k_a1_beta, dim3(1), dim3(64), 0, st, part.ptr + nb, nb, tol, s.ptr,
-                       done.ptr);
-    hipLaunchKernelGGL(k_a1_pupdate, g1(n), dim3(256), 0, st, p, r.ptr, n, s.ptr, done.ptr);
+    hipLaunchKernelGGL(k_a1_update, dim3(nb), dim3(256), 0, st, x, r.ptr, p, Ap, n, nb, part.ptr,
+                       rr_old, done.ptr, part.ptr + nb);
+    hipLaunchKernelGGL(k_a1_pupdate, g1(n), dim3(256), 0, st, p, r.ptr, n, part.ptr + nb, nb, tol,
+                       rr_old, s.ptr + 1, rr_next, done.ptr);
     MGP_HIP_CHECK(hipGetLastError());
     if ((it & 3) == 3 || it == max_iter - 1) {
       int dh = 0;
@@ -1121,23 +1221,29 @@ struct LanczosSolve {
   Provider& pv;
   int64_t n;
   hipStream_t st;
-  int r, nb;
-  DevBuf<float> Q, wbuf;
+  int r, nb, nbd;
+  DevBuf<float> Q, wbuf, ab;
   DevBuf<double> part, coef;
+  DevBuf<int> stop;
   float* w;
-  std::vector<double> alpha, beta, inner;
-  float beta_prev = 0.0f;
+  float* vnext;  // where the next vector also goes (the caller's product input)
+  std::vector<double> alpha, beta;
   int j = 0;
   bool finished = false;
 
-  LanczosSolve(Provider& pv_, int r_, float* w_ext = nullptr)
-      : pv(pv_), n(pv_.n), st(pv_.st), r(r_), nb(reduction_chunks(pv_.n)) {
+  LanczosSolve(Provider& pv_, int r_, float* w_ext = nullptr, float* v_ext = nullptr)
+      : pv(pv_), n(pv_.n), st(pv_.st), r(r_), nb(cg_chunks(pv_.n)), nbd(reduction_chunks(pv_.n)),
+        vnext(v_ext) {
     MGP_REQUIRE(r >= 1 && r <= 1000, "Lanczos rank must be in [1, 1000]");
     Q.ensure((size_t)r * n);
     w = w_ext ? w_ext : wbuf.ensure(n);
-    part.ensure((size_t)(r + 1) * nb + 8);
-    coef.ensure((size_t)r + 1);
+    part.ensure(std::max((size_t)(r + 1) * nbd, (size_t)nb) + 8);
+    coef.ensure((size_t)2 * r);
+    ab.ensure((size_t)2 * r);
+    stop.ensure(1);
     fill(Q.ptr, (int64_t)r * n, 0.0f, st);
+    fill(ab.ptr, (int64_t)2 * r, 0.0f, st);
+    fill(reinterpret_cast<float*>(stop.ptr), 1, 0.0f, st);  // integer 0
     // Deterministic +-1 start vector (jit_prediction.mojo:999-1015).
     std::vector<float> z(n);
     float zsq = 0.0f;
@@ -1154,44 +1260,52 @@ struct LanczosSolve {
     const float zn = std::sqrt(zsq);
     for (int64_t i = 0; i < n; ++i) z[i] /= zn;
     MGP_HIP_CHECK(hipMemcpyAsync(Q.ptr, z.data(), n * sizeof(float), hipMemcpyHostToDevice, st));
+    if (vnext) copy(vnext, Q.ptr, n, st);
     // The start vector's host buffer must outlive the copy.
     MGP_HIP_CHECK(hipStreamSynchronize(st));
-    alpha.assign(r, 0.0);
-    beta.assign(std::max(r - 1, 0), 0.0);
-    inner.assign(r + 1, 0.0);
   }
   const float* vec() const { return Q.ptr + (size_t)j * n; }
   void step() {
     const float* v = vec();
-    const float aj = dot_f(v, w, n, part, st);
-    alpha[j] = aj;
-    hipLaunchKernelGGL(k_three_term, g1(n), dim3(256), 0, st, w, v,
-                       j > 0 ? Q.ptr + (size_t)(j - 1) * n : nullptr, aj, beta_prev, n);
+    const dim3 blk(256);
+    coldot_partial(v, w, n, 1, nb, part.ptr, st);
+    hipLaunchKernelGGL(k_lz_three_term, g1(n), blk, 0, st, w, v,
+                       j > 0 ? Q.ptr + (size_t)(j - 1) * n : nullptr, part.ptr, nb, j, r, ab.ptr,
+                       stop.ptr, n);
     // Full re-orthogonalisation against Q_0..Q_j, at most two passes; the
     // second pass runs only if the first saw an inner product >= 1e-5.
     for (int pass = 0; pass < 2; ++pass) {
-      multi_dot(Q.ptr, j + 1, w, n, part.ptr, nb, coef.ptr, st);
-      MGP_HIP_CHECK(hipMemcpyAsync(inner.data(), coef.ptr, (j + 1) * sizeof(double),
-                                   hipMemcpyDeviceToHost, st));
+      double* c = coef.ptr + (size_t)pass * r;
+      const double* first = pass ? coef.ptr : nullptr;
+      const float* bp = j > 0 ? ab.ptr + r + j - 1 : nullptr;
+      hipLaunchKernelGGL(k_lz_dots, dim3(nbd, j + 1), blk, 0, st, Q.ptr, w, n, nbd, first,
+                         bp, stop.ptr, part.ptr);
+      hipLaunchKernelGGL(k_lz_coefs, dim3(j + 1), dim3(64), 0, st, part.ptr, nbd, first, bp,
+                         stop.ptr, c);
+      hipLaunchKernelGGL(k_lz_axpy, dim3((unsigned)ceil_div(n, 64)), blk, 0, st, Q.ptr, j + 1, c,
+                         first, bp, stop.ptr, w, n);
+    }
+    coldot_partial(w, w, n, 1, nb, part.ptr, st);
+    hipLaunchKernelGGL(k_lz_next, g1(n), blk, 0, st, w, part.ptr, nb, j, r, ab.ptr, stop.ptr,
+                       j + 1 < r ? Q.ptr + (size_t)(j + 1) * n : nullptr, vnext, n);
+    MGP_HIP_CHECK(hipGetLastError());
+    // a breakdown leaves the remaining Q columns zero; looked for now and
+    // then, its later iterations do nothing
+    if ((j & 15) == 15) {
+      int sh = 0;
+      MGP_HIP_CHECK(hipMemcpyAsync(&sh, stop.ptr, sizeof(int), hipMemcpyDeviceToHost, st));
       MGP_HIP_CHECK(hipStreamSynchronize(st));
-      double mx = 0.0;
-      for (int k = 0; k <= j; ++k) mx = std::max(mx, std::fabs(inner[k]));
-      multi_axpy(Q.ptr, j + 1, coef.ptr, w, n, st);
-      if (mx < 1e-5) break;
+      if (sh) finished = true;
     }
-    const float bj = std::sqrt(dot_f(w, w, n, part, st));
-    if (j < r - 1) beta[j] = bj;
-    if (bj < 1e-10f) {  // remaining Q columns stay zero
-      finished = true;
-      return;
-    }
-    if (j + 1 < r)
-      hipLaunchKernelGGL(k_scale_into, g1(n), dim3(256), 0, st, Q.ptr + (size_t)(j + 1) * n, w,
-                         bj, n);
-    beta_prev = bj;
     if (++j >= r) finished = true;
   }
   void finish(PredictState& ps) {
+    std::vector<float> h((size_t)2 * r);
+    MGP_HIP_CHECK(hipMemcpyAsync(h.data(), ab.ptr, h.size() * sizeof(float),
+                                 hipMemcpyDeviceToHost, st));
+    MGP_HIP_CHECK(hipStreamSynchronize(st));
+    alpha.assign(h.begin(), h.begin() + r);
+    beta.assign(h.begin() + r, h.begin() + r + std::max(r - 1, 0));
     std::vector<double> ev, V;
     if (!tridiag_eigh(alpha, beta, ev, &V))
       throw Error(ST_NUMERIC, "Lanczos tridiagonal eigendecomposition did not converge");
@@ -1244,11 +1358,10 @@ int solve_alpha_and_root(Provider& pv, const float* y_host, float mean, int max_
   V2.ensure((size_t)2 * n);
   O2.ensure((size_t)2 * n);
   AlphaSolve a(pv, y_host, mean, max_iter, tol, ps, V2.ptr, O2.ptr);
-  LanczosSolve l(pv, rank, O2.ptr + n);
+  LanczosSolve l(pv, rank, O2.ptr + n, V2.ptr + n);
   *alpha_s = 0.0;
   while (!a.finished || !l.finished) {
     if (!a.finished && !l.finished) {
-      copy(V2.ptr + n, l.vec(), n, pv.st);
       pv.forward(V2.ptr, 2, O2.ptr);
       a.step();
       if (a.finished) *alpha_s = secs_since(t0);

@@ -159,12 +159,6 @@ void gradient_traces(const Provider& pv, const float* Lf, const float* Rf, int n
                      double* g_host, hipStream_t st);
 
 // ---------------------------------------------------------------- Lanczos
-// out[j] = Q_j . w for j < nvec (Q [nvec][n]), fp64 via partials.
-void multi_dot(const float* Q, int nvec, const float* w, int64_t n, double* part,
-               int nb, double* out, hipStream_t st);
-// w -= sum_j coef[j] Q_j
-void multi_axpy(const float* Q, int nvec, const double* coef, float* w, int64_t n,
-                hipStream_t st);
 // S[c*n + i] = sum_k Q[k*n + i] * T[k*r + c]  (n x r times r x r)
 void gemm_nr_rr(const float* Q, const float* T, int64_t n, int r, float* S,
                 hipStream_t st);

@@ -1195,30 +1195,6 @@ __global__ __launch_bounds__(256) void k_low_rank_sample(
 }
 
 // ------------------------------------------------------------- Lanczos
-__global__ void k_multi_dot_part(const float* __restrict__ Q, const float* __restrict__ w,
-                                 int64_t n, int nb, double* __restrict__ part) {
-  __shared__ double sm[4];
-  const int j = blockIdx.y;
-  const int64_t chunk = (n + nb - 1) / nb;
-  const int64_t i0 = (int64_t)blockIdx.x * chunk, i1 = min(n, i0 + chunk);
-  const float* q = Q + (int64_t)j * n;
-  double acc = 0.0;
-  for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x)
-    acc += (double)q[i] * (double)w[i];
-  const double t = block_sum_d(acc, sm);
-  if (threadIdx.x == 0) part[(int64_t)j * nb + blockIdx.x] = t;
-}
-
-__global__ void k_multi_axpy(const float* __restrict__ Q, int nvec,
-                             const double* __restrict__ coef, float* __restrict__ w,
-                             int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s = 0.0;
-  for (int j = 0; j < nvec; ++j) s += coef[j] * (double)Q[(int64_t)j * n + i];
-  w[i] = (float)((double)w[i] - s);
-}
-
 __global__ void k_gemm_nr_rr(const float* __restrict__ Q, const float* __restrict__ T,
                              int64_t n, int r, int c0, float* __restrict__ S) {
   extern __shared__ float ts[];  // [r][16]
@@ -1781,20 +1757,6 @@ void gradient_traces(const Provider& pv, const float* Lf, const float* Rf, int n
   for (int q = 0; q < nls; ++q)
     g_host[q] = os * acc[q] / (s * s * (double)pv.lengthscale(q));
   g_host[nls] = acc[nterms - 1];
-}
-
-void multi_dot(const float* Q, int nvec, const float* w, int64_t n, double* part, int nb,
-               double* out, hipStream_t st) {
-  if (nvec <= 0) return;
-  hipLaunchKernelGGL(k_multi_dot_part, dim3(nb, nvec), dim3(kBlock), 0, st, Q, w, n, nb, part);
-  coldot_finalize(part, nb, nvec, out, st);
-}
-
-void multi_axpy(const float* Q, int nvec, const double* coef, float* w, int64_t n,
-                hipStream_t st) {
-  if (nvec <= 0) return;
-  hipLaunchKernelGGL(k_multi_axpy, grid1(n), dim3(kBlock), 0, st, Q, nvec, coef, w, n);
-  MGP_HIP_CHECK(hipGetLastError());
 }
 
 void gemm_nr_rr(const float* Q, const float* T, int64_t n, int r, float* S, hipStream_t st) {
