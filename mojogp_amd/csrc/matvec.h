@@ -166,6 +166,10 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
                   const PackedPoints& cols, const float* V_dev, float* out_dev,
                   MatvecWorkspace& ws, hipStream_t st, int force_splits = 0);
 constexpr int64_t kSymMinBlocks = 48;
+// One and two right-hand sides run on the symmetric VALU product (k_sym_vec)
+// from this many points on.
+constexpr int kSymVecCols = 2;
+constexpr int64_t kSymVecMinPoints = 5000;
 // True when a square product of the packed points with ncols right-hand
 // sides (own work buffers) runs on the symmetric kernel, whose result for
 // each column does not depend on the other columns.

@@ -243,11 +243,12 @@ __global__ void k_pack_rhs16(const float* __restrict__ V, int64_t n, int ncols,
   P[(base + 1) * 64 + lane] = lo;
 }
 
-// Single right-hand side: zero padded copy.
+// One right-hand side per grid row: zero padded copy.
 __global__ void k_pad_vec(const float* __restrict__ V, int64_t n, int64_t npad,
                           float* __restrict__ P) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < npad) P[j] = j < n ? V[j] : 0.0f;
+  if (j < npad)
+    P[(int64_t)blockIdx.y * npad + j] = j < n ? V[(int64_t)blockIdx.y * n + j] : 0.0f;
 }
 
 // 2^kPScaleLog2 * k / os from the scaled squared distance s, returned as a
@@ -1270,6 +1271,291 @@ __global__ __launch_bounds__(64 * kSymWaves) void k_sym_tile(
 }
 
 // ---------------------------------------------------------------------------
+// Symmetric product with one or two right-hand sides (the solve for alpha, the
+// Lanczos root): every off-diagonal kernel value is formed once, as in
+// k_sym_tile, but both of its products are VALU FMAs (out[i] += k v[j] in the
+// lane that owns row i; out[j] += k v[i] summed over the 16 lanes of a column
+// by DPP adds once per 64 rows), so the values need no fp16 split and no
+// matrix product: ~13 instructions a value against ~10 + 14 % of a wave's time
+// on the matrix cores for 16 padded columns, and half the values of the
+// one-sided kernel.  Blocks of 256 points (4 waves of 4 row tiles) keep the
+// work divisible down to a few thousand points; the transposed partials are
+// n^2 / 128 bytes a column.
+// n = 20000, Matern-5/2: the kernel takes 83 us for one column and 111 for
+// two, the one-sided one 112 and 151; n = 100000: 1.70 ms a product against
+// 2.32 on k_sym_tile.
+// ---------------------------------------------------------------------------
+constexpr int kVecR = 4;                               // row tiles per wave
+constexpr int kVecWaves = 4;                           // waves per workgroup
+constexpr int kVecRows = 16 * kVecR * kVecWaves;       // points per block
+constexpr int kVecPairs = kVecRows / 32;               // column-tile pairs per block
+constexpr int kVecSteps = 2;                           // column-tile pairs per LDS stage
+constexpr int kVecStages = kVecPairs / kVecSteps;      // LDS stages per block
+static_assert((16 * kPackTileAlign) % kVecRows == 0, "blocks must tile the packed points");
+
+// x + (x of the lane that the DPP control names), within rows of 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {
+  const int y = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true);
+  return x + __builtin_bit_cast(float, y);
+}
+__device__ __forceinline__ float row16_sum(float x) {
+  x = dpp_add<0xB1>(x);   // quad_perm [1,0,3,2]
+  x = dpp_add<0x4E>(x);   // quad_perm [2,3,0,1]
+  x = dpp_add<0x141>(x);  // row_half_mirror
+  return dpp_add<0x140>(x);  // row_mirror
+}
+
+// V: [NV][npad] fp32, zero past n (npad = nb 256).  fwd[(split NV + v) npad + i],
+// tp[((b hmax + delta - 1) NV + v) 256 + column], both without os.
+template <int KIND, int KB, int NV>
+__global__ __launch_bounds__(64 * kVecWaves) void k_sym_vec(
+    const h8* __restrict__ Bi, const h8* __restrict__ Aj, const float* __restrict__ V,
+    int64_t npad, int64_t nb, int64_t splits, int64_t sps, int64_t hmax,
+    float* __restrict__ fwd, float* __restrict__ tp) {
+  constexpr int R = kVecR, W = kVecWaves;
+  constexpr int kA = 2 * KB;
+  __shared__ h8 lds[2][kVecSteps * kA][64];
+  __shared__ __align__(16) float tbuf[2][NV][W][32 * kVecSteps];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // XCD-aware order (k_sym_tile)
+  const int64_t per = (int64_t)gridDim.x / kXcds;
+  const int64_t L = (int64_t)(blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+  if (L >= nb * splits) return;
+  const int64_t b = L % nb;
+  const int64_t split = L / nb;
+  const int64_t tile0 = (b * W + wave) * R;
+  const int li = lane & 15;
+  const int lj = 4 * (lane >> 4);
+
+  h8 bi[R][KB];
+  float vi[R][NV];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) bi[r][kb] = Bi[((tile0 + r) * KB + kb) * 64 + lane];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) vi[r][v] = V[v * npad + 16 * (tile0 + r) + li];
+  }
+  __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // row operands before the loop (k_sym_tile)
+  float acc[R][NV];
+  double accd[R][NV];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      acc[r][v] = 0.0f;
+      accd[r][v] = 0.0;
+    }
+  const float clampv = clamp_reg();
+  float one = 1.0f;
+  asm volatile("" : "+v"(one));
+
+  // stages [g0, g1) of the row block's (span + 1) kVecStages
+  const int64_t g0 = split * sps, g1 = min(g0 + sps, (sym_span(b, nb) + 1) * kVecStages);
+  auto stage_u0 = [&](int64_t g) {
+    int64_t J = b + g / kVecStages;
+    if (J >= nb) J -= nb;
+    return J * kVecPairs + (g % kVecStages) * kVecSteps;
+  };
+  auto fill = [&](int st, int64_t u0) __attribute__((always_inline)) {
+    for (int q = wave; q < kVecSteps * kA; q += W)
+      __builtin_amdgcn_global_load_lds((const g_void*)(Aj + (2 * u0 * KB + q) * 64 + lane),
+                                       (lds_void*)&lds[st][q][0], 16, 0, 0);
+  };
+  // One pair of column tiles against the wave's row tiles.  SYM: transposed
+  // sums into tbuf; MASK: the exact zero self-distance of diagonal tiles.
+  auto step = [&](int st, int k, int64_t u, auto mask_tag, auto sym_tag)
+                  __attribute__((always_inline)) {
+    constexpr bool MASK = decltype(mask_tag)::value;
+    constexpr bool SYM = decltype(sym_tag)::value;
+    const int64_t jt0 = 2 * u;
+    h8 a0[KB], a1[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      a0[kb] = lds[st][k * kA + kb][lane];
+      a1[kb] = lds[st][k * kA + KB + kb][lane];
+    }
+    f4 v0[NV], v1[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      v0[v] = *reinterpret_cast<const f4*>(V + v * npad + 16 * jt0 + lj);
+      v1[v] = *reinterpret_cast<const f4*>(V + v * npad + 16 * jt0 + 16 + lj);
+    }
+    auto dist = [&](int r, f4& s0, f4& s1) __attribute__((always_inline)) {
+      s0 = f4{0.f, 0.f, 0.f, 0.f};
+      s1 = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0[kb], bi[r][kb], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1[kb], bi[r][kb], s1, 0, 0, 0);
+      }
+    };
+    float t0[NV][4], t1[NV][4];
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) t0[v][q] = t1[v][q] = 0.0f;
+    f4 S0[2], S1[2];
+    dist(0, S0[0], S1[0]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      f4 s0 = S0[r & 1], s1 = S1[r & 1];
+      if (r + 1 < R) dist(r + 1, S0[(r + 1) & 1], S1[(r + 1) & 1]);
+      if constexpr (MASK) {
+        const int64_t dt = tile0 + r;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (jt0 == dt && li == lj + q) s0[q] = 0.0f;
+          if (jt0 + 1 == dt && li == lj + q) s1[q] = 0.0f;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float f0, g0, f1, g1;
+        kval_scaled<KIND>(s0[q], clampv, one, f0, g0);
+        kval_scaled<KIND>(s1[q], clampv, one, f1, g1);
+        const float k0 = f0 * g0, k1 = f1 * g1;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          acc[r][v] = fmaf(k0, v0[v][q], acc[r][v]);
+          acc[r][v] = fmaf(k1, v1[v][q], acc[r][v]);
+          if constexpr (SYM) {
+            t0[v][q] = fmaf(k0, vi[r][v], t0[v][q]);
+            t1[v][q] = fmaf(k1, vi[r][v], t1[v][q]);
+          }
+        }
+      }
+    }
+    if constexpr (SYM) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        f4 w0, w1;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          w0[q] = row16_sum(t0[v][q]);
+          w1[q] = row16_sum(t1[v][q]);
+        }
+        if (li == 0) {
+          *reinterpret_cast<f4*>(&tbuf[st][v][wave][32 * k + lj]) = w0;
+          *reinterpret_cast<f4*>(&tbuf[st][v][wave][32 * k + 16 + lj]) = w1;
+        }
+      }
+    }
+  };
+  // Adds the waves' transposed sums of stage g and writes them.
+  auto reduce_stage = [&](int64_t g) __attribute__((always_inline)) {
+    const int64_t delta = g / kVecStages;
+    if (delta == 0) return;
+    for (int q = threadIdx.x; q < NV * 32 * kVecSteps; q += 64 * W) {
+      const int v = q / (32 * kVecSteps), j = q - v * (32 * kVecSteps);
+      double t = 0.0;
+#pragma unroll
+      for (int w = 0; w < W; ++w) t += (double)tbuf[g & 1][v][w][j];
+      tp[((b * hmax + delta - 1) * NV + v) * kVecRows + (g % kVecStages) * (32 * kVecSteps) + j] =
+          (float)ldexp(t, -kPScaleLog2);
+    }
+  };
+  auto flush = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        accd[r][v] += (double)acc[r][v];
+        acc[r][v] = 0.0f;
+      }
+  };
+  // The barrier at the top of stage g makes its operands visible, frees the
+  // operand buffer of stage g - 1 and completes that stage's transposed sums,
+  // whose buffer is written again only two stages later.
+  if (g0 < g1) fill((int)(g0 & 1), stage_u0(g0));
+  for (int64_t g = g0; g < g1; ++g) {
+    const int st = (int)(g & 1);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (g + 1 < g1) fill(st ^ 1, stage_u0(g + 1));
+    if (g > g0) reduce_stage(g - 1);
+    const int64_t u0 = stage_u0(g);
+    if (g < kVecStages) {
+#pragma unroll
+      for (int k = 0; k < kVecSteps; ++k) step(st, k, u0 + k, std::true_type{}, std::false_type{});
+    } else {
+#pragma unroll
+      for (int k = 0; k < kVecSteps; ++k) step(st, k, u0 + k, std::false_type{}, std::true_type{});
+    }
+    if (g % kVecStages == kVecStages - 1) flush();  // every 256 columns
+  }
+  if (g0 < g1) {
+    __syncthreads();
+    reduce_stage(g1 - 1);
+  }
+  flush();
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      // the row's columns are spread over the four lane groups: fold them
+      double tot = accd[r][v];
+      tot += __shfl_xor(tot, 16);
+      tot += __shfl_xor(tot, 32);
+      if (lane < 16)
+        fwd[(split * NV + v) * npad + 16 * (tile0 + r) + li] = (float)ldexp(tot, -kPScaleLog2);
+    }
+}
+
+// out[v m + j] = os (split sums + the transposed partials of the row blocks
+// that formed j's column block) + noise V: fp64, rounded once.  Four threads
+// per point each add a quarter of the splits and deltas in order (one thread's
+// chain of dependent-latency loads took 14.5 us at n = 20000, 40 deltas), the
+// quarters are added in order.
+constexpr int kVecRedPts = 64, kVecRedGroups = 4;
+__global__ __launch_bounds__(kVecRedPts* kVecRedGroups) void k_sym_vec_reduce(
+    const float* __restrict__ fwd, int splits, const float* __restrict__ tp, int nv, int64_t npad,
+    int64_t nb, int64_t hmax, int64_t m, float os, float noise, const float* __restrict__ V,
+    float* __restrict__ out) {
+  __shared__ double sm[kVecRedGroups][kVecRedPts];
+  const int t = threadIdx.x % kVecRedPts, grp = threadIdx.x / kVecRedPts;
+  const int64_t j = (int64_t)blockIdx.x * kVecRedPts + t;  // < npad, a multiple of 64
+  const int v = blockIdx.y;
+  double tot = 0.0;
+  const int s0 = splits * grp / kVecRedGroups, s1 = splits * (grp + 1) / kVecRedGroups;
+#pragma unroll 4
+  for (int s = s0; s < s1; ++s) tot += fwd[((int64_t)s * nv + v) * npad + j];
+  const int64_t J = j / kVecRows, jl = j - J * kVecRows;
+  const int64_t l0 = 1 + hmax * grp / kVecRedGroups, l1 = 1 + hmax * (grp + 1) / kVecRedGroups;
+  // unformed slots (nb even, the last delta) are read and dropped by a select,
+  // so eight loads stay in flight
+  auto slot = [&](int64_t dl, bool& formed) __attribute__((always_inline)) {
+    int64_t bb = J - dl;
+    bb += bb < 0 ? nb : 0;
+    formed = dl <= sym_span(bb, nb);
+    return tp[((bb * hmax + dl - 1) * nv + v) * kVecRows + jl];
+  };
+  int64_t dl = l0;
+  for (; dl + 8 <= l1; dl += 8) {
+    float x[8];
+    bool ok[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) x[q] = slot(dl + q, ok[q]);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) tot += ok[q] ? (double)x[q] : 0.0;
+  }
+  for (; dl < l1; ++dl) {
+    bool ok;
+    const float x = slot(dl, ok);
+    tot += ok ? (double)x : 0.0;
+  }
+  sm[grp][t] = tot;
+  __syncthreads();
+  if (grp > 0 || j >= m) return;
+#pragma unroll
+  for (int g = 1; g < kVecRedGroups; ++g) tot += sm[g][t];
+  out[(int64_t)v * m + j] =
+      (float)((double)os * tot + (double)noise * (double)V[(int64_t)v * npad + j]);
+}
+
+// ---------------------------------------------------------------------------
 // Gradient traces on the matrix cores (Gram-form kernels).
 //
 // The difference trace (grad_pair.hip) spends 4 d + ~10 VALU instructions per
@@ -2200,6 +2486,12 @@ bool sym_route(const MatvecArgs& a, const PackedPoints& rows, const PackedPoints
   const char* env = std::getenv("MGP_SYM_MATVEC");
   const int mode = env == nullptr ? -1 : (env[0] == '0' ? 0 : 1);
   if (mode == 0) return false;
+  if (nc <= kSymVecCols) {
+    const int64_t vb = ceil_div(std::max<int64_t>(a.n, 1), kVecRows);
+    if (vb * kVecRows > rows.ntiles_alloc * 16) return false;
+    if (mode < 0 && a.n < kSymVecMinPoints) return false;
+    return (double)vb * (double)(vb / 2) * kVecRows * nc * 4 <= kSymMaxBytes;
+  }
   const int64_t nb = ceil_div(std::max<int64_t>(a.n, 1), kSymRows);
   if (nb * kSymRows > rows.ntiles_alloc * 16) return false;
   if (mode < 0 && nb < kSymMinBlocks) return false;
@@ -2244,7 +2536,10 @@ SymFn pick_sym(int kb) {
 // sums (`split_bytes`) cost their extra read in the reduction (priced at 2 us
 // per stage, a short stage, so the choice leans towards fewer splits).
 // Cached per kernel, block count and device.
-int64_t delta_splits(int64_t nb, int stages, const void* fn, int threads, double split_bytes) {
+// granule: pieces into which a delta may be cut (1: whole deltas); the count
+// returned is for ranges of ceil((hmax + 1) granule / splits) pieces.
+int64_t delta_splits(int64_t nb, int stages, const void* fn, int threads, double split_bytes,
+                     int granule = 1) {
   static std::mutex mu;
   static std::unordered_map<std::string, int64_t> cache;
   int dev = 0;
@@ -2262,11 +2557,12 @@ int64_t delta_splits(int64_t nb, int stages, const void* fn, int threads, double
   constexpr double kStageUs = 2.0, kReduceBytesPerUs = 6.0e6;
   int64_t best_s = 1, last_dps = -1;
   double best = 0.0;
-  for (int64_t s0 = 1; s0 <= std::min<int64_t>(hmax + 1, 64); ++s0) {
-    const int64_t dps = ceil_div(hmax + 1, s0);
+  const int64_t pieces = (hmax + 1) * granule;
+  for (int64_t s0 = 1; s0 <= std::min<int64_t>(pieces, 64); ++s0) {
+    const int64_t dps = ceil_div(pieces, s0);
     if (dps == last_dps) continue;
     last_dps = dps;
-    const int64_t splits = ceil_div(hmax + 1, dps);
+    const int64_t splits = ceil_div(pieces, dps);
     const int64_t items = nb * splits;
     const int64_t per = round_up(items, (int64_t)kXcds) / kXcds;
     double make = 0.0;
@@ -2277,8 +2573,8 @@ int64_t delta_splits(int64_t nb, int stages, const void* fn, int threads, double
         const int64_t L = x * per + k;
         if (L >= items) break;
         const int64_t b = L % nb, d0 = (L / nb) * dps;
-        const int64_t d1 = std::min(d0 + dps, sym_span(b, nb) + 1);
-        const double cost = (double)std::max<int64_t>(d1 - d0, 0) * stages + 1.0;
+        const int64_t d1 = std::min(d0 + dps, (sym_span(b, nb) + 1) * granule);
+        const double cost = (double)std::max<int64_t>(d1 - d0, 0) * stages / granule + 1.0;
         const double t = cu.top();
         cu.pop();
         cu.push(t + cost);
@@ -2294,6 +2590,66 @@ int64_t delta_splits(int64_t nb, int stages, const void* fn, int threads, double
   }
   cache.emplace(key, best_s);
   return best_s;
+}
+
+using VecFn = void (*)(const h8*, const h8*, const float*, int64_t, int64_t, int64_t, int64_t,
+                       int64_t, float*, float*);
+
+template <int KIND, int NV>
+VecFn pick_vec(int kb) {
+  switch (kb) {
+    case 1: return k_sym_vec<KIND, 1, NV>;
+    case 2: return k_sym_vec<KIND, 2, NV>;
+    case 3: return k_sym_vec<KIND, 3, NV>;
+  }
+  return nullptr;
+}
+
+template <int KIND>
+VecFn pick_vec_cols(int kb, int nc) {
+  return nc == 1 ? pick_vec<KIND, 1>(kb) : pick_vec<KIND, 2>(kb);
+}
+
+// out = (K + noise I) V for one or two columns of V (k_sym_vec).
+void sym_vec_matvec(const MatvecArgs& a, const PackedPoints& pts, const float* Vc, int nc,
+                    float* outc, MatvecWorkspace& ws, hipStream_t st) {
+  const int64_t n = a.n, nb = ceil_div(std::max<int64_t>(n, 1), kVecRows), hmax = nb / 2;
+  const int64_t npad = nb * kVecRows;
+  VecFn fn = a.kind == KIND_RBF        ? pick_vec_cols<KIND_RBF>(pts.kb, nc)
+             : a.kind == KIND_MATERN32 ? pick_vec_cols<KIND_MATERN32>(pts.kb, nc)
+                                       : pick_vec_cols<KIND_MATERN52>(pts.kb, nc);
+  MGP_REQUIRE(fn != nullptr, "no symmetric kernel for this shape");
+  // the same split count for one and two columns: a column's result does not
+  // depend on its neighbour
+  VecFn one = a.kind == KIND_RBF        ? pick_vec_cols<KIND_RBF>(pts.kb, 1)
+              : a.kind == KIND_MATERN32 ? pick_vec_cols<KIND_MATERN32>(pts.kb, 1)
+                                        : pick_vec_cols<KIND_MATERN52>(pts.kb, 1);
+  int64_t splits = delta_splits(nb, kVecStages, reinterpret_cast<const void*>(one),
+                                64 * kVecWaves, (double)npad * 4, kVecStages);
+  const int64_t sps = ceil_div((hmax + 1) * kVecStages, splits);
+  splits = ceil_div((hmax + 1) * kVecStages, sps);
+  float* vp = ws.vpack.ensure((size_t)nc * npad);
+  float* fwd = ws.partial.ensure((size_t)splits * nc * npad);
+  float* tp = ws.sym_tp.ensure((size_t)std::max<int64_t>(nb * hmax, 1) * nc * kVecRows);
+  hipLaunchKernelGGL(k_pad_vec, dim3((unsigned)ceil_div(npad, 256), (unsigned)nc), dim3(256), 0,
+                     st, Vc, n, npad, vp);
+  if (ws.time_tile) MGP_HIP_CHECK(hipEventRecord(ws.ev0, st));
+  hipLaunchKernelGGL(fn, dim3((unsigned)round_up(nb * splits, kXcds)), dim3(64 * kVecWaves), 0, st,
+                     reinterpret_cast<const h8*>(pts.B.ptr), reinterpret_cast<const h8*>(pts.A.ptr),
+                     vp, npad, nb, splits, sps, hmax, fwd, tp);
+  MGP_HIP_CHECK(hipGetLastError());
+  if (ws.time_tile) {
+    MGP_HIP_CHECK(hipEventRecord(ws.ev1, st));
+    MGP_HIP_CHECK(hipEventSynchronize(ws.ev1));
+    float ms = 0.f;
+    MGP_HIP_CHECK(hipEventElapsedTime(&ms, ws.ev0, ws.ev1));
+    ws.tile_ms += ms;
+    ws.tile_calls += 1;
+  }
+  hipLaunchKernelGGL(k_sym_vec_reduce, dim3((unsigned)ceil_div(n, kVecRedPts), (unsigned)nc),
+                     dim3(kVecRedPts * kVecRedGroups), 0, st, fwd, (int)splits, tp, nc, npad, nb, hmax, n, a.outputscale, a.noise, vp,
+                     outc);
+  MGP_HIP_CHECK(hipGetLastError());
 }
 
 // out = (K + noise I) V for nc <= 16 columns of V on the symmetric kernel.
@@ -2489,7 +2845,10 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
     float* outc = out_dev + (int64_t)c0 * a.m;
     const float* Vin = a.square ? V_dev + (int64_t)c0 * a.m : nullptr;
     if (force_splits <= 0 && sym_route(a, rows, cols, nc, ws)) {
-      sym_matvec(a, rows, Vc, nc, outc, ws, st);
+      if (nc <= kSymVecCols)
+        sym_vec_matvec(a, rows, Vc, nc, outc, ws, st);
+      else
+        sym_matvec(a, rows, Vc, nc, outc, ws, st);
       continue;
     }
 
