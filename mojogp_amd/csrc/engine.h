@@ -166,6 +166,7 @@ TrainResult train(Provider& pv, const float* y_host, const std::vector<float>& i
 struct PredictState {
   DevBuf<float> alpha;  // [n]
   DevBuf<float> root;   // [rank][n]
+  RhsPack root_pack;    // its packing, where many predictions follow (prediction caches)
   int rank = 0;
   bool has_alpha = false;
 };

@@ -1469,15 +1469,13 @@ void predict_from_state(Provider& pv, const PredictState& ps, const float* Xs_ho
   if (variance_method == 1) {
     MGP_REQUIRE(ps.rank > 0, "LOVE variance needs an inverse root");
     auto t1 = Clock::now();
-    DevBuf<float> Vs, var;
-    Vs.ensure((size_t)ps.rank * m);
-    var.ensure(m);
-    pv.cross(pv.test, ps.root.ptr, ps.rank, Vs.ptr);
-    DevBuf<float> dv;
-    if (pv.nonstationary()) pv.diag_values(pv.test, m, dv.ensure((size_t)m));
-    love_variance(Vs.ptr, m, ps.rank, pv.kdiag(), var.ptr, st,
-                  pv.nonstationary() ? dv.ptr : nullptr);
-    MGP_HIP_CHECK(hipMemcpyAsync(var_out, var.ptr, m * sizeof(float), hipMemcpyDeviceToHost, st));
+    float* Vs = pv.love_v.ensure((size_t)ps.rank * m);
+    float* var = pv.love_var.ensure((size_t)m);
+    pv.cross(pv.test, ps.root.ptr, ps.rank, Vs, ps.root_pack.ncols > 0 ? &ps.root_pack : nullptr);
+    float* dv = nullptr;
+    if (pv.nonstationary()) pv.diag_values(pv.test, m, dv = pv.love_diag.ensure((size_t)m));
+    love_variance(Vs, m, ps.rank, pv.kdiag(), var, st, dv);
+    MGP_HIP_CHECK(hipMemcpyAsync(var_out, var, m * sizeof(float), hipMemcpyDeviceToHost, st));
     MGP_HIP_CHECK(hipStreamSynchronize(st));
     t.variance_s = secs_since(t1);
   } else if (variance_method == 2) {

@@ -109,6 +109,20 @@ struct PackedRhs {
   const uint32_t* colmax = nullptr;
 };
 
+// All columns of a right-hand side block packed once for many products over the
+// same column points (the LOVE root of a prediction cache), in the 64-column
+// chunks of fused_matvec.
+struct RhsPack {
+  int ncols = 0;
+  int64_t col_tiles = -1;      // column tiles of the points it was packed for
+  DevBuf<float> data;          // fp16 parts of every chunk
+  std::vector<size_t> offset;  // first float of each chunk
+  DevBuf<uint32_t> colmax;     // [chunks][64]
+  DevBuf<uint32_t> parts;      // scratch of the packing
+};
+void pack_rhs(const PackedPoints& cols, const float* V, int ncols, RhsPack& out,
+              hipStream_t st);
+
 struct MatvecArgs {
   int kind = KIND_RBF;
   float outputscale = 1.f;
@@ -131,6 +145,9 @@ struct MatvecArgs {
   // product's workspace and stay valid until that workspace's next product on
   // the same stream.
   PackedRhs* reuse = nullptr;
+  // Optional packing of all ncols columns, made by pack_rhs for these column
+  // points (no task mixing); V is still read by a chunk of one column.
+  const RhsPack* packed = nullptr;
 };
 
 // out[c*m + i] = os * sum_j k(r_i, c_j) V[c*n + j]  (+ noise*V[c*m+i] if square)

@@ -201,10 +201,30 @@ __global__ void k_col_absmax_final(const uint32_t* __restrict__ part, int chunks
 
 // Vp[((g*upairs + u)*2 + part)*64 + lane] (8 fp16): element e holds
 // V'[c = 16g + lane%16][j = 16 (2u + e/4) + 4 (lane/16) + e%4], part 0 = hi,
-// part 1 = lo.  One thread per (g, u, lane).
-__global__ void k_pack_rhs16(const float* __restrict__ V, int64_t n, int ncols,
-                             int ncg, int64_t upairs, const uint32_t* __restrict__ colmax,
-                             int vec4, h8* __restrict__ P) {
+// part 1 = lo.  One thread per (g, u, lane).  Every workgroup takes the column
+// maxima from their row-chunk parts itself (a launch of its own for them costs
+// 2 to 4 us); the first one stores them for the kernels that undo the scaling.
+__global__ __launch_bounds__(256) void k_pack_rhs16(const float* __restrict__ V, int64_t n,
+                                                    int ncols, int ncg, int64_t upairs,
+                                                    const uint32_t* __restrict__ part, int chunks,
+                                                    uint32_t* __restrict__ colmax, int vec4,
+                                                    h8* __restrict__ P) {
+  __shared__ uint32_t pm[256], cmax[64];
+  {
+    const int cols = 16 * ncg, per = 256 / cols;  // threads per column
+    const int c = threadIdx.x % cols, b0 = threadIdx.x / cols;
+    uint32_t mx = 0;
+    if (c < ncols)
+      for (int b = b0; b < chunks; b += per) mx = max(mx, part[(int64_t)c * chunks + b]);
+    pm[threadIdx.x] = mx;
+    __syncthreads();
+    if (threadIdx.x < cols) {
+      for (int q = 1; q < per; ++q) mx = max(mx, pm[threadIdx.x + q * cols]);
+      cmax[threadIdx.x] = mx;
+      if (blockIdx.x == 0 && threadIdx.x < ncols) colmax[threadIdx.x] = mx;
+    }
+    __syncthreads();
+  }
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (int64_t)ncg * upairs * 64) return;
   const int lane = (int)(idx & 63);
@@ -212,7 +232,7 @@ __global__ void k_pack_rhs16(const float* __restrict__ V, int64_t n, int ncols,
   const int g = (int)((idx >> 6) / upairs);
   const int c = 16 * g + (lane & 15);
   h8 hi, lo;
-  const int shift = c < ncols ? col_shift(colmax[c]) : 0;
+  const int shift = c < ncols ? col_shift(cmax[c]) : 0;
   // rows j0 .. j0 + 3 (e < 4) and j0 + 16 .. j0 + 19 (e >= 4)
   const int64_t j0 = 32 * u + 4 * (lane >> 4);
   float x[8];
@@ -2461,6 +2481,29 @@ struct ChunkBuffers {
   }
 };
 
+// Row chunks of the column maxima: 1024 rows, up to 64 chunks.
+int absmax_chunks(int64_t n) {
+  return (int)std::min<int64_t>(ceil_div(std::max<int64_t>(n, 1), 1024), 64);
+}
+
+// Packs nc <= 16 ncg right-hand sides V ([nc][n]) for col_pairs column-tile
+// pairs: their maxima into colmax (parts: [64][absmax_chunks(n)] scratch).
+void launch_pack_rhs(const float* V, int64_t n, int nc, int ncg, int64_t col_pairs,
+                     uint32_t* parts, uint32_t* colmax, h8* packed, hipStream_t st) {
+  const int chunks = absmax_chunks(n);
+  const int vec4 = (n % 4 == 0 && reinterpret_cast<uintptr_t>(V) % 16 == 0) ? 1 : 0;
+  hipLaunchKernelGGL(k_col_absmax_part, dim3((unsigned)chunks, (unsigned)nc), dim3(256), 0, st, V,
+                     n, vec4, parts);
+  const int64_t total = (int64_t)ncg * col_pairs * 64;  // 8-half vectors per part
+  hipLaunchKernelGGL(k_pack_rhs16, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, V, n,
+                     nc, ncg, col_pairs, parts, chunks, colmax, vec4, packed);
+  MGP_HIP_CHECK(hipGetLastError());
+}
+
+// Column groups of 16 a tile launch carries for nc <= 64 right-hand sides (0:
+// one column on the VALU).
+int rhs_groups(int nc) { return nc == 1 ? 0 : (nc <= 16 ? 1 : (nc <= 32 ? 2 : 4)); }
+
 size_t rhs_pack_bytes(int64_t col_tiles, int ncg) {
   if (ncg == 0) return (size_t)round_up(col_tiles * 16 * 4, 256);
   return (size_t)round_up((int64_t)ncg * (col_tiles / 2) * 64 * 32, 256);
@@ -2468,9 +2511,33 @@ size_t rhs_pack_bytes(int64_t col_tiles, int ncg) {
 
 }  // namespace
 
+void pack_rhs(const PackedPoints& cols, const float* V, int ncols, RhsPack& out, hipStream_t st) {
+  MGP_REQUIRE(cols.kb >= 1 && ncols >= 1, "right-hand sides are packed for the tile path");
+  const int64_t col_pairs = cols.ntiles / 2;
+  out.ncols = 0;  // valid once everything is launched
+  out.offset.clear();
+  size_t total = 0;
+  for (int c0 = 0; c0 < ncols; c0 += 64) {
+    out.offset.push_back(total);
+    total += (size_t)rhs_groups(std::min(64, ncols - c0)) * col_pairs * 64 * 2 * 4;
+  }
+  out.data.ensure(total);
+  out.colmax.ensure(64 * out.offset.size());
+  out.parts.ensure((size_t)64 * absmax_chunks(cols.n));
+  for (int c0 = 0; c0 < ncols; c0 += 64) {
+    const int nc = std::min(64, ncols - c0), ncg = rhs_groups(nc);
+    if (ncg == 0) continue;  // one column left over: packed by each product
+    launch_pack_rhs(V + (int64_t)c0 * cols.n, cols.n, nc, ncg, col_pairs, out.parts.ptr,
+                    out.colmax.ptr + c0, reinterpret_cast<h8*>(out.data.ptr + out.offset[c0 / 64]),
+                    st);
+  }
+  out.col_tiles = cols.ntiles;
+  out.ncols = ncols;
+}
+
 size_t fused_matvec_min_arena(const PackedPoints& cols, int ncols) {
   const int nc = std::min(ncols, 64);
-  const int ncg = nc == 1 ? 0 : (nc <= 16 ? 1 : (nc <= 32 ? 2 : 4));
+  const int ncg = rhs_groups(nc);
   size_t b = rhs_pack_bytes(cols.ntiles, ncg);
   if (ncg > 0) b += 256 + (size_t)round_up(64 * 64 * 4, 256);
   return b;
@@ -2662,18 +2729,9 @@ void sym_matvec(const MatvecArgs& a, const PackedPoints& pts, const float* Vc, i
   const int64_t mpad = nb * kSymRows;
 
   uint32_t* colmax = ws.colmax.ensure(64);
-  const int chunks = (int)std::min<int64_t>(ceil_div(std::max<int64_t>(n, 1), 4096), 64);
-  uint32_t* cpart = ws.colmax_part.ensure((size_t)64 * chunks);
-  const int vec4 = (n % 4 == 0 && reinterpret_cast<uintptr_t>(Vc) % 16 == 0) ? 1 : 0;
-  hipLaunchKernelGGL(k_col_absmax_part, dim3((unsigned)chunks, (unsigned)nc), dim3(256), 0, st,
-                     Vc, n, vec4, cpart);
-  hipLaunchKernelGGL(k_col_absmax_final, dim3((unsigned)nc), dim3(64), 0, st, cpart, chunks,
-                     colmax);
-  const int64_t total = pairs * 64;  // 8-half vectors per part, one column group
-  float* vp = ws.vpack.ensure((size_t)total * 2 * 4);
-  hipLaunchKernelGGL(k_pack_rhs16, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, Vc,
-                     n, nc, 1, pairs, colmax, vec4, reinterpret_cast<h8*>(vp));
-  MGP_HIP_CHECK(hipGetLastError());
+  uint32_t* cpart = ws.colmax_part.ensure((size_t)64 * absmax_chunks(n));
+  float* vp = ws.vpack.ensure((size_t)pairs * 64 * 2 * 4);
+  launch_pack_rhs(Vc, n, nc, 1, pairs, cpart, colmax, reinterpret_cast<h8*>(vp), st);
 
   SymFn fn = a.kind == KIND_RBF        ? pick_sym<KIND_RBF>(pts.kb)
              : a.kind == KIND_MATERN32 ? pick_sym<KIND_MATERN32>(pts.kb)
@@ -2839,7 +2897,7 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
   const int chunk = mixing ? (64 / a.mix_T) * a.mix_T : 64;
   for (int c0 = 0; c0 < a.ncols; c0 += chunk) {
     const int nc = std::min(chunk, a.ncols - c0);
-    const int ncg = nc == 1 ? 0 : (nc <= 16 ? 1 : (nc <= 32 ? 2 : 4));
+    const int ncg = rhs_groups(nc);
     const int cpad = ncg == 0 ? 1 : 16 * ncg;
     const float* Vc = V_dev + (int64_t)c0 * a.n;
     float* outc = out_dev + (int64_t)c0 * a.m;
@@ -2860,7 +2918,12 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
     const uint32_t* colmax = nullptr;
     PackedRhs* share = (a.reuse != nullptr && a.ncols <= chunk && ncg > 0 && ws.arena == nullptr)
                            ? a.reuse : nullptr;
-    if (share != nullptr && share->vp != nullptr && share->src == Vc &&
+    if (a.packed != nullptr && ncg > 0 && a.packed->ncols == a.ncols &&
+        a.packed->col_tiles == col_tiles) {
+      const size_t q = (size_t)(c0 / chunk);
+      vp = a.packed->data.ptr + a.packed->offset[q];
+      colmax = a.packed->colmax.ptr + 64 * q;
+    } else if (share != nullptr && share->vp != nullptr && share->src == Vc &&
         share->col_tiles == col_tiles && share->ncols == nc) {
       vp = share->vp;
       colmax = share->colmax;
@@ -2872,18 +2935,9 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
       vp = padded;
     } else {
       uint32_t* cm = buf.take(ws.colmax, 64);
-      const int chunks = (int)std::min<int64_t>(ceil_div(std::max<int64_t>(a.n, 1), 4096), 64);
-      uint32_t* cpart = buf.take(ws.colmax_part, (size_t)64 * chunks);
-      const int vec4 = (a.n % 4 == 0 && reinterpret_cast<uintptr_t>(Vc) % 16 == 0) ? 1 : 0;
-      hipLaunchKernelGGL(k_col_absmax_part, dim3((unsigned)chunks, (unsigned)nc), dim3(256), 0,
-                         st, Vc, a.n, vec4, cpart);
-      hipLaunchKernelGGL(k_col_absmax_final, dim3((unsigned)nc), dim3(64), 0, st, cpart, chunks,
-                         cm);
-      const int64_t total = (int64_t)ncg * col_pairs * 64;  // 8-half vectors per part
-      float* packed = buf.take(ws.vpack, (size_t)total * 2 * 4);
-      hipLaunchKernelGGL(k_pack_rhs16, dim3((unsigned)ceil_div(total, 256)), dim3(256),
-                         0, st, Vc, a.n, nc, ncg, col_pairs, cm, vec4,
-                         reinterpret_cast<h8*>(packed));
+      uint32_t* cpart = buf.take(ws.colmax_part, (size_t)64 * absmax_chunks(a.n));
+      float* packed = buf.take(ws.vpack, (size_t)ncg * col_pairs * 64 * 2 * 4);
+      launch_pack_rhs(Vc, a.n, nc, ncg, col_pairs, cpart, cm, reinterpret_cast<h8*>(packed), st);
       vp = packed;
       colmax = cm;
       if (share != nullptr) {
@@ -2987,17 +3041,9 @@ void SmallCg::begin(const float* p) {
                        npad, ws->vpack.ptr);
   } else {
     colmax = ws->colmax.ensure(64);
-    const int chunks = (int)std::min<int64_t>(ceil_div(a.n, 4096), 64);
-    uint32_t* cpart = ws->colmax_part.ensure((size_t)64 * chunks);
-    const int vec4 = (a.n % 4 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0) ? 1 : 0;
-    hipLaunchKernelGGL(k_col_absmax_part, dim3((unsigned)chunks, (unsigned)nc), dim3(256), 0, st,
-                       p, a.n, vec4, cpart);
-    hipLaunchKernelGGL(k_col_absmax_final, dim3((unsigned)nc), dim3(64), 0, st, cpart, chunks,
-                       colmax);
-    const int64_t total = col_pairs * 64;
-    vp = ws->vpack.ensure((size_t)total * 2 * 4);
-    hipLaunchKernelGGL(k_pack_rhs16, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, p,
-                       a.n, nc, 1, col_pairs, colmax, vec4, reinterpret_cast<h8*>(vp));
+    uint32_t* cpart = ws->colmax_part.ensure((size_t)64 * absmax_chunks(a.n));
+    vp = ws->vpack.ensure((size_t)col_pairs * 64 * 2 * 4);
+    launch_pack_rhs(p, a.n, nc, 1, col_pairs, cpart, colmax, reinterpret_cast<h8*>(vp), st);
   }
   MGP_HIP_CHECK(hipGetLastError());
 }

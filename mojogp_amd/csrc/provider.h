@@ -131,8 +131,11 @@ struct Provider {
   DevBuf<float> gscale;  // per-parameter scale of the gradient sums
   void gradient(const float* V, int ncols, float* out);
 
-  // K(Xs, X) V for a packed test set.
-  void cross(const PackedPoints& rows, const float* V, int ncols, float* out);
+  // K(Xs, X) V for a packed test set; packed: V's packing for the tile route
+  // (pack_rhs over train), if the caller keeps one.
+  void cross(const PackedPoints& rows, const float* V, int ncols, float* out,
+             const RhsPack* packed = nullptr);
+  DevBuf<float> love_v, love_var, love_diag;  // LOVE variance of a test set
   // out[c*n + i] = k(rows[r0 + c], x_i) for c < nrows (dense cross block).
   void fill_block(const PackedPoints& rows, int64_t r0, int64_t nrows, float* out);
 };

@@ -260,7 +260,7 @@ void Provider::forward_mixed(const float* V, int ncols, const float* mix, int T,
 }
 
 void Provider::cross(const PackedPoints& rows, const float* V, int ncols,
-                     float* out) {
+                     float* out, const RhsPack* packed) {
   if (is_tree) {
     tree_matvec(tree, tparams.ptr, rows.z.ptr, rows.n, train.z.ptr, n, V, ncols, 0.f, false,
                 out, tree_ws, st);
@@ -278,6 +278,7 @@ void Provider::cross(const PackedPoints& rows, const float* V, int ncols,
     direct_matvec(a, rows, train, d, V, out, ws, st);
     return;
   }
+  a.packed = packed;
   fused_matvec(a, rows, train, V, out, ws, st);
 }
 
