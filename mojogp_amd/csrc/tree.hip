@@ -2,6 +2,7 @@
 // gradient traces evaluated per pair from raw coordinate differences (VALU;
 // the Gram-form tile path serves single radial leaves).  Tree semantics and
 // reference citations are in kernel_tree.h.
+#include "sym_common.h"
 #include "tree.h"
 #include "tree_jit.h"
 
@@ -17,6 +18,7 @@ namespace {
 constexpr int kTile = 128;      // column points per LDS tile
 constexpr int kMaxCols = 16;    // right-hand sides per pass
 constexpr int kGradCols = 16;   // gradient-trace factor columns per pass
+typedef float f4t __attribute__((ext_vector_type(4)));
 static_assert(kTreeChunk % 4 == 0 && kTile % kTreeChunk == 0, "float4 chunk reads");
 
 void require(bool ok, const std::string& msg) {
@@ -34,6 +36,56 @@ __global__ void k_tree_reduce(const float* __restrict__ part, int splits, int64_
   float o = (float)s;
   if (add_noise) o = fmaf(noise, V[idx], o);
   out[idx] = o;
+}
+
+// out[c][j] = sum_y fwd[y][c][j] + the transposed partials of the row blocks
+// that formed j's column block (delta order) + noise V: fp64, rounded once.
+// Four threads per point own four right-hand sides each; unformed slots (nb
+// even, the last delta) are read and dropped by a select.
+__global__ __launch_bounds__(256) void k_tree_sym_reduce(
+    const float* __restrict__ fwd, int splits, const float* __restrict__ tp, int block,
+    int64_t nb, int64_t hmax, int64_t n, int nc, float noise, const float* __restrict__ V,
+    float* __restrict__ out) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t j = t >> 2;
+  const int c4 = 4 * (int)(t & 3);
+  if (j >= n) return;
+  const int64_t npad = nb * block;
+  double tot[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int y = 0; y < splits; ++y)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tot[e] += fwd[((int64_t)y * 16 + c4 + e) * npad + j];
+  const int64_t J = j / block, jl = j - J * block;
+  auto slot = [&](int64_t dl, bool& formed) __attribute__((always_inline)) {
+    int64_t bb = J - dl;
+    bb += bb < 0 ? nb : 0;
+    formed = dl <= sym_span(bb, nb);
+    return __builtin_nontemporal_load(reinterpret_cast<const f4t*>(
+        tp + ((bb * hmax + dl - 1) * block + jl) * 16 + c4));
+  };
+  int64_t dl = 1;
+  for (; dl + 8 <= hmax + 1; dl += 8) {
+    f4t v[8];
+    bool ok[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = slot(dl + q, ok[q]);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tot[e] += ok[q] ? (double)v[q][e] : 0.0;
+  }
+  for (; dl <= hmax; ++dl) {
+    bool ok;
+    const f4t v = slot(dl, ok);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tot[e] += ok ? (double)v[e] : 0.0;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (c4 + e < nc) {
+      const int64_t idx = (int64_t)(c4 + e) * n + j;
+      out[idx] = (float)(tot[e] + (double)noise * (double)V[idx]);
+    }
 }
 
 // out[i] = K(x_i, x_i)
@@ -304,6 +356,60 @@ double tree_diag(const KernelTree& t, const float* params) {
   return v[(size_t)t.nnodes - 1];
 }
 
+namespace {
+// Square products with 5 to 16 right-hand sides from this many points on run
+// on the symmetric kernel (RBF x periodic + RQ, d = 6, 16 columns, us
+// one-sided / symmetric: 61 / 66 at n = 4096, 85 / 73 at 5000, 226 / 172 at
+// 10000, 738 / 522 at 20000; below, too few block pairs fill the chip); a model
+// of this size repays its compilation, as for the gradient kernel.
+constexpr int64_t kTreeSymMin = 5000;
+constexpr int kTreeSymMinCols = 5;
+constexpr double kTreeSymMaxBytes = 8e9;
+
+// out = (K + noise I) V for nc <= 16 columns on the symmetric kernel.
+void tree_sym_matvec(const KernelTree& t, const float* p_dev, const float* X, int64_t n,
+                     const float* V, int nc, float noise, float* out, DevBuf<float>& work,
+                     hipStream_t st) {
+  const TreeSymJitKernel jk = tree_sym_jit_kernel(t);
+  int dev = 0, cus = 0;
+  MGP_HIP_CHECK(hipGetDevice(&dev));
+  MGP_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const int64_t nb = ceil_div(n, (int64_t)jk.block), hmax = nb / 2;
+  const int64_t stages = (hmax + 1) * (jk.block / jk.stage);
+  const int64_t slots = (int64_t)std::max(cus, 1) * jk.per_cu;
+  // rounds of (stages a workgroup + about a third of one of set-up); a split's
+  // forward partials cost little beside a stage
+  int64_t best = 1;
+  double best_cost = 0.0;
+  for (int64_t s = 1; s <= std::min<int64_t>(stages, 64); ++s) {
+    const int64_t sps = ceil_div(stages, s);
+    if (ceil_div(stages, sps) != s) continue;
+    const double cost = (double)ceil_div(nb * s, slots) * ((double)sps + 0.35) + 0.02 * (double)s;
+    if (s == 1 || cost < best_cost) {
+      best_cost = cost;
+      best = s;
+    }
+  }
+  long long nn = n, nbb = nb, sp = best, sps = ceil_div(stages, best), hm = hmax;
+  const size_t nf = (size_t)best * 16 * nb * jk.block;
+  float* fwd = work.ensure(nf + (size_t)std::max<int64_t>(nb * hmax, 1) * jk.block * 16);
+  float* tp = fwd + nf;
+  int ncc = nc;
+  void* args[] = {(void*)&X, &nn, (void*)&p_dev, (void*)&V, &ncc, &nbb, &sp, &sps, &hm,
+                  (void*)&fwd, (void*)&tp};
+  MGP_HIP_CHECK(hipModuleLaunchKernel(jk.fn, (unsigned)nb, (unsigned)best, 1, 256, 1, 1, 0, st,
+                                      args, nullptr));
+  hipLaunchKernelGGL(k_tree_sym_reduce, dim3((unsigned)ceil_div(4 * n, 256)), dim3(256), 0, st, fwd,
+                     (int)best, tp, jk.block, nb, hmax, n, nc, noise, V, out);
+  MGP_HIP_CHECK(hipGetLastError());
+}
+
+bool tree_sym_route(const KernelTree& t, int64_t m, int64_t n, int nc, bool square) {
+  return square && m == n && t.table_size == 0 && n >= kTreeSymMin && nc >= kTreeSymMinCols &&
+         (double)n * (double)n * 16 * 4 / 512 <= kTreeSymMaxBytes;
+}
+}  // namespace
+
 void tree_matvec(const KernelTree& t, const float* p_dev, const float* Xr, int64_t m,
                  const float* Xc, int64_t n, const float* V, int ncols, float noise,
                  bool square, float* out, DevBuf<float>& work, hipStream_t st) {
@@ -316,6 +422,11 @@ void tree_matvec(const KernelTree& t, const float* p_dev, const float* Xr, int64
       1, std::min<int64_t>(ceil_div(2048, rows), tiles));
   for (int c0 = 0; c0 < ncols; c0 += kMaxCols) {
     const int nc = std::min(kMaxCols, ncols - c0);
+    if (Xr == Xc && tree_sym_route(t, m, n, nc, square)) {
+      tree_sym_matvec(t, p_dev, Xc, n, V + (int64_t)c0 * n, nc, noise, out + (int64_t)c0 * n, work,
+                      st);
+      continue;
+    }
     float* part = work.ensure((size_t)splits * nc * m);
     // the tree's straight-line kernel (tree_jit.hip)
     const TreeJitKernel jk = tree_jit_kernel(t, nc);

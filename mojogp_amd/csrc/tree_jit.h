@@ -23,6 +23,20 @@ TreeJitKernel tree_jit_kernel(const KernelTree& t, int nc);
 // The generated source (tests and inspection).
 std::string tree_jit_source(const KernelTree& t);
 
+struct TreeSymJitKernel {
+  hipFunction_t fn = nullptr;  // extern "C" k_tree_sym_jit
+  int per_cu = 1;              // workgroups a CU holds
+  int block = 0, stage = 0;    // points per block, columns per stage
+};
+
+// The symmetric product kernel of tree t (no correlation tables) for up to 16
+// right-hand sides: arguments (const float* X, long long n, const float* p,
+// const float* V, int nc, long long nb, long long splits, long long sps, long
+// long hmax, float* fwd, float* tp), grid (nb, splits), 256 threads; see
+// tree_sym_source for the layouts.  Compiled on first use per (tree, device).
+TreeSymJitKernel tree_sym_jit_kernel(const KernelTree& t);
+std::string tree_sym_jit_source(const KernelTree& t);
+
 struct TreeGradJitKernel {
   hipFunction_t fn = nullptr;  // extern "C" k_tree_grad_jit; null: not generated for this tree
   int block = 0;               // points per block

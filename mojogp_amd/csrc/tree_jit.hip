@@ -31,6 +31,8 @@ constexpr int kJitTile = 128;  // column points per LDS tile
 const int kJitCols[] = {1, 2, 4, 8, 16};
 constexpr int kJitMfmaMinCols = 8;   // column counts from here use the MFMA product
 constexpr int kJitMfmaRowTiles = 2;  // 16-row tiles per wave in the MFMA kernel
+constexpr int kTreeSymBlock = 256;   // points per block of the symmetric product kernel
+constexpr int kTreeSymStage = 64;    // columns per LDS stage of it
 constexpr int kTreeGradBlock = 128;  // points per block of the gradient kernel
 
 std::string f(float v) {
@@ -583,6 +585,148 @@ extern "C" __global__ __launch_bounds__(256) void k_tree_grad_jit(
   return s.str();
 }
 
+// Symmetric product kernel of the tree (square products, stationary in the
+// sense K_ij = K_ji): every off-diagonal value is formed once and used for both
+// of its entries.  A value costs ~15 VALU instructions per leaf and dimension
+// beside the 64 cycles a pair of fp32 matrix instructions spends on it, so
+// halving the values is worth the transposition.  Blocks of 256 points, row
+// block b taking stages [g0, g1) (64 columns each) of its own block and of the
+// column blocks (b + delta) mod nb of the cyclic half.  Per 16 x 16 tile a lane
+// evaluates the pairs (row lane%16, columns 4 (lane/16) + s), the A operands of
+// out_I += K V_J; their rows go through a wave-private LDS tile (stride 20:
+// conflict-free both ways) and come back as the A operands of out_J += K^T V_I
+// with the rows' right-hand sides in registers.  The waves' transposed sums
+// are added in LDS and written per stage: tp[((b hmax + delta - 1) 256 + j) 16
+// + c]; forward sums (fp64 across stages) fwd[(split 16 + c) npad + i].
+std::string tree_sym_source(const KernelTree& t) {
+  std::string pro, pair;
+  emit_tree(t, pro, pair);
+  pair += tree_value_return(t);
+  const int D = t.d, DP = (D + 3) / 4 * 4;
+  std::ostringstream s;
+  s << "#define D " << D << "\n#define DP " << DP << "\n#define BLK " << kTreeSymBlock
+    << "\n#define R " << kTreeSymBlock / 64 << "\n#define ST " << kTreeSymStage << "\n"
+    << R"(typedef float f4m __attribute__((ext_vector_type(4)));
+#define VS 20
+extern "C" __global__ __launch_bounds__(256) void k_tree_sym_jit(
+    const float* __restrict__ X, long long n, const float* __restrict__ p,
+    const float* __restrict__ V, int nc, long long nb, long long splits, long long sps,
+    long long hmax, float* __restrict__ fwd, float* __restrict__ tp) {
+  __shared__ __align__(16) float sx[ST * DP];
+  __shared__ __align__(16) float sv[ST * VS];
+  __shared__ __align__(16) float tsc[4][2][16 * VS];
+  __shared__ __align__(16) f4m tbuf[4][ST / 16][64];
+)" << pro
+    << R"(  auto kval = [&](const float* __restrict__ xi, const float* __restrict__ xj)
+      __attribute__((always_inline)) -> float {
+)" << pair
+    << R"(  };
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lm = lane & 15, lq = lane >> 4;
+  const long long b = blockIdx.x, split = blockIdx.y, npad = nb * BLK;
+  const long long i0 = b * BLK + wave * (16 * R);
+  float xi[R][DP], vr[R][4];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const long long i = i0 + 16 * r + lm;
+#pragma unroll
+    for (int k = 0; k < DP; ++k) xi[r][k] = (i < n && k < D) ? X[i * D + k] : 0.0f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const long long ii = i0 + 16 * r + 4 * lq + s;
+      vr[r][s] = (ii < n && lm < nc) ? V[(long long)lm * n + ii] : 0.0f;
+    }
+  }
+  double acc[R][4];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[r][q] = 0.0;
+  const int per = BLK / ST;
+  const long long span = (nb & 1) ? (nb - 1) / 2 : (b < nb / 2 ? nb / 2 : nb / 2 - 1);
+  const long long g0 = split * sps, gl = (span + 1) * per;
+  const long long g1 = g0 + sps < gl ? g0 + sps : gl;
+  for (long long g = g0; g < g1; ++g) {
+    const long long dl = g / per;
+    long long J = b + dl;
+    if (J >= nb) J -= nb;
+    const long long j0 = J * BLK + (g % per) * ST;
+    // (the previous stage's operands are free: its second barrier)
+    for (int q = threadIdx.x; q < ST * DP; q += 256) {
+      const int jj = q / DP, k = q - jj * DP;
+      sx[q] = (j0 + jj < n && k < D) ? X[(j0 + jj) * D + k] : 0.0f;
+    }
+    for (int q = threadIdx.x; q < ST * 16; q += 256) {
+      const int c = q / ST, jj = q - c * ST;
+      sv[jj * VS + c] = (c < nc && j0 + jj < n) ? V[(long long)c * n + j0 + jj] : 0.0f;
+    }
+    __syncthreads();
+    f4m d1[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) d1[r] = f4m{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int ct = 0; ct < ST / 16; ++ct) {
+      f4m d2 = f4m{0.0f, 0.0f, 0.0f, 0.0f};
+      float kv[R][4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int jj = 16 * ct + 4 * lq + s;
+        float xj[DP];
+#pragma unroll
+        for (int k = 0; k < DP; k += 4) {
+          const f4m x = *reinterpret_cast<const f4m*>(sx + jj * DP + k);
+          xj[k] = x[0]; xj[k + 1] = x[1]; xj[k + 2] = x[2]; xj[k + 3] = x[3];
+        }
+        const float v = sv[jj * VS + lm];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          kv[r][s] = kval(xi[r], xj);
+          d1[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[r][s], v, d1[r], 0, 0, 0);
+        }
+      }
+      if (dl > 0) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          float* sc = tsc[wave][r & 1];
+          *reinterpret_cast<f4m*>(sc + lm * VS + 4 * lq) =
+              f4m{kv[r][0], kv[r][1], kv[r][2], kv[r][3]};
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            d2 = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[(4 * lq + s) * VS + lm], vr[r][s], d2, 0,
+                                                      0, 0);
+        }
+        tbuf[wave][ct][lane] = d2;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[r][q] += (double)d1[r][q];
+    __syncthreads();
+    if (dl > 0) {
+      // lane of column tile ct: columns 4 (lane/16) + q, right-hand side lane%16
+      float* dst = tp + ((b * hmax + dl - 1) * BLK + (g % per) * ST) * 16;
+      for (int q = threadIdx.x; q < ST * 4; q += 256) {
+        const int ct = q >> 6, ln = q & 63;
+        const f4m a = tbuf[0][ct][ln], bb = tbuf[1][ct][ln], c = tbuf[2][ct][ln],
+                  e = tbuf[3][ct][ln];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          dst[(16 * ct + 4 * (ln >> 4) + k) * 16 + (ln & 15)] =
+              (float)((double)a[k] + (double)bb[k] + (double)c[k] + (double)e[k]);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      fwd[(split * 16 + lm) * npad + i0 + 16 * r + 4 * lq + q] = (float)acc[r][q];
+}
+)";
+  return s.str();
+}
+
 std::string spec_key(const KernelTree& t) {
   std::ostringstream o;
   o << t.d << ' ' << t.nparams << ' ' << t.nleaves << ' ' << t.nnodes << ' ' << t.table_size;
@@ -658,11 +802,37 @@ Compiled compile_tree(const KernelTree& t) {
 
 // Gradient kernels per (tree, device); fn null where the tree has none.
 std::map<std::pair<std::string, int>, hipFunction_t> g_jit_grad;
+// Symmetric product kernels and their workgroups per CU.
+std::map<std::pair<std::string, int>, std::pair<hipFunction_t, int>> g_jit_sym;
 
 }  // namespace
 
 std::string tree_jit_source(const KernelTree& t) { return tree_source(t); }
 std::string tree_grad_jit_source(const KernelTree& t) { return tree_grad_source(t); }
+std::string tree_sym_jit_source(const KernelTree& t) { return tree_sym_source(t); }
+
+TreeSymJitKernel tree_sym_jit_kernel(const KernelTree& t) {
+  MGP_REQUIRE(t.table_size == 0, "correlation tables need not be symmetric");
+  int dev = 0;
+  MGP_HIP_CHECK(hipGetDevice(&dev));
+  const auto key = std::make_pair(spec_key(t), dev);
+  std::lock_guard<std::mutex> lk(g_jit_mu);
+  auto it = g_jit_sym.find(key);
+  if (it == g_jit_sym.end()) {
+    hipFunction_t fn = nullptr;
+    MGP_HIP_CHECK(hipModuleGetFunction(
+        &fn, compile_source(tree_sym_source(t), "kernel_tree_sym_jit.hip"), "k_tree_sym_jit"));
+    int per_cu = 0;
+    MGP_HIP_CHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, 0));
+    it = g_jit_sym.emplace(key, std::make_pair(fn, std::max(per_cu, 1))).first;
+  }
+  TreeSymJitKernel out;
+  out.fn = it->second.first;
+  out.per_cu = it->second.second;
+  out.block = kTreeSymBlock;
+  out.stage = kTreeSymStage;
+  return out;
+}
 
 TreeGradJitKernel tree_grad_jit_kernel(const KernelTree& t) {
   int dev = 0;
