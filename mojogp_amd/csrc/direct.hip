@@ -12,12 +12,13 @@
 // accurate as one accumulated on the VALU) or, for up to 4 right-hand sides,
 // VALU FMAs.  Issue bound: at d = 5 the value costs ~62 cycles per 64 pairs
 // and the matrix instruction 32, ~250 us for n = 20011 one-sided; measured 313
-// to 330 us with the reduction (11 right-hand sides, Matern-1/2) against 18.7
-// ms for one row per thread with every product added in fp64 (79 workgroups,
-// run-time dimension loops).  Splitting the values for the 16-bit matrix cores
+// to 330 us with the reduction (11 right-hand sides, Matern-1/2) and 263 us
+// over unordered pairs, against 18.7 ms for one row per thread with every
+// product added in fp64 (79 workgroups, run-time dimension loops).  Splitting the values for the 16-bit matrix cores
 // would shorten the matrix part but costs accuracy that these products had.
 #include "kval.h"
 #include "matvec.h"
+#include "sym_common.h"
 
 #include <algorithm>
 #include <vector>
@@ -285,6 +286,289 @@ int64_t diff_splits(int64_t row_blocks, int64_t tiles, int64_t slots) {
   return best;
 }
 
+// ---------------------------------------------------------------------------
+// Square products with 5 to 16 right-hand sides: every unordered pair is formed
+// once.  Blocks of 64 R points (4 waves of R row tiles); row block b takes
+// stages (64 columns each) of its own block and of the column blocks (b +
+// delta) mod nb of the cyclic half (sym_span).  Per 16 x 16 tile a lane
+// evaluates the pairs (row lane%16, columns 4 (lane/16) + s), the A operands of
+// out_I += K V_J; their rows go through a wave-private LDS tile (stride 20:
+// conflict-free both ways) and come back as the A operands of out_J += K^T V_I
+// with the rows' right-hand sides in registers.  The waves' transposed sums
+// are added in LDS and written per stage.  The value's 2 d + 7 instructions
+// are paid once for two entries, the matrix instructions (32 cycles per 4
+// columns of a tile) per entry.  Matern-1/2, 16 right-hand sides, one-sided ->
+// here: d = 5 n = 20011 321 -> 266 us, n = 40000 1147 -> 837; d = 16 1816 ->
+// 1213 at n = 40000.
+// fwd[(split 16 + c) npad + i] (fp64 across stages, then float),
+// tp[((b hmax + delta - 1) BLK + j) 16 + c].
+// ---------------------------------------------------------------------------
+constexpr int kDiffSymStage = 64;
+constexpr int diff_sym_rows(int D) { return D > 10 ? 2 : 4; }
+
+template <int KIND, int D>
+__global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
+    const float* __restrict__ Z, int64_t n, int d, const float* __restrict__ V, int nc,
+    int64_t nb, int64_t sps, int64_t hmax, float lim, float* __restrict__ fwd,
+    float* __restrict__ tp) {
+  constexpr int R = diff_sym_rows(D), BLK = 64 * R, ST = kDiffSymStage, VS = 20;
+  constexpr int DS = D <= 2 ? D : (D + 3) / 4 * 4;
+  constexpr int per = BLK / ST;
+  __shared__ __align__(16) float sx[ST * DS];
+  __shared__ __align__(16) float sv[ST * VS];
+  __shared__ __align__(16) float tsc[kDiffWaves][2][16 * VS];
+  __shared__ f4 tbuf[kDiffWaves][ST / 16][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lm = lane & 15, lq = lane >> 4;
+  const int64_t b = blockIdx.x, split = blockIdx.y, npad = nb * BLK;
+  const int64_t i0 = b * BLK + wave * (16 * R);
+  float xi[R][D], vr[R][4];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int64_t i = i0 + 16 * r + lm;
+#pragma unroll
+    for (int k = 0; k < D; ++k) xi[r][k] = (i < n && k < d) ? Z[i * d + k] : 0.0f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int64_t ii = i0 + 16 * r + 4 * lq + s;
+      vr[r][s] = (ii < n && lm < nc) ? V[(int64_t)lm * n + ii] : 0.0f;
+    }
+  }
+  double acc[R][4];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[r][q] = 0.0;
+  const int64_t g0 = split * sps, g1 = min(g0 + sps, (sym_span(b, nb) + 1) * per);
+  for (int64_t g = g0; g < g1; ++g) {
+    const int64_t dl = g / per;
+    int64_t J = b + dl;
+    if (J >= nb) J -= nb;
+    const int64_t j0 = J * BLK + (g % per) * ST;
+    // (the previous stage's operands are free: its second barrier)
+    for (int q = threadIdx.x; q < ST * D; q += 64 * kDiffWaves) {
+      const int jj = q / D, k = q - jj * D;
+      sx[jj * DS + k] = (j0 + jj < n && k < d) ? Z[(j0 + jj) * d + k] : 0.0f;
+    }
+    for (int q = threadIdx.x; q < ST * 16; q += 64 * kDiffWaves) {
+      const int c = q / ST, jj = q - c * ST;
+      sv[jj * VS + c] = (c < nc && j0 + jj < n) ? V[(int64_t)c * n + j0 + jj] : 0.0f;
+    }
+    __syncthreads();
+    f4 d1[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) d1[r] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int ct = 0; ct < ST / 16; ++ct) {
+      f4 d2 = f4{0.f, 0.f, 0.f, 0.f};
+      float kv[R][4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int jj = 16 * ct + 4 * lq + s;
+        float xj[DS];
+        if constexpr (D <= 2) {
+#pragma unroll
+          for (int k = 0; k < D; ++k) xj[k] = sx[jj * DS + k];
+        } else {
+#pragma unroll
+          for (int k = 0; k < DS; k += 4) {
+            const f4 x = *reinterpret_cast<const f4*>(&sx[jj * DS + k]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xj[k + e] = x[e];
+          }
+        }
+        const float v = sv[jj * VS + lm];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          float r2 = 0.0f;
+#pragma unroll
+          for (int k = 0; k < D; ++k) {
+            const float df = xi[r][k] - xj[k];
+            r2 = fmaf(df, df, r2);
+          }
+          kv[r][s] = kval<KIND>(r2, lim);
+          d1[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[r][s], v, d1[r], 0, 0, 0);
+        }
+      }
+      if (dl > 0) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          float* sc = tsc[wave][r & 1];
+          *reinterpret_cast<f4*>(sc + lm * VS + 4 * lq) =
+              f4{kv[r][0], kv[r][1], kv[r][2], kv[r][3]};
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            d2 = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[(4 * lq + s) * VS + lm], vr[r][s], d2, 0,
+                                                      0, 0);
+        }
+        tbuf[wave][ct][lane] = d2;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[r][q] += (double)d1[r][q];
+    __syncthreads();
+    if (dl > 0) {
+      // lane of column tile ct: columns 4 (lane/16) + q, right-hand side lane%16
+      float* dst = tp + ((b * hmax + dl - 1) * BLK + (g % per) * ST) * 16;
+      for (int q = threadIdx.x; q < ST * 4; q += 64 * kDiffWaves) {
+        const int ct = q >> 6, ln = q & 63;
+        double t[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int w = 0; w < kDiffWaves; ++w)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) t[k] += (double)tbuf[w][ct][ln][k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          dst[(16 * ct + 4 * (ln >> 4) + k) * 16 + (ln & 15)] = (float)t[k];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      fwd[(split * 16 + lm) * npad + i0 + 16 * r + 4 * lq + q] = (float)acc[r][q];
+}
+
+// out[c][j] = os (split sums + the transposed partials of the row blocks that
+// formed j's column block, in delta order) + noise V: fp64, rounded once.
+// Four threads per point own four right-hand sides each; unformed slots (nb
+// even, the last delta) are read and dropped by a select.
+__global__ __launch_bounds__(256) void k_diff_sym_reduce(
+    const float* __restrict__ fwd, int splits, const float* __restrict__ tp, int block,
+    int64_t nb, int64_t hmax, int64_t n, int nc, float os, float noise,
+    const float* __restrict__ V, float* __restrict__ out) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t j = t >> 2;
+  const int c4 = 4 * (int)(t & 3);
+  if (j >= n) return;
+  const int64_t npad = nb * block;
+  double tot[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int y = 0; y < splits; ++y)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tot[e] += fwd[((int64_t)y * 16 + c4 + e) * npad + j];
+  const int64_t J = j / block, jl = j - J * block;
+  auto slot = [&](int64_t dl, bool& formed) __attribute__((always_inline)) {
+    int64_t bb = J - dl;
+    bb += bb < 0 ? nb : 0;
+    formed = dl <= sym_span(bb, nb);
+    return __builtin_nontemporal_load(reinterpret_cast<const f4*>(
+        tp + ((bb * hmax + dl - 1) * block + jl) * 16 + c4));
+  };
+  int64_t dl = 1;
+  for (; dl + 8 <= hmax + 1; dl += 8) {
+    f4 v[8];
+    bool ok[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = slot(dl + q, ok[q]);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tot[e] += ok[q] ? (double)v[q][e] : 0.0;
+  }
+  for (; dl <= hmax; ++dl) {
+    bool ok;
+    const f4 v = slot(dl, ok);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tot[e] += ok ? (double)v[e] : 0.0;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (c4 + e < nc) {
+      const int64_t idx = (int64_t)(c4 + e) * n + j;
+      out[idx] = diff_epilogue(tot[e], os, noise, V[idx]);
+    }
+}
+
+using DiffSymFn = void (*)(const float*, int64_t, int, const float*, int, int64_t, int64_t,
+                           int64_t, float, float*, float*);
+struct DiffSymKernel {
+  DiffSymFn fn;
+  int block;
+};
+
+template <int KIND>
+DiffSymKernel pick_diff_sym_d(int d) {
+#define MGP_DIFF_CASE(DV) \
+  if (d <= DV) return {k_diff_sym<KIND, DV>, 64 * diff_sym_rows(DV)};
+  MGP_DIFF_CASE(1)
+  MGP_DIFF_CASE(2)
+  MGP_DIFF_CASE(3)
+  MGP_DIFF_CASE(4)
+  MGP_DIFF_CASE(5)
+  MGP_DIFF_CASE(6)
+  MGP_DIFF_CASE(8)
+  MGP_DIFF_CASE(10)
+  MGP_DIFF_CASE(12)
+  MGP_DIFF_CASE(16)
+  MGP_DIFF_CASE(20)
+  MGP_DIFF_CASE(24)
+  MGP_DIFF_CASE(32)
+#undef MGP_DIFF_CASE
+  return {nullptr, 0};
+}
+
+DiffSymKernel pick_diff_sym(int kind, int d) {
+  switch (kind) {
+    case KIND_RBF: return pick_diff_sym_d<KIND_RBF>(d);
+    case KIND_MATERN12: return pick_diff_sym_d<KIND_MATERN12>(d);
+    case KIND_MATERN32: return pick_diff_sym_d<KIND_MATERN32>(d);
+    default: return pick_diff_sym_d<KIND_MATERN52>(d);
+  }
+}
+
+// Half the values pay for the transposed products, their partial sums and the
+// reduction from here on, earlier where a value costs more (one-sided ->
+// symmetric us, Matern-1/2, 5 right-hand sides: d = 1 n = 10000 85 -> 89,
+// 12000 100 -> 102, 13500 128 -> 114; d = 5 9000 83 -> 87, 10300 110 -> 98;
+// d = 10 7000 74 -> 80, 8000 89 -> 84; d = 16 5000 70 -> 71, 6000 80 -> 74; d =
+// 24 5000 78 -> 83, 6500 114 -> 96).  Up to 4 right-hand sides the one-sided
+// kernel spends no matrix instructions.
+constexpr int64_t kDiffSymMin = 5500;
+constexpr int64_t kDiffSymBase = 12600, kDiffSymPerDim = 450;
+constexpr double kDiffSymMaxBytes = 8e9;  // of transposed partials (at most n^2 / 4)
+
+bool diff_sym_route(const MatvecArgs& a, const PackedPoints& rows, const PackedPoints& cols,
+                    int d, int nc, const MatvecWorkspace& ws) {
+  return a.square && &rows == &cols && a.m == a.n && ws.arena == nullptr && nc >= 5 && nc <= 16 &&
+         a.n >= kDiffSymMin && a.n + kDiffSymPerDim * d >= kDiffSymBase && (double)a.n * (double)a.n / 4 <= kDiffSymMaxBytes;
+}
+
+void diff_sym_matvec(const MatvecArgs& a, const PackedPoints& pts, int d, const float* V, int nc,
+                     float* out, MatvecWorkspace& ws, int cus, hipStream_t st) {
+  const DiffSymKernel k = pick_diff_sym(a.kind, d);
+  MGP_REQUIRE(k.fn != nullptr, "no difference kernel for this shape");
+  int per_cu = 0;
+  MGP_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      &per_cu, reinterpret_cast<const void*>(k.fn), 64 * kDiffWaves, 0));
+  const int64_t n = a.n, nb = ceil_div(n, (int64_t)k.block), hmax = nb / 2;
+  const int64_t stages = (hmax + 1) * (k.block / kDiffSymStage);
+  const int64_t slots = (int64_t)std::max(cus, 1) * std::max(per_cu, 1);
+  // rounds of (stages a workgroup + about half of one of set-up)
+  int64_t splits = 1;
+  double best = 0.0;
+  for (int64_t s = 1; s <= std::min<int64_t>(stages, 64); ++s) {
+    const int64_t sps = ceil_div(stages, s);
+    if (ceil_div(stages, sps) != s) continue;
+    const double cost = (double)ceil_div(nb * s, slots) * ((double)sps + 0.5) + 0.05 * (double)s;
+    if (s == 1 || cost < best) {
+      best = cost;
+      splits = s;
+    }
+  }
+  float* fwd = ws.partial.ensure((size_t)splits * 16 * nb * k.block);
+  float* tp = ws.sym_tp.ensure((size_t)std::max<int64_t>(nb * hmax, 1) * k.block * 16);
+  hipLaunchKernelGGL(k.fn, dim3((unsigned)nb, (unsigned)splits), dim3(64 * kDiffWaves), 0, st,
+                     pts.z.ptr, n, d, V, nc, nb, ceil_div(stages, splits), hmax, pts.exp2_limit,
+                     fwd, tp);
+  hipLaunchKernelGGL(k_diff_sym_reduce, dim3((unsigned)ceil_div(4 * n, 256)), dim3(256), 0, st, fwd,
+                     (int)splits, tp, k.block, nb, hmax, n, nc, a.outputscale, a.noise, V, out);
+  MGP_HIP_CHECK(hipGetLastError());
+}
+
 }  // namespace
 
 void direct_matvec(const MatvecArgs& a, const PackedPoints& rows, const PackedPoints& cols, int d,
@@ -302,6 +586,12 @@ void direct_matvec(const MatvecArgs& a, const PackedPoints& rows, const PackedPo
     const int left = a.ncols - c0;
     const int form = left == 1 ? kDiff1 : left <= 4 ? kDiff4 : left <= 16 ? kDiff16 : kDiff64;
     const int nc = std::min(kDiffCols[form], left);
+    if (diff_sym_route(a, rows, cols, d, nc, ws)) {
+      diff_sym_matvec(a, rows, d, V_dev + (int64_t)c0 * a.n, nc, out_dev + (int64_t)c0 * a.m, ws,
+                      cus, st);
+      c0 += nc;
+      continue;
+    }
     const DiffKernel k = pick_diff(a.kind, form, d);
     MGP_REQUIRE(k.fn != nullptr, "no difference kernel for this shape");
     const int64_t row_blocks = ceil_div(a.m, k.rows);

@@ -87,3 +87,25 @@ def test_fixed_arena(n, t):
         src.free()
         dst.free()
     assert _err(got, want) <= 2e-7  # the same fp64 sums in another order, rounded once
+
+
+@pytest.mark.parametrize("kind", [ok.MATERN12, ok.RBF])
+@pytest.mark.parametrize("n,d,t", [(12151, 1, 5), (11264, 3, 16), (10241, 6, 70), (7296, 12, 11),
+                                   (5503, 32, 7)])
+def test_symmetric_blocks(kind, n, d, t):
+    """Square products on unordered pairs: odd and even counts of 256- and
+    128-point blocks, ragged last stage, a second column chunk; repeated calls
+    bit for bit the same."""
+    rng = np.random.default_rng(n + d)
+    X = rng.normal(size=(n, d)).astype(np.float32)
+    V = rng.normal(size=(t, n)).astype(np.float32)
+    params = np.concatenate([rng.uniform(0.7, 1.4, d) * np.sqrt(d), [1.2]]).astype(np.float32)
+    p = NativeProvider(kind, True, X, params, 0.1)
+    try:
+        got = p.direct_matvec(V)
+        assert np.array_equal(got, p.direct_matvec(V))
+    finally:
+        p.close()
+    rows = np.unique(np.concatenate([np.arange(0, n, 31), np.arange(n - 70, n)]))
+    ref = ok.forward_matvec(kind, X, V, params, 0.1, True, rows=rows)
+    assert _err(got[:, rows], ref) <= 2e-6
