@@ -1273,7 +1273,8 @@ struct LanczosSolve {
                        j > 0 ? Q.ptr + (size_t)(j - 1) * n : nullptr, part.ptr, nb, j, r, ab.ptr,
                        stop.ptr, n);
     // Full re-orthogonalisation against Q_0..Q_j, at most two passes; the
-    // second pass runs only if the first saw an inner product >= 1e-5.
+    // second pass runs only if the first saw an inner product >= 1e-5 or >=
+    // 1/100 of the last beta.
     for (int pass = 0; pass < 2; ++pass) {
       double* c = coef.ptr + (size_t)pass * r;
       const double* first = pass ? coef.ptr : nullptr;

@@ -172,13 +172,14 @@ struct MatvecWorkspace {
   int64_t tile_calls = 0;
 };
 
-// A square product (rows and cols the same packed points) with 1..16
-// right-hand sides runs on the symmetric kernel, which forms each
-// off-diagonal kernel value once for both of its entries, when the points fill
-// at least kSymMinBlocks 512-point blocks (n >= 47 * 512 + 1 = 24065) and its
-// transposed partial sums (n^2/16 bytes) stay within kSymMaxBytes.  The environment variable
+// A square product (rows and cols the same packed points) forms each
+// off-diagonal kernel value once for both of its entries: with 3..16 right-hand
+// sides on k_sym_tile, when the points fill at least kSymMinBlocks 512-point
+// blocks (n >= 47 * 512 + 1 = 24065), with 1 and 2 on k_sym_vec from
+// kSymVecMinPoints points on, while the transposed partial sums (n^2/16 bytes
+// for k_sym_tile) stay within kSymMaxBytes.  The environment variable
 // MGP_SYM_MATVEC=0 turns that route off, =1 takes it for every square product
-// the kernel can serve (any n), for tests and measurements.
+// the kernels can serve (any n), for tests and measurements.
 void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
                   const PackedPoints& cols, const float* V_dev, float* out_dev,
                   MatvecWorkspace& ws, hipStream_t st, int force_splits = 0);
@@ -228,10 +229,10 @@ struct SmallCg {
 // the fixed-arena mode rejects the call.
 size_t fused_matvec_min_arena(const PackedPoints& cols, int ncols);
 
-// Reference-form product evaluated per pair from per-dimension differences of
-// the scaled coordinates (no Gram form; direct.hip).  Used as an independent
-// device cross-check and for dimensions beyond the MFMA tile path.
-// Split partials come from ws (its fixed arena when it has one).
+// Product evaluated per pair from per-dimension differences of the scaled
+// coordinates (no Gram form; direct.hip): Matern-1/2, point sets beyond the Gram
+// bound, dimensions beyond the MFMA tile path, and an independent cross-check.
+// Partials come from ws (its fixed arena when it has one).
 void direct_matvec(const MatvecArgs& a, const PackedPoints& rows,
                    const PackedPoints& cols, int d, const float* V_dev,
                    float* out_dev, MatvecWorkspace& ws, hipStream_t st);

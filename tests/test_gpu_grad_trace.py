@@ -80,8 +80,8 @@ def test_mfma_trace_matches_pair_loop_and_oracle(monkeypatch, kind, ard, d, n, T
 
 @pytest.mark.parametrize("kind,d", [(ok.MATERN52, 16), (ok.RBF, 8)])
 def test_mfma_trace_auto_route_at_size(monkeypatch, kind, d):
-    """From 4096 points on the default route is the matrix-core trace: its
-    gradient matches the pair-loop trace of the same solves."""
+    """At this size the default route is the matrix-core trace: its gradient
+    matches the difference-form trace of the same solves."""
     n = 20_000
     rng = np.random.default_rng(d)
     X = rng.normal(size=(n, d)).astype(np.float32)
