@@ -641,6 +641,10 @@ BBMMResult bbmm_step(Provider& pv, Precond& P, bool use_precond, const float* y_
   out.converged = cg.converged;
   out.cg_loop_ms = cg.loop_ms;
   out.alpha_dev = sol;
+  // the probe norms arrive with the dot product's wait
+  std::vector<float> norms(std::max(T, 1), 1.0f);
+  if (T > 0)
+    MGP_HIP_CHECK(hipMemcpyAsync(norms.data(), pn, T * sizeof(float), hipMemcpyDeviceToHost, st));
   out.inv_quad = dot_f(y_c, sol, n, w.part, st);
 
   float logdet = 0.0f;
@@ -655,10 +659,6 @@ BBMMResult bbmm_step(Provider& pv, Precond& P, bool use_precond, const float* y_
   out.nll = (0.5f * out.inv_quad + 0.5f * logdet + constant) / (float)n;
 
   // Gradient factors: Lf = [-alpha/2 | (0.5/T) U], Rf = [alpha | P^-1 Z].
-  std::vector<float> norms(std::max(T, 1), 1.0f);
-  if (T > 0)
-    MGP_HIP_CHECK(hipMemcpyAsync(norms.data(), pn, T * sizeof(float), hipMemcpyDeviceToHost, st));
-  MGP_HIP_CHECK(hipStreamSynchronize(st));
   std::vector<float> lfac(C), rfac(C);
   lfac[0] = -0.5f;
   rfac[0] = 1.0f;

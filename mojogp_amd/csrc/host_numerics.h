@@ -16,10 +16,11 @@ namespace mgp {
 
 // Eigen-decomposition of a symmetric tridiagonal matrix (diag d[m], off e[m-1])
 // by implicit QL with Wilkinson shifts.  Eigenvalues ascending in `evals`;
-// `evecs` (row-major m x m, columns are eigenvectors) if non-null.  Returns
-// false if an eigenvalue failed to converge within 1000*m sweeps.
+// `evecs` (row-major, columns are eigenvectors) if non-null: the first `rows`
+// rows of the m x m matrix, all of them by default.  Returns false if an
+// eigenvalue failed to converge within 1000*m sweeps.
 bool tridiag_eigh(const std::vector<double>& d, const std::vector<double>& e,
-                  std::vector<double>& evals, std::vector<double>* evecs);
+                  std::vector<double>& evals, std::vector<double>* evecs, int rows = -1);
 
 // SLQ estimate of log|A| from per-probe tridiagonals (GPyTorch conventions of
 // the reference: skip probes with NaN/+-1e20 entries, skip negative

@@ -6,14 +6,22 @@
 
 namespace mgp {
 
+// sqrt(a^2 + b^2): the plain form where the squares stay inside the exponent
+// range (hypot took 40% of a QL sweep), hypot elsewhere and for NaN.
+static inline double norm2(double a, double b) {
+  const double t = a * a + b * b;
+  return t > 1e-200 && t < 1e300 ? std::sqrt(t) : std::hypot(a, b);
+}
+
 bool tridiag_eigh(const std::vector<double>& diag, const std::vector<double>& off,
-                  std::vector<double>& evals, std::vector<double>* evecs) {
+                  std::vector<double>& evals, std::vector<double>* evecs, int rows) {
   const int m = (int)diag.size();
+  rows = rows < 0 ? m : std::min(rows, m);
   std::vector<double> d(diag), e(m, 0.0);
   for (int i = 0; i + 1 < m; ++i) e[i] = i < (int)off.size() ? off[i] : 0.0;
   if (evecs) {
-    evecs->assign((size_t)m * m, 0.0);
-    for (int i = 0; i < m; ++i) (*evecs)[(size_t)i * m + i] = 1.0;
+    evecs->assign((size_t)rows * m, 0.0);
+    for (int i = 0; i < rows; ++i) (*evecs)[(size_t)i * m + i] = 1.0;
   }
   const int max_sweeps = 1000 * std::max(m, 1);
   for (int l = 0; l < m; ++l) {
@@ -28,14 +36,14 @@ bool tridiag_eigh(const std::vector<double>& diag, const std::vector<double>& of
       if (sweeps++ == max_sweeps) return false;
       // Wilkinson shift from the leading 2x2 block.
       double g = (d[l + 1] - d[l]) / (2.0 * e[l]);
-      double r = std::hypot(g, 1.0);
+      double r = norm2(g, 1.0);
       g = d[mm] - d[l] + e[l] / (g + std::copysign(r, g));
       double s = 1.0, c = 1.0, p = 0.0;
       int i = mm - 1;
       bool deflated = false;
       for (; i >= l; --i) {
         const double f = s * e[i], b = c * e[i];
-        r = std::hypot(f, g);
+        r = norm2(f, g);
         e[i + 1] = r;
         if (r == 0.0) {
           d[i + 1] -= p;
@@ -52,7 +60,7 @@ bool tridiag_eigh(const std::vector<double>& diag, const std::vector<double>& of
         g = c * r - b;
         if (evecs) {
           double* V = evecs->data();
-          for (int k = 0; k < m; ++k) {
+          for (int k = 0; k < rows; ++k) {
             const double fv = V[(size_t)k * m + i + 1];
             V[(size_t)k * m + i + 1] = s * V[(size_t)k * m + i] + c * fv;
             V[(size_t)k * m + i] = c * V[(size_t)k * m + i] - s * fv;
@@ -74,7 +82,7 @@ bool tridiag_eigh(const std::vector<double>& diag, const std::vector<double>& of
       std::swap(d[i], d[k]);
       if (evecs) {
         double* V = evecs->data();
-        for (int r = 0; r < m; ++r) std::swap(V[(size_t)r * m + i], V[(size_t)r * m + k]);
+        for (int r = 0; r < rows; ++r) std::swap(V[(size_t)r * m + i], V[(size_t)r * m + k]);
       }
     }
   }
@@ -105,7 +113,10 @@ float slq_logdet(const std::vector<std::vector<float>>& diags,
     }
     if (bad) continue;
     std::vector<double> ev, V;
-    if (!tridiag_eigh(d, e, ev, &V)) continue;
+    // The rotations mix the columns of V row by row, so the first components
+    // need the first row alone: O(m^2) instead of O(m^3) (10 probes, m = 20:
+    // 375 -> 149 us, m = 30: 909 -> 327 us, with norm2).
+    if (!tridiag_eigh(d, e, ev, &V, 1)) continue;
     float max_eig = 1e-10f;
     for (int i = 0; i < m; ++i) max_eig = std::max(max_eig, (float)ev[i]);
     const float clamp = max_eig * 1e-6f;
