@@ -397,6 +397,7 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
           float* sc = tsc[wave][r & 1];
           *reinterpret_cast<f4*>(sc + lm * VS + 4 * lq) =
               f4{kv[r][0], kv[r][1], kv[r][2], kv[r][3]};
+          wave_lds_sync();  // (the other buffer's reads, too, stay before its next store)
 #pragma unroll
           for (int s = 0; s < 4; ++s)
             d2 = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[(4 * lq + s) * VS + lm], vr[r][s], d2, 0,

@@ -41,6 +41,15 @@ __device__ __forceinline__ uint64_t tr_read(const uint64_t* p) {
   return __builtin_bit_cast(uint64_t, v);
 }
 
+// Orders a wave's LDS stores before the loads that follow, in which other lanes
+// of the same wave read them.  The hardware keeps a wave's LDS accesses in
+// order; this holds the compiler to it (no instruction is emitted).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The chunk lane `lane` fetches for the transposed operand of a 16x16 tile.
 __device__ __forceinline__ int sym_read_chunk(int lane) {
   return sym_chunk(4 * (lane >> 4) + ((lane >> 2) & 3), lane & 3);

@@ -608,6 +608,12 @@ std::string tree_sym_source(const KernelTree& t) {
     << "\n#define R " << kTreeSymBlock / 64 << "\n#define ST " << kTreeSymStage << "\n"
     << R"(typedef float f4m __attribute__((ext_vector_type(4)));
 #define VS 20
+// a wave's LDS stores before its later loads of other lanes' words
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 extern "C" __global__ __launch_bounds__(256) void k_tree_sym_jit(
     const float* __restrict__ X, long long n, const float* __restrict__ p,
     const float* __restrict__ V, int nc, long long nb, long long splits, long long sps,
@@ -690,6 +696,7 @@ extern "C" __global__ __launch_bounds__(256) void k_tree_sym_jit(
           float* sc = tsc[wave][r & 1];
           *reinterpret_cast<f4m*>(sc + lm * VS + 4 * lq) =
               f4m{kv[r][0], kv[r][1], kv[r][2], kv[r][3]};
+          wave_lds_sync();  // (the other buffer's reads, too, stay before its next store)
 #pragma unroll
           for (int s = 0; s < 4; ++s)
             d2 = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[(4 * lq + s) * VS + lm], vr[r][s], d2, 0,
