@@ -6,16 +6,21 @@
 //   fused_forward_matvec_ncols  mojogp/codegen_engine/emit/gpu_kernel.py:151-260
 //   fused_cross_matvec_ncols    mojogp/codegen_engine/emit/gpu_kernel.py:487-565
 //
-// Per pair 2 d + ~5 VALU instructions form the value, which enters the product
-// with the right-hand sides as an operand of the fp32 matrix cores
-// (v_mfma_f32_16x16x4_f32: the values keep their 24 bits, so a product is as
-// accurate as one accumulated on the VALU) or, for up to 4 right-hand sides,
-// VALU FMAs.  Issue bound: at d = 5 the value costs ~62 cycles per 64 pairs
-// and the matrix instruction 32, ~250 us for n = 20011 one-sided; measured 313
-// to 330 us with the reduction (11 right-hand sides, Matern-1/2) and 263 us
-// over unordered pairs, against 18.7 ms for one row per thread with every
-// product added in fp64 (79 workgroups, run-time dimension loops).  Splitting the values for the 16-bit matrix cores
-// would shorten the matrix part but costs accuracy that these products had.
+// Per pair 2 d + ~5 VALU instructions form the fp32 value, which enters the
+// product with the right-hand sides in fp64: as an operand of
+// v_mfma_f64_16x16x4_f64 or, for up to 4 right-hand sides, of VALU FMAs.
+// Issue bound: at d = 5 the value costs ~62 cycles per 64 pairs, the matrix
+// instruction 64, so 200 us (side by side) to 320 us for n = 20011 one-sided;
+// measured 411 us with the reduction (11 right-hand sides, Matern-1/2) and 373
+// us over unordered pairs, against 18.7 ms for one row per thread (79
+// workgroups, run-time dimension loops).
+//
+// fp32 matrix sums (64 columns before fp64) took 330 and 263 us, but lost
+// accuracy that one fp64 addition per product had: relative error of rough
+// right-hand sides, one addition / fp32 sums / here: d = 1, n = 3001, 11
+// columns 7.7e-8 / 1.8e-7 / 5.8e-8; d = 5, n = 12807 1.4e-7 / 2.2e-7 / 1.4e-7;
+// of a predictive mean (alpha's terms cancel), n = 3001 3.6e-6 / 6.9e-6 /
+// 3.0e-6.
 #include "kval.h"
 #include "matvec.h"
 #include "sym_common.h"
@@ -28,6 +33,7 @@ namespace mgp {
 namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef double d4 __attribute__((ext_vector_type(4)));
 
 constexpr int kDiffTile = 64;    // column points per LDS tile
 constexpr int kDiffWaves = 4;    // waves per workgroup
@@ -38,8 +44,9 @@ enum DiffForm { kDiff1 = 0, kDiff4, kDiff16, kDiff64, kDiffForms };
 constexpr int kDiffCols[kDiffForms] = {1, 4, 16, 64};
 
 // 16-row tiles per wave: row coordinates (R x D) and accumulators stay in
-// registers with at least 3 waves per SIMD (n = 30000, 16 right-hand sides:
-// d = 16 1.12 ms with 4, 1.03 ms with 2; d = 5 at n = 20011 332 and 344 us).
+// registers with at least 3 waves per SIMD (n = 30000, 16 right-hand sides,
+// symmetric: d = 16 1.05 ms with 4, 0.98 ms with 2; d = 5 0.74 and 0.76 ms; one
+// right-hand side at d = 24 1.21 and 1.12 ms).
 constexpr int diff_rows(int D, int form) {
   return D > 10 || form == kDiff64 ? 2 : 4;
 }
@@ -52,9 +59,9 @@ __device__ __forceinline__ float diff_epilogue(double tot, float os, float noise
 // Sums over the columns [y tps 64, (y + 1) tps 64) of split y, for rows
 // i0 + 16 r + lane%16 of each wave.  Step s of a column tile: lane l evaluates
 // the pairs (row 16 r + l%16, column 4 s + l/16), r < R, from one LDS read of
-// the column point; they are the A operand of v_mfma_f32_16x16x4_f32 with
-// B = V[column][l%16], whose result holds rows 16 r + 4 (l/16) + q of
-// right-hand side l%16.  fp32 within a tile (64 columns), fp64 across tiles.
+// the column point; they are the A operand of v_mfma_f64_16x16x4_f64 with
+// B = V[column][l%16], whose result holds rows 16 r + 4 q + l/16 of right-hand
+// side l%16.  Products and sums in fp64 throughout.
 // part != nullptr: part[(y nc + c) m + i] = the fp64 sums; else (one split)
 // the epilogue out = os sum (+ noise V).
 template <int KIND, int D, int FORM>
@@ -81,13 +88,15 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_tile(
 #pragma unroll
     for (int k = 0; k < D; ++k) xi[r][k] = (i < m && k < d) ? Zr[i * d + k] : 0.0f;
   }
-  // fp64 sums: MFMA form [r][g][q], VALU form [r][c] of this lane's columns
-  constexpr int NA = MFMA ? 4 * G : NC;
-  double accd[R][NA];
+  d4 am[R][G];        // matrix forms
+  double acc[R][NC];  // VALU forms: this lane's columns
 #pragma unroll
-  for (int r = 0; r < R; ++r)
+  for (int r = 0; r < R; ++r) {
 #pragma unroll
-    for (int a = 0; a < NA; ++a) accd[r][a] = 0.0;
+    for (int g = 0; g < G; ++g) am[r][g] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[r][c] = 0.0;
+  }
 
   const int64_t tiles = (n + kDiffTile - 1) / kDiffTile;
   const int64_t t0 = (int64_t)blockIdx.y * tps, t1 = min(tiles, t0 + tps);
@@ -105,16 +114,6 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_tile(
       sv[jj * NC + c] = (jj < cnt && c < nc) ? V[(int64_t)c * n + j0 + jj] : 0.0f;
     }
     __syncthreads();
-    // fp32 within the tile, fp64 across tiles
-    float acc[R][NA];
-    f4 am[R][G];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-#pragma unroll
-      for (int a = 0; a < NA; ++a) acc[r][a] = 0.0f;
-#pragma unroll
-      for (int g = 0; g < G; ++g) am[r][g] = f4{0.f, 0.f, 0.f, 0.f};
-    }
     const int steps = (cnt + 3) / 4;
 #pragma unroll 2
     for (int s = 0; s < steps; ++s) {
@@ -131,13 +130,13 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_tile(
           for (int e = 0; e < 4; ++e) xj[k + e] = x[e];
         }
       }
-      float v[MFMA ? G : NC];
+      double v[MFMA ? G : NC];
       if constexpr (MFMA) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) v[g] = sv[jj * NC + 16 * g + lm];
+        for (int g = 0; g < G; ++g) v[g] = (double)sv[jj * NC + 16 * g + lm];
       } else {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) v[c] = sv[jj * NC + c];
+        for (int c = 0; c < NC; ++c) v[c] = (double)sv[jj * NC + c];
       }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -147,27 +146,15 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_tile(
           const float df = xi[r][k] - xj[k];
           r2 = fmaf(df, df, r2);
         }
-        const float kv = kval<KIND>(r2, lim);
+        const double kv = (double)kval<KIND>(r2, lim);
         if constexpr (MFMA) {
 #pragma unroll
           for (int g = 0; g < G; ++g)
-            am[r][g] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv, v[g], am[r][g], 0, 0, 0);
+            am[r][g] = __builtin_amdgcn_mfma_f64_16x16x4f64(kv, v[g], am[r][g], 0, 0, 0);
         } else {
 #pragma unroll
-          for (int c = 0; c < NC; ++c) acc[r][c] = fmaf(kv, v[c], acc[r][c]);
+          for (int c = 0; c < NC; ++c) acc[r][c] = fma(kv, v[c], acc[r][c]);
         }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if constexpr (MFMA) {
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) accd[r][4 * g + q] += (double)am[r][g][q];
-      } else {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) accd[r][c] += (double)acc[r][c];
       }
     }
   }
@@ -187,12 +174,12 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_tile(
 #pragma unroll
       for (int g = 0; g < G; ++g)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) put(16 * g + lm, i0 + 16 * r + 4 * lq + q, accd[r][4 * g + q]);
+        for (int q = 0; q < 4; ++q) put(16 * g + lm, i0 + 16 * r + 4 * q + lq, am[r][g][q]);
     } else {
       // the four lane groups hold the row's columns 4 s + l/16: fold them
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
-        double tot = accd[r][c];
+        double tot = acc[r][c];
         tot += __shfl_xor(tot, 16);
         tot += __shfl_xor(tot, 32);
         if (lq == 0) put(c, i0 + 16 * r + lm, tot);
@@ -294,13 +281,13 @@ int64_t diff_splits(int64_t row_blocks, int64_t tiles, int64_t slots) {
 // evaluates the pairs (row lane%16, columns 4 (lane/16) + s), the A operands of
 // out_I += K V_J; their rows go through a wave-private LDS tile (stride 20:
 // conflict-free both ways) and come back as the A operands of out_J += K^T V_I
-// with the rows' right-hand sides in registers.  The waves' transposed sums
-// are added in LDS and written per stage.  The value's 2 d + 7 instructions
-// are paid once for two entries, the matrix instructions (32 cycles per 4
-// columns of a tile) per entry.  Matern-1/2, 16 right-hand sides, one-sided ->
-// here: d = 5 n = 20011 321 -> 266 us, n = 40000 1147 -> 837; d = 16 1816 ->
-// 1213 at n = 40000.
-// fwd[(split 16 + c) npad + i] (fp64 across stages, then float),
+// with the rows' right-hand sides in registers, both in fp64 (as k_diff_tile).
+// The waves' transposed sums are added in LDS and written per stage.  The
+// value's 2 d + 7 instructions are paid once for two entries, the matrix
+// instructions (64 cycles per 4 columns of a tile) per entry.  Matern-1/2, 16
+// right-hand sides, one-sided -> here: d = 1 n = 30000 685 -> 649 us; d = 5 n =
+// 20011 417 -> 378, n = 30000 871 -> 737; d = 16 n = 30000 1177 -> 982.
+// fwd[(split 16 + c) npad + i] (one rounding per split, as tp's per stage),
 // tp[((b hmax + delta - 1) BLK + j) 16 + c].
 // ---------------------------------------------------------------------------
 constexpr int kDiffSymStage = 64;
@@ -317,13 +304,14 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
   __shared__ __align__(16) float sx[ST * DS];
   __shared__ __align__(16) float sv[ST * VS];
   __shared__ __align__(16) float tsc[kDiffWaves][2][16 * VS];
-  __shared__ f4 tbuf[kDiffWaves][ST / 16][64];
+  __shared__ d4 tbuf[kDiffWaves][ST / 16][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lm = lane & 15, lq = lane >> 4;
   const int64_t b = blockIdx.x, split = blockIdx.y, npad = nb * BLK;
   const int64_t i0 = b * BLK + wave * (16 * R);
-  float xi[R][D], vr[R][4];
+  float xi[R][D];
+  double vr[R][4];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int64_t i = i0 + 16 * r + lm;
@@ -332,14 +320,12 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int64_t ii = i0 + 16 * r + 4 * lq + s;
-      vr[r][s] = (ii < n && lm < nc) ? V[(int64_t)lm * n + ii] : 0.0f;
+      vr[r][s] = (ii < n && lm < nc) ? (double)V[(int64_t)lm * n + ii] : 0.0;
     }
   }
-  double acc[R][4];
+  d4 acc[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) acc[r][q] = 0.0;
+  for (int r = 0; r < R; ++r) acc[r] = d4{0.0, 0.0, 0.0, 0.0};
   const int64_t g0 = split * sps, g1 = min(g0 + sps, (sym_span(b, nb) + 1) * per);
   for (int64_t g = g0; g < g1; ++g) {
     const int64_t dl = g / per;
@@ -356,12 +342,9 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
       sv[jj * VS + c] = (c < nc && j0 + jj < n) ? V[(int64_t)c * n + j0 + jj] : 0.0f;
     }
     __syncthreads();
-    f4 d1[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) d1[r] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int ct = 0; ct < ST / 16; ++ct) {
-      f4 d2 = f4{0.f, 0.f, 0.f, 0.f};
+      d4 d2 = d4{0.0, 0.0, 0.0, 0.0};
       float kv[R][4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
@@ -378,7 +361,7 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
             for (int e = 0; e < 4; ++e) xj[k + e] = x[e];
           }
         }
-        const float v = sv[jj * VS + lm];
+        const double v = (double)sv[jj * VS + lm];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           float r2 = 0.0f;
@@ -388,7 +371,7 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
             r2 = fmaf(df, df, r2);
           }
           kv[r][s] = kval<KIND>(r2, lim);
-          d1[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[r][s], v, d1[r], 0, 0, 0);
+          acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)kv[r][s], v, acc[r], 0, 0, 0);
         }
       }
       if (dl > 0) {
@@ -400,19 +383,15 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
           wave_lds_sync();  // (the other buffer's reads, too, stay before its next store)
 #pragma unroll
           for (int s = 0; s < 4; ++s)
-            d2 = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[(4 * lq + s) * VS + lm], vr[r][s], d2, 0,
-                                                      0, 0);
+            d2 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)sc[(4 * lq + s) * VS + lm], vr[r][s],
+                                                      d2, 0, 0, 0);
         }
         tbuf[wave][ct][lane] = d2;
       }
     }
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc[r][q] += (double)d1[r][q];
     __syncthreads();
     if (dl > 0) {
-      // lane of column tile ct: columns 4 (lane/16) + q, right-hand side lane%16
+      // lane of column tile ct: columns 4 q + lane/16, right-hand side lane%16
       float* dst = tp + ((b * hmax + dl - 1) * BLK + (g % per) * ST) * 16;
       for (int q = threadIdx.x; q < ST * 4; q += 64 * kDiffWaves) {
         const int ct = q >> 6, ln = q & 63;
@@ -420,10 +399,10 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
 #pragma unroll
         for (int w = 0; w < kDiffWaves; ++w)
 #pragma unroll
-          for (int k = 0; k < 4; ++k) t[k] += (double)tbuf[w][ct][ln][k];
+          for (int k = 0; k < 4; ++k) t[k] += tbuf[w][ct][ln][k];
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          dst[(16 * ct + 4 * (ln >> 4) + k) * 16 + (ln & 15)] = (float)t[k];
+          dst[(16 * ct + 4 * k + (ln >> 4)) * 16 + (ln & 15)] = (float)t[k];
       }
     }
   }
@@ -431,7 +410,7 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_sym(
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      fwd[(split * 16 + lm) * npad + i0 + 16 * r + 4 * lq + q] = (float)acc[r][q];
+      fwd[(split * 16 + lm) * npad + i0 + 16 * r + 4 * q + lq] = (float)acc[r][q];
 }
 
 // out[c][j] = os (split sums + the transposed partials of the row blocks that
@@ -523,19 +502,22 @@ DiffSymKernel pick_diff_sym(int kind, int d) {
 
 // Half the values pay for the transposed products, their partial sums and the
 // reduction from here on, earlier where a value costs more (one-sided ->
-// symmetric us, Matern-1/2, 5 right-hand sides: d = 1 n = 10000 85 -> 89,
-// 12000 100 -> 102, 13500 128 -> 114; d = 5 9000 83 -> 87, 10300 110 -> 98;
-// d = 10 7000 74 -> 80, 8000 89 -> 84; d = 16 5000 70 -> 71, 6000 80 -> 74; d =
-// 24 5000 78 -> 83, 6500 114 -> 96).  Up to 4 right-hand sides the one-sided
-// kernel spends no matrix instructions.
+// symmetric us, Matern-1/2, 11 right-hand sides: d = 1 n = 14000 171 -> 183,
+// 16000 217 -> 215, 30000 679 -> 643; d = 3 11000 133 -> 141, 14000 198 -> 194;
+// d = 5 11000 144 -> 150, 12000 169 -> 152; d = 10 7000 90 -> 102, 8000 108 ->
+// 106, 9000 144 -> 127; d = 16 5000 84 -> 81, 6000 95 -> 84, 7000 110 -> 107; d =
+// 24 5000 90 -> 96, 6000 116 -> 100).  Up to 4 right-hand sides the one-sided
+// kernel spends no matrix instructions (n = 30000, d = 16, 4 columns: 865 ->
+// 942).
 constexpr int64_t kDiffSymMin = 5500;
-constexpr int64_t kDiffSymBase = 12600, kDiffSymPerDim = 450;
+constexpr int64_t kDiffSymBase = 15500, kDiffSymPerDim = 750;
 constexpr double kDiffSymMaxBytes = 8e9;  // of transposed partials (at most n^2 / 4)
 
 bool diff_sym_route(const MatvecArgs& a, const PackedPoints& rows, const PackedPoints& cols,
                     int d, int nc, const MatvecWorkspace& ws) {
   return a.square && &rows == &cols && a.m == a.n && ws.arena == nullptr && nc >= 5 && nc <= 16 &&
-         a.n >= kDiffSymMin && a.n + kDiffSymPerDim * d >= kDiffSymBase && (double)a.n * (double)a.n / 4 <= kDiffSymMaxBytes;
+         a.n >= kDiffSymMin && a.n + kDiffSymPerDim * d >= kDiffSymBase &&
+         (double)a.n * (double)a.n / 4 <= kDiffSymMaxBytes;
 }
 
 void diff_sym_matvec(const MatvecArgs& a, const PackedPoints& pts, int d, const float* V, int nc,

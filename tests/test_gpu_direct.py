@@ -91,7 +91,7 @@ def test_fixed_arena(n, t):
 
 @pytest.mark.parametrize("kind", [ok.MATERN12, ok.RBF])
 @pytest.mark.parametrize("n,d,t", [(12151, 1, 5), (11264, 3, 16), (10241, 6, 70), (7296, 12, 11),
-                                   (5503, 32, 7)])
+                                   (5503, 32, 7), (15105, 1, 5), (13313, 3, 16), (11265, 6, 70)])
 def test_symmetric_blocks(kind, n, d, t):
     """Square products on unordered pairs: odd and even counts of 256- and
     128-point blocks, ragged last stage, a second column chunk; repeated calls
@@ -109,3 +109,34 @@ def test_symmetric_blocks(kind, n, d, t):
     rows = np.unique(np.concatenate([np.arange(0, n, 31), np.arange(n - 70, n)]))
     ref = ok.forward_matvec(kind, X, V, params, 0.1, True, rows=rows)
     assert _err(got[:, rows], ref) <= 2e-6
+
+
+@pytest.mark.parametrize("kind", [ok.MATERN12, ok.MATERN52])
+@pytest.mark.parametrize("n,d,t", [(3001, 1, 1), (2000, 5, 3), (3001, 1, 11), (1500, 7, 40),
+                                   (15001, 1, 5), (13000, 4, 16), (6001, 24, 9)])
+def test_sums_are_fp64(kind, n, d, t):
+    """Right-hand sides without a common sign, on equal points: every kernel
+    value is exactly 1, so what is left is the rounding of the sums.  Products
+    and sums are fp64; the result is rounded once (one-sided, half an ulp), and
+    on unordered pairs (the last three) the partial sums once each, whose mean
+    squares add up to at most n, the result's own another n."""
+    rng = np.random.default_rng(n + t)
+    X = np.tile(rng.normal(size=d).astype(np.float32), (n, 1))
+    V = rng.normal(size=(t, n)).astype(np.float32)
+    os = np.float32(1.25)  # exact in any product below
+    p = NativeProvider(kind, False, X, np.array([0.7, os], np.float32), 0.5)
+    try:
+        got = p.direct_matvec(V).astype(np.float64)
+        cross = p.cross_matvec(X[:70], V) if kind == ok.MATERN12 else None
+    finally:
+        p.close()
+    V = V.astype(np.float64)
+    want = 1.25 * V.sum(axis=1, keepdims=True)
+    ulp = 2.0**-24 * (1 + 1e-6)
+    if cross is not None:
+        assert np.all(np.abs(cross - want) <= ulp * np.abs(want))
+    want = want + 0.5 * V
+    if n < 5500:
+        assert np.all(np.abs(got - want) <= ulp * np.abs(want))
+    else:
+        assert np.sqrt(np.mean((got - want) ** 2)) <= 1.25 * 2.0**-24 * np.sqrt(2.0 * n)
