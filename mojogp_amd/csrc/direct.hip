@@ -515,9 +515,11 @@ constexpr double kDiffSymMaxBytes = 8e9;  // of transposed partials (at most n^2
 
 bool diff_sym_route(const MatvecArgs& a, const PackedPoints& rows, const PackedPoints& cols,
                     int d, int nc, const MatvecWorkspace& ws) {
-  return a.square && &rows == &cols && a.m == a.n && ws.arena == nullptr && nc >= 5 && nc <= 16 &&
-         a.n >= kDiffSymMin && a.n + kDiffSymPerDim * d >= kDiffSymBase &&
-         (double)a.n * (double)a.n / 4 <= kDiffSymMaxBytes;
+  if (!a.square || &rows != &cols || a.m != a.n || ws.arena != nullptr || nc > 16) return false;
+  if ((double)a.n * (double)a.n / 4 > kDiffSymMaxBytes) return false;
+  const int mode = sym_switch();
+  if (mode >= 0) return mode == 1;
+  return nc >= 5 && a.n >= kDiffSymMin && a.n + kDiffSymPerDim * d >= kDiffSymBase;
 }
 
 void diff_sym_matvec(const MatvecArgs& a, const PackedPoints& pts, int d, const float* V, int nc,

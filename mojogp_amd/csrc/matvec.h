@@ -178,8 +178,9 @@ struct MatvecWorkspace {
 // blocks (n >= 47 * 512 + 1 = 24065), with 1 and 2 on k_sym_vec from
 // kSymVecMinPoints points on, while the transposed partial sums (n^2/16 bytes
 // for k_sym_tile) stay within kSymMaxBytes.  The environment variable
-// MGP_SYM_MATVEC=0 turns that route off, =1 takes it for every square product
-// the kernels can serve (any n), for tests and measurements.
+// MGP_SYM_MATVEC=0 turns every symmetric route off (these, the difference
+// products' and the kernel trees'), =1 takes it for every square product the
+// kernels can serve (any n), for tests and measurements.
 void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
                   const PackedPoints& cols, const float* V_dev, float* out_dev,
                   MatvecWorkspace& ws, hipStream_t st, int force_splits = 0);

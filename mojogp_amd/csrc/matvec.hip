@@ -2550,8 +2550,7 @@ bool sym_route(const MatvecArgs& a, const PackedPoints& rows, const PackedPoints
                const MatvecWorkspace& ws) {
   if (!a.square || a.mix != nullptr || ws.arena != nullptr || &rows != &cols) return false;
   if (nc < 1 || nc > 16 || a.m != a.n || a.n != rows.n) return false;
-  const char* env = std::getenv("MGP_SYM_MATVEC");
-  const int mode = env == nullptr ? -1 : (env[0] == '0' ? 0 : 1);
+  const int mode = sym_switch();
   if (mode == 0) return false;
   if (nc <= kSymVecCols) {
     const int64_t vb = ceil_div(std::max<int64_t>(a.n, 1), kVecRows);
@@ -2567,6 +2566,11 @@ bool sym_route(const MatvecArgs& a, const PackedPoints& rows, const PackedPoints
 }
 
 }  // namespace
+
+int sym_switch() {
+  const char* env = std::getenv("MGP_SYM_MATVEC");
+  return env == nullptr ? -1 : (env[0] == '0' ? 0 : 1);
+}
 
 bool symmetric_route_taken(const PackedPoints& pts, int ncols) {
   MatvecArgs a;

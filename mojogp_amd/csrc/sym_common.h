@@ -11,6 +11,10 @@ namespace mgp {
 
 constexpr int kXcds = 8;  // XCDs of the MI355X (workgroups are dealt to them in turn)
 
+// The environment variable MGP_SYM_MATVEC: -1 unset, 0 symmetric products off,
+// 1 taken for every square product their kernels can serve.
+int sym_switch();
+
 // Off-diagonal column blocks formed by row block b of nb: row block b forms
 // blocks (b, (b + delta) mod nb) for delta = 1 .. sym_span(b, nb), so every
 // unordered pair of distinct blocks is formed exactly once and every row

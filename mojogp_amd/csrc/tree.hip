@@ -405,8 +405,11 @@ void tree_sym_matvec(const KernelTree& t, const float* p_dev, const float* X, in
 }
 
 bool tree_sym_route(const KernelTree& t, int64_t m, int64_t n, int nc, bool square) {
-  return square && m == n && t.table_size == 0 && n >= kTreeSymMin && nc >= kTreeSymMinCols &&
-         (double)n * (double)n * 16 * 4 / 512 <= kTreeSymMaxBytes;
+  if (!square || m != n || t.table_size != 0) return false;
+  if ((double)n * (double)n * 16 * 4 / 512 > kTreeSymMaxBytes) return false;
+  const int mode = sym_switch();
+  if (mode >= 0) return mode == 1;
+  return n >= kTreeSymMin && nc >= kTreeSymMinCols;
 }
 }  // namespace
 
