@@ -80,7 +80,7 @@ def test_tree_products(monkeypatch, name, n, t):
 @pytest.mark.parametrize("kind", ["difference", "tree"])
 def test_off_above_the_automatic_line(monkeypatch, kind):
     rng = np.random.default_rng(3)
-    n, t = 13000, 8
+    n, t = 16000, 8  # the lines at d = 2: 14000 for the differences, less for the tree
     X = rng.normal(size=(n, 2)).astype(np.float32)
     V = rng.normal(size=(t, n)).astype(np.float32)
     if kind == "tree":
