@@ -150,7 +150,8 @@ __global__ __launch_bounds__(64 * kDiffWaves) void k_diff_tile(
         if constexpr (MFMA) {
 #pragma unroll
           for (int g = 0; g < G; ++g)
-            am[r][g] = __builtin_amdgcn_mfma_f64_16x16x4f64(kv, v[g], am[r][g], 0, 0, 0);
+            if (g == 0 || 16 * g < nc)  // (uniform) groups past nc hold no right-hand side
+              am[r][g] = __builtin_amdgcn_mfma_f64_16x16x4f64(kv, v[g], am[r][g], 0, 0, 0);
         } else {
 #pragma unroll
           for (int c = 0; c < NC; ++c) acc[r][c] = fma(kv, v[c], acc[r][c]);
@@ -511,6 +512,14 @@ DiffSymKernel pick_diff_sym(int kind, int d) {
 // 942).
 constexpr int64_t kDiffSymMin = 5500;
 constexpr int64_t kDiffSymBase = 15500, kDiffSymPerDim = 750;
+// 17 to 32 right-hand sides: two groups of the 64-column form evaluate as many
+// pairs as two symmetric passes and sum fewer partials, but keep fewer waves on
+// a CU.  Two groups -> two passes, 32 columns, us: d = 1 n = 14000 370 -> 376,
+// 20011 709 -> 652, 40000 2686 -> 2154; d = 5 12000 315 -> 294, 20011 799 ->
+// 743, 40000 2899 -> 2429; d = 16 9000 256 -> 281, 20011 1016 -> 955, 40000 3711
+// -> 3546; d = 24 20011 1172 -> 1270.
+constexpr int kDiffPairMaxDim = 16;
+constexpr int64_t kDiffPairMin = 20000;
 constexpr double kDiffSymMaxBytes = 8e9;  // of transposed partials (at most n^2 / 4)
 
 bool diff_sym_route(const MatvecArgs& a, const PackedPoints& rows, const PackedPoints& cols,
@@ -567,9 +576,12 @@ void direct_matvec(const MatvecArgs& a, const PackedPoints& rows, const PackedPo
   for (int c0 = 0; c0 < a.ncols;) {
     // up to 4 columns on the VALU (a value then costs at most 4 FMAs against
     // the 32 cycles of its matrix instruction), up to 16 in one matrix
-    // group; four groups share the values of a wider product
+    // group; up to four groups share the values of a wider product
     const int left = a.ncols - c0;
-    const int form = left == 1 ? kDiff1 : left <= 4 ? kDiff4 : left <= 16 ? kDiff16 : kDiff64;
+    int form = left == 1 ? kDiff1 : left <= 4 ? kDiff4 : left <= 16 ? kDiff16 : kDiff64;
+    if (left > 16 && left <= 32 && d <= kDiffPairMaxDim && a.n >= kDiffPairMin &&
+        diff_sym_route(a, rows, cols, d, 16, ws))
+      form = kDiff16;
     const int nc = std::min(kDiffCols[form], left);
     if (diff_sym_route(a, rows, cols, d, nc, ws)) {
       diff_sym_matvec(a, rows, d, V_dev + (int64_t)c0 * a.n, nc, out_dev + (int64_t)c0 * a.m, ws,

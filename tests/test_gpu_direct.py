@@ -140,3 +140,35 @@ def test_sums_are_fp64(kind, n, d, t):
         assert np.all(np.abs(got - want) <= ulp * np.abs(want))
     else:
         assert np.sqrt(np.mean((got - want) ** 2)) <= 1.25 * 2.0**-24 * np.sqrt(2.0 * n)
+
+
+@pytest.mark.parametrize("t", [17, 32, 33, 48, 49])
+def test_unused_column_groups(t):
+    """A product of 17 to 63 columns skips the 16-column groups it does not
+    fill: the same bits as the first columns of a full one."""
+    rng = np.random.default_rng(t)
+    n = 1333
+    X = rng.normal(size=(n, 3)).astype(np.float32)
+    V = rng.normal(size=(64, n)).astype(np.float32)
+    p = NativeProvider(ok.MATERN12, False, X, np.array([0.9, 1.1], np.float32), 0.1)
+    try:
+        assert np.array_equal(p.forward_matvec(V[:t]), p.forward_matvec(V)[:t])
+    finally:
+        p.close()
+
+
+@pytest.mark.parametrize("n,d,t", [(19999, 2, 20), (20000, 16, 17), (20003, 3, 32), (20001, 17, 24),
+                                   (20000, 1, 33)])
+def test_two_symmetric_passes(n, d, t):
+    """17 to 32 columns around the line where they run as two symmetric passes."""
+    rng = np.random.default_rng(n + t)
+    X = rng.normal(size=(n, d)).astype(np.float32)
+    V = rng.normal(size=(t, n)).astype(np.float32)
+    params = np.concatenate([rng.uniform(0.7, 1.4, d) * np.sqrt(d), [1.2]]).astype(np.float32)
+    p = NativeProvider(ok.MATERN12, True, X, params, 0.1)
+    try:
+        got = p.forward_matvec(V)
+    finally:
+        p.close()
+    rows = np.unique(np.concatenate([np.arange(0, n, 61), np.arange(n - 70, n)]))
+    assert _err(got[:, rows], ok.forward_matvec(ok.MATERN12, X, V, params, 0.1, True, rows=rows)) <= 2e-6
