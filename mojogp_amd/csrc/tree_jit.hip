@@ -325,7 +325,8 @@ std::string tree_source(const KernelTree& t) {
 // Backward pass of one pair and the final factors of its sums: the pair code
 // (after emit_tree's) adds w dK/dtheta_q, less a factor that depends on the
 // parameters only, into g[q]; fin holds that factor per parameter (C
-// expressions of p), applied once per thread.  False when two leaves or
+// expressions of p in double: rounded to fp32 it would scale the whole sum by
+// up to 1 + 2^-24), applied once per thread.  False when two leaves or
 // scales share a parameter slot (their factors differ).
 bool emit_tree_grad(const KernelTree& t, std::string& pair, std::vector<std::string>& fin) {
   std::ostringstream Q;
@@ -340,7 +341,7 @@ bool emit_tree_grad(const KernelTree& t, std::string& pair, std::vector<std::str
     used[(size_t)q] = 1;
     fin[(size_t)q] = factor;
   };
-  auto pq = [](int q) { return "p[" + std::to_string(q) + "]"; };
+  auto pq = [](int q) { return "(double)p[" + std::to_string(q) + "]"; };
   for (int i = 0; i < t.nnodes; ++i)
     Q << "  float a" << i << " = " << (i == t.nnodes - 1 ? "w" : "0.0f") << ";\n";
   for (int i = t.nnodes - 1; i >= 0; --i) {
@@ -383,7 +384,7 @@ bool emit_tree_grad(const KernelTree& t, std::string& pair, std::vector<std::str
       }
       for (int q = 0; q < nls; ++q)
         add(lf.p0 + q, h, lf.ard ? L + "x" + std::to_string(q) : L + "raw", factor);
-      add(ios, A, L, "1.0f / " + pq(ios));
+      add(ios, A, L, "1.0 / " + pq(ios));
       continue;
     }
     if (lf.kind == KIND_PERIODIC) {
@@ -397,12 +398,12 @@ bool emit_tree_grad(const KernelTree& t, std::string& pair, std::vector<std::str
           << "il" << (lf.ard ? q : 0) << ", " << L << "c);\n";
         if (lf.ard)
           add(lf.p0 + q, L + "h * " + n, n,
-              "2.0f / (" + pq(lf.p0 + q) + " * " + pq(lf.p0 + q) + ")");
+              "2.0 / (" + pq(lf.p0 + q) + " * " + pq(lf.p0 + q) + ")");
       }
-      if (!lf.ard) add(lf.p0, L + "h", L + "s", "2.0f / " + pq(lf.p0));
-      add(ip, L + "h", L + "c", "4.0f / " + pq(ip));
+      if (!lf.ard) add(lf.p0, L + "h", L + "s", "2.0 / " + pq(lf.p0));
+      add(ip, L + "h", L + "c", "4.0 / " + pq(ip));
       Q << "  g[" << ios << "] += " << L << "h;\n";
-      own(ios, "1.0f / " + pq(ios));
+      own(ios, "1.0 / " + pq(ios));
       continue;
     }
     // radial / RQ lengthscales: dk/dl_q = h u_q^2 / l_q with u_q = dx_q / l_q
@@ -428,12 +429,12 @@ bool emit_tree_grad(const KernelTree& t, std::string& pair, std::vector<std::str
     if (lf.ard)
       for (int q = 0; q < lf.ndim; ++q) {
         const std::string u = L + "u" + std::to_string(q);
-        add(lf.p0 + q, L + "h * " + u, u, "1.0f / " + pq(lf.p0 + q));
+        add(lf.p0 + q, L + "h * " + u, u, "1.0 / " + pq(lf.p0 + q));
       }
     else
-      add(lf.p0, L + "h", L + "r2", "1.0f / " + pq(lf.p0));
+      add(lf.p0, L + "h", L + "r2", "1.0 / " + pq(lf.p0));
     Q << "  g[" << ios << "] += " << L << "a;\n";
-    own(ios, "1.0f / " + pq(ios));
+    own(ios, "1.0 / " + pq(ios));
   }
   pair = Q.str();
   return ok;

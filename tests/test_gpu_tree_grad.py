@@ -81,3 +81,26 @@ def test_categorical_tree_is_not_folded():
     finally:
         p.close()
     _check(T, X, params, L, R, got)
+
+
+@pytest.mark.parametrize("n", [700, 9001])
+def test_parameter_factors_are_not_rounded(n):
+    """Equal points and small whole weights: every product and sum is exact in
+    fp32 or fp64, so the outputscale's trace, sum W, is exact too (a factor 1 /
+    outputscale rounded to fp32 would leave up to 6e-8)."""
+    node = RBF() + RQ()
+    rng = np.random.default_rng(n)
+    X = np.tile(np.array([[0.5, -1.0]], np.float32), (n, 1))
+    L, R = (rng.integers(1, 4, size=(3, n)).astype(np.float32) for _ in range(2))
+    p = NativeProvider(None, False, X, np.array([0.7, 3.0, 1.1, 1.3, 7.0], np.float32), 0.2,
+                       tree_spec=node.to_tree_spec(2))
+    try:
+        got = p.gradient_trace(L, R)
+    finally:
+        p.close()
+    want = float((L.astype(np.float64).sum(1) * R.astype(np.float64).sum(1)).sum())
+    print(f"n={n} relative", (got[[1, 4]] - want) / want, flush=True)
+    if n >= 9000:  # the generated kernel
+        assert np.all(np.abs(got[[1, 4]] - want) <= 1e-12 * want)
+    else:
+        assert np.all(np.abs(got[[1, 4]] - want) <= 16 * 2.0**-24 * want)
