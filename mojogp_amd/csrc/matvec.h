@@ -204,8 +204,12 @@ struct SmallCgScalars {
   float* hist_alpha;  // [max_tridiag][C]
   float* hist_beta;
 };
-// From here on a column's traffic through one CU costs more than the launches.
-constexpr int64_t kSmallCgMax = 16384;
+// From here on a column's traffic through one CU costs more than the launches:
+// us an iteration, separate kernels / this, 11 columns: RBF d = 1 n = 6000 40.4 /
+// 37.3, 8000 46.8 / 49.1, 16384 99 / 127; Matern-5/2 d = 6 43.7 / 41.2, 53.2 /
+// 55.8, 124 / 152; d = 16 45.2 / 42.6, 54.6 / 57.6, 136 / 165; 3 and 16 columns
+// within 1 us of these differences.
+constexpr int64_t kSmallCgMax = 7000;
 bool small_cg_route(int kind, const PackedPoints& pts, int ncols);
 struct SmallCg {
   MatvecArgs a;  // square, m = n = pts->n, ncols, outputscale, scalar noise

@@ -3067,8 +3067,8 @@ void SmallCg::step(float* x, float* r, float* p, const SmallCgScalars& s, int it
                      pairs_per_split, (int64_t)0, a.m, a.ncols, a.outputscale, a.noise, colmax,
                      (const float*)nullptr, (float*)nullptr, ws->partial.ptr, mpad, cpad);
   MGP_HIP_CHECK(hipGetLastError());
-  auto k = a.n <= 4096 ? k_cg_small<1> : a.n <= 8192 ? k_cg_small<2> : k_cg_small<4>;
-  static_assert(kSmallCgMax <= 4 * 4 * kSmallCgThreads, "quads per thread");
+  auto k = a.n <= 4096 ? k_cg_small<1> : k_cg_small<2>;
+  static_assert(kSmallCgMax <= 2 * 4 * kSmallCgThreads, "quads per thread");
   hipLaunchKernelGGL(k, dim3((unsigned)a.ncols), dim3(kSmallCgThreads), 0, st, ws->partial.ptr,
                      (int)splits, cpad, mpad, (int)a.n, a.outputscale, a.noise, noise_vec, x, r, p,
                      s, iter, max_tridiag, ncg == 0 ? 1 : 0, colmax, vp);

@@ -1,8 +1,8 @@
 """The two-launch CG iteration of small unpreconditioned systems against the
 general one (the symmetric product forced by MGP_SYM_MATVEC=1 takes the
-separate vector kernels): edges of the quads a thread carries (4096, 8192 and
-16384 points), ragged sizes, 1 .. 16 columns, a noise vector, and the oracle's
-solve at convergence.
+separate vector kernels): edges of the quads a thread carries (4096 points) and
+of the route (7000; larger sizes run the separate kernels on both sides), ragged
+sizes, 1 .. 16 columns, a noise vector, and the oracle's solve at convergence.
 
 Three iterations of the same recurrence on products that agree to ~2e-7:
 alpha and beta are ratios of inner products perturbed by ~1e-6, and more
@@ -48,7 +48,8 @@ def _bbmm(p, y, probes, iters, general):
 @pytest.mark.parametrize("n,probes,vec", [(5, 3, False), (63, 0, False), (1001, 15, True),
                                           (4096, 10, False), (4097, 10, True), (8193, 4, False),
                                           (16384, 10, False), (16381, 0, True),
-                                          (16385, 2, False)])
+                                          (16385, 2, False), (6999, 15, True), (7000, 3, False),
+                                          (7001, 10, False)])
 def test_iterations_match_the_general_path(n, probes, vec):
     rng = np.random.default_rng(n)
     d = 3
