@@ -531,7 +531,8 @@ bool diff_sym_route(const MatvecArgs& a, const PackedPoints& rows, const PackedP
   return nc >= 5 && a.n >= kDiffSymMin && a.n + kDiffSymPerDim * d >= kDiffSymBase;
 }
 
-void diff_sym_matvec(const MatvecArgs& a, const PackedPoints& pts, int d, const float* V, int nc,
+// False, with nothing launched, where its partial sums do not fit the device.
+bool diff_sym_matvec(const MatvecArgs& a, const PackedPoints& pts, int d, const float* V, int nc,
                      float* out, MatvecWorkspace& ws, int cus, hipStream_t st) {
   const DiffSymKernel k = pick_diff_sym(a.kind, d);
   MGP_REQUIRE(k.fn != nullptr, "no difference kernel for this shape");
@@ -553,14 +554,16 @@ void diff_sym_matvec(const MatvecArgs& a, const PackedPoints& pts, int d, const 
       splits = s;
     }
   }
-  float* fwd = ws.partial.ensure((size_t)splits * 16 * nb * k.block);
-  float* tp = ws.sym_tp.ensure((size_t)std::max<int64_t>(nb * hmax, 1) * k.block * 16);
+  float* fwd = ws.partial.try_ensure((size_t)splits * 16 * nb * k.block);
+  float* tp = ws.sym_tp.try_ensure((size_t)std::max<int64_t>(nb * hmax, 1) * k.block * 16);
+  if (fwd == nullptr || tp == nullptr) return false;
   hipLaunchKernelGGL(k.fn, dim3((unsigned)nb, (unsigned)splits), dim3(64 * kDiffWaves), 0, st,
                      pts.z.ptr, n, d, V, nc, nb, ceil_div(stages, splits), hmax, pts.exp2_limit,
                      fwd, tp);
   hipLaunchKernelGGL(k_diff_sym_reduce, dim3((unsigned)ceil_div(4 * n, 256)), dim3(256), 0, st, fwd,
                      (int)splits, tp, k.block, nb, hmax, n, nc, a.outputscale, a.noise, V, out);
   MGP_HIP_CHECK(hipGetLastError());
+  return true;
 }
 
 }  // namespace
@@ -583,9 +586,9 @@ void direct_matvec(const MatvecArgs& a, const PackedPoints& rows, const PackedPo
         diff_sym_route(a, rows, cols, d, 16, ws))
       form = kDiff16;
     const int nc = std::min(kDiffCols[form], left);
-    if (diff_sym_route(a, rows, cols, d, nc, ws)) {
-      diff_sym_matvec(a, rows, d, V_dev + (int64_t)c0 * a.n, nc, out_dev + (int64_t)c0 * a.m, ws,
-                      cus, st);
+    if (diff_sym_route(a, rows, cols, d, nc, ws) &&
+        diff_sym_matvec(a, rows, d, V_dev + (int64_t)c0 * a.n, nc, out_dev + (int64_t)c0 * a.m, ws,
+                        cus, st)) {
       c0 += nc;
       continue;
     }

@@ -2681,8 +2681,9 @@ VecFn pick_vec_cols(int kb, int nc) {
   return nc == 1 ? pick_vec<KIND, 1>(kb) : pick_vec<KIND, 2>(kb);
 }
 
-// out = (K + noise I) V for one or two columns of V (k_sym_vec).
-void sym_vec_matvec(const MatvecArgs& a, const PackedPoints& pts, const float* Vc, int nc,
+// out = (K + noise I) V for one or two columns of V (k_sym_vec).  False, with
+// nothing launched, where its partial sums do not fit the device.
+bool sym_vec_matvec(const MatvecArgs& a, const PackedPoints& pts, const float* Vc, int nc,
                     float* outc, MatvecWorkspace& ws, hipStream_t st) {
   const int64_t n = a.n, nb = ceil_div(std::max<int64_t>(n, 1), kVecRows), hmax = nb / 2;
   const int64_t npad = nb * kVecRows;
@@ -2699,9 +2700,10 @@ void sym_vec_matvec(const MatvecArgs& a, const PackedPoints& pts, const float* V
                                 64 * kVecWaves, (double)npad * 4, kVecStages);
   const int64_t sps = ceil_div((hmax + 1) * kVecStages, splits);
   splits = ceil_div((hmax + 1) * kVecStages, sps);
-  float* vp = ws.vpack.ensure((size_t)nc * npad);
-  float* fwd = ws.partial.ensure((size_t)splits * nc * npad);
-  float* tp = ws.sym_tp.ensure((size_t)std::max<int64_t>(nb * hmax, 1) * nc * kVecRows);
+  float* vp = ws.vpack.try_ensure((size_t)nc * npad);
+  float* fwd = ws.partial.try_ensure((size_t)splits * nc * npad);
+  float* tp = ws.sym_tp.try_ensure((size_t)std::max<int64_t>(nb * hmax, 1) * nc * kVecRows);
+  if (vp == nullptr || fwd == nullptr || tp == nullptr) return false;
   hipLaunchKernelGGL(k_pad_vec, dim3((unsigned)ceil_div(npad, 256), (unsigned)nc), dim3(256), 0,
                      st, Vc, n, npad, vp);
   if (ws.time_tile) MGP_HIP_CHECK(hipEventRecord(ws.ev0, st));
@@ -2718,9 +2720,10 @@ void sym_vec_matvec(const MatvecArgs& a, const PackedPoints& pts, const float* V
     ws.tile_calls += 1;
   }
   hipLaunchKernelGGL(k_sym_vec_reduce, dim3((unsigned)ceil_div(n, kVecRedPts), (unsigned)nc),
-                     dim3(kVecRedPts * kVecRedGroups), 0, st, fwd, (int)splits, tp, nc, npad, nb, hmax, n, a.outputscale, a.noise, vp,
-                     outc);
+                     dim3(kVecRedPts * kVecRedGroups), 0, st, fwd, (int)splits, tp, nc, npad, nb,
+                     hmax, n, a.outputscale, a.noise, vp, outc);
   MGP_HIP_CHECK(hipGetLastError());
+  return true;
 }
 
 // out = (K + noise I) V for nc <= 16 columns of V on the symmetric kernel.
@@ -2907,11 +2910,11 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
     float* outc = out_dev + (int64_t)c0 * a.m;
     const float* Vin = a.square ? V_dev + (int64_t)c0 * a.m : nullptr;
     if (force_splits <= 0 && sym_route(a, rows, cols, nc, ws)) {
-      if (nc <= kSymVecCols)
-        sym_vec_matvec(a, rows, Vc, nc, outc, ws, st);
-      else
+      if (nc > kSymVecCols) {
         sym_matvec(a, rows, Vc, nc, outc, ws, st);
-      continue;
+        continue;
+      }
+      if (sym_vec_matvec(a, rows, Vc, nc, outc, ws, st)) continue;
     }
 
     // Pack right-hand sides (or take the packing a previous product of the

@@ -125,6 +125,23 @@ struct DevBuf {
     }
     return ptr;
   }
+  // The same, or null where the device has no memory left for it (the buffer
+  // is then empty), for a caller that can do with less.
+  T* try_ensure(size_t n) {
+    if (n == 0) n = 1;
+    if (n > count) {
+      release();
+      const hipError_t e = hipMalloc(reinterpret_cast<void**>(&ptr), n * sizeof(T));
+      if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        ptr = nullptr;
+        return nullptr;
+      }
+      MGP_HIP_CHECK(e);
+      count = n;
+    }
+    return ptr;
+  }
 };
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }

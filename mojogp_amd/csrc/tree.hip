@@ -366,8 +366,9 @@ constexpr int64_t kTreeSymMin = 5000;
 constexpr int kTreeSymMinCols = 5;
 constexpr double kTreeSymMaxBytes = 8e9;
 
-// out = (K + noise I) V for nc <= 16 columns on the symmetric kernel.
-void tree_sym_matvec(const KernelTree& t, const float* p_dev, const float* X, int64_t n,
+// out = (K + noise I) V for nc <= 16 columns on the symmetric kernel.  False,
+// with nothing launched, where its partial sums do not fit the device.
+bool tree_sym_matvec(const KernelTree& t, const float* p_dev, const float* X, int64_t n,
                      const float* V, int nc, float noise, float* out, DevBuf<float>& work,
                      hipStream_t st) {
   const TreeSymJitKernel jk = tree_sym_jit_kernel(t);
@@ -392,7 +393,8 @@ void tree_sym_matvec(const KernelTree& t, const float* p_dev, const float* X, in
   }
   long long nn = n, nbb = nb, sp = best, sps = ceil_div(stages, best), hm = hmax;
   const size_t nf = (size_t)best * 16 * nb * jk.block;
-  float* fwd = work.ensure(nf + (size_t)std::max<int64_t>(nb * hmax, 1) * jk.block * 16);
+  float* fwd = work.try_ensure(nf + (size_t)std::max<int64_t>(nb * hmax, 1) * jk.block * 16);
+  if (fwd == nullptr) return false;
   float* tp = fwd + nf;
   int ncc = nc;
   void* args[] = {(void*)&X, &nn, (void*)&p_dev, (void*)&V, &ncc, &nbb, &sp, &sps, &hm,
@@ -402,6 +404,7 @@ void tree_sym_matvec(const KernelTree& t, const float* p_dev, const float* X, in
   hipLaunchKernelGGL(k_tree_sym_reduce, dim3((unsigned)ceil_div(4 * n, 256)), dim3(256), 0, st, fwd,
                      (int)best, tp, jk.block, nb, hmax, n, nc, noise, V, out);
   MGP_HIP_CHECK(hipGetLastError());
+  return true;
 }
 
 bool tree_sym_route(const KernelTree& t, int64_t m, int64_t n, int nc, bool square) {
@@ -425,11 +428,10 @@ void tree_matvec(const KernelTree& t, const float* p_dev, const float* Xr, int64
       1, std::min<int64_t>(ceil_div(2048, rows), tiles));
   for (int c0 = 0; c0 < ncols; c0 += kMaxCols) {
     const int nc = std::min(kMaxCols, ncols - c0);
-    if (Xr == Xc && tree_sym_route(t, m, n, nc, square)) {
-      tree_sym_matvec(t, p_dev, Xc, n, V + (int64_t)c0 * n, nc, noise, out + (int64_t)c0 * n, work,
-                      st);
+    if (Xr == Xc && tree_sym_route(t, m, n, nc, square) &&
+        tree_sym_matvec(t, p_dev, Xc, n, V + (int64_t)c0 * n, nc, noise, out + (int64_t)c0 * n,
+                        work, st))
       continue;
-    }
     float* part = work.ensure((size_t)splits * nc * m);
     // the tree's straight-line kernel (tree_jit.hip)
     const TreeJitKernel jk = tree_jit_kernel(t, nc);
