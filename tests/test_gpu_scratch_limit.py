@@ -2,12 +2,15 @@
 memory run on their one-sided kernel, which needs little, with its results to
 the bit; the next product with memory at hand is symmetric again."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from mojogp_amd import RBF, RQ, Periodic
 from mojogp_amd._provider import NativeProvider
 from oracle import kernels as ok
+from test_zz_no_alloc import _Dev, _hip
 
 pytestmark = pytest.mark.gpu
 
@@ -28,7 +31,7 @@ def _provider(route, X):
 
 
 def test_falls_back(monkeypatch):
-    import torch
+    hip = _hip()  # (the runtime that the library runs on)
     held = []
     for route, n, t in CASES:
         rng = np.random.default_rng(n)
@@ -38,17 +41,17 @@ def test_falls_back(monkeypatch):
         monkeypatch.setenv("MGP_SYM_MATVEC", "0")
         one = [p.forward_matvec(V) for _, p, V in held]
         monkeypatch.delenv("MGP_SYM_MATVEC")
-        torch.cuda.synchronize()
-        hold = torch.empty(max(torch.cuda.mem_get_info()[0] - LEFT, 1), dtype=torch.uint8,
-                           device="cuda")
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipDeviceSynchronize() == 0
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        hold = _Dev(hip, free.value - LEFT)
         got = []
         try:
             for route, p, V in held:
                 print(route, flush=True)
                 got.append(p.forward_matvec(V))
         finally:
-            del hold
-            torch.cuda.empty_cache()
+            hold.free()
         sym = [p.forward_matvec(V) for _, p, V in held]
     finally:
         for _, p, _ in held:
