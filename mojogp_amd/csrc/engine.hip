@@ -1450,6 +1450,11 @@ void exact_variance(Provider& pv, int64_t m, const ExactVarianceOptions& o, floa
   MGP_HIP_CHECK(hipStreamSynchronize(st));
 }
 
+// K(Xs, X) S of the LOVE variance ([rank][m] floats) stays with the provider up
+// to 64 MB (rank 200: 80000 points); an allocation (~0.1 ms) is nothing beside a
+// larger one's time.
+constexpr size_t kLoveKeep = (size_t)16 << 20;
+
 void predict_from_state(Provider& pv, const PredictState& ps, const float* Xs_host, int64_t m,
                         float mean, int variance_method, float* mean_out, float* var_out,
                         PredictTimes& t, const ExactVarianceOptions* exact,
@@ -1478,6 +1483,7 @@ void predict_from_state(Provider& pv, const PredictState& ps, const float* Xs_ho
     love_variance(Vs, m, ps.rank, pv.kdiag(), var, st, dv);
     MGP_HIP_CHECK(hipMemcpyAsync(var_out, var, m * sizeof(float), hipMemcpyDeviceToHost, st));
     MGP_HIP_CHECK(hipStreamSynchronize(st));
+    if (pv.love_v.count > kLoveKeep) pv.love_v.release();
     t.variance_s = secs_since(t1);
   } else if (variance_method == 2) {
     auto t1 = Clock::now();
