@@ -362,11 +362,10 @@ int mgp_prepare_prediction_cache(void* handle, const float* y, const mgp_predict
       c->variance_method = opts->variance_method;
       c->exact = exact_options(*opts);
       prepare_state(*pv, y, *opts, alpha_in, nullptr, c->state, info);
-      // every prediction from this cache multiplies by the root
-      if (c->state.rank > 0 && !pv->is_tree && pv->train.kb >= 1) {
+      // every prediction from this cache multiplies by the root, on the tile
+      // route where the training points allow it
+      if (c->state.rank > 0 && !pv->is_tree && gram_form_ok(pv->kind, pv->train, pv->train))
         pack_rhs(pv->train, c->state.root.ptr, c->state.rank, c->state.root_pack, pv->st);
-        MGP_HIP_CHECK(hipStreamSynchronize(pv->st));
-      }
     } catch (...) {
       delete c;
       throw;

@@ -118,8 +118,9 @@ struct RhsPack {
   DevBuf<float> data;          // fp16 parts of every chunk
   std::vector<size_t> offset;  // first float of each chunk
   DevBuf<uint32_t> colmax;     // [chunks][64]
-  DevBuf<uint32_t> parts;      // scratch of the packing
 };
+// Waits for the stream; leaves out empty (ncols 0: products pack for themselves)
+// where the device has no memory for a second copy of V.
 void pack_rhs(const PackedPoints& cols, const float* V, int ncols, RhsPack& out,
               hipStream_t st);
 

@@ -2521,16 +2521,21 @@ void pack_rhs(const PackedPoints& cols, const float* V, int ncols, RhsPack& out,
     out.offset.push_back(total);
     total += (size_t)rhs_groups(std::min(64, ncols - c0)) * col_pairs * 64 * 2 * 4;
   }
-  out.data.ensure(total);
-  out.colmax.ensure(64 * out.offset.size());
-  out.parts.ensure((size_t)64 * absmax_chunks(cols.n));
+  DevBuf<uint32_t> parts;
+  if (out.data.try_ensure(total) == nullptr ||
+      out.colmax.try_ensure(64 * out.offset.size()) == nullptr ||
+      parts.try_ensure((size_t)64 * absmax_chunks(cols.n)) == nullptr) {
+    out.data.release();
+    return;
+  }
   for (int c0 = 0; c0 < ncols; c0 += 64) {
     const int nc = std::min(64, ncols - c0), ncg = rhs_groups(nc);
     if (ncg == 0) continue;  // one column left over: packed by each product
-    launch_pack_rhs(V + (int64_t)c0 * cols.n, cols.n, nc, ncg, col_pairs, out.parts.ptr,
+    launch_pack_rhs(V + (int64_t)c0 * cols.n, cols.n, nc, ncg, col_pairs, parts.ptr,
                     out.colmax.ptr + c0, reinterpret_cast<h8*>(out.data.ptr + out.offset[c0 / 64]),
                     st);
   }
+  MGP_HIP_CHECK(hipStreamSynchronize(st));  // parts is released on return
   out.col_tiles = cols.ntiles;
   out.ncols = ncols;
 }

@@ -48,3 +48,19 @@ def test_large_test_set_is_not_kept():
         m.destroy_provider(info)
     assert np.array_equal(small["variance"], again["variance"])
     assert np.abs(large["variance"][::1000] - small["variance"]).max() <= 1e-5
+
+
+@pytest.mark.parametrize("kind,copies", [("matern52", 2), ("matern12", 1)])
+def test_root_is_packed_where_it_is_read(kind, copies):
+    """A cache holds alpha, the root and, where predictions take the tile route,
+    the root's packing (the difference products never read one)."""
+    n, rank = 100_000, 64  # the root: 26 MB
+    m, info, cache, params = _cache(kind, n, rank)
+    try:
+        held = -_free()
+        load_engine().destroy_prediction_cache(cache)
+        held += _free()
+    finally:
+        m.destroy_provider(info)
+    print(kind, held / (4.0 * n * rank), "roots", flush=True)
+    assert copies * 0.9 <= held / (4.0 * n * rank) <= copies + 0.2
