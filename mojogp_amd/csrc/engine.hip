@@ -1213,6 +1213,13 @@ int solve_columns(const CGOperator& op, const float* B, int C, int max_iter, flo
 
 namespace {
 
+// Iterations between looks at the breakdown flag: 4 from this many points on,
+// 16 below.  A look idles the device for ~20 us (rank 100, n = 65536: 111 ms
+// with one in 16 iterations, 113.6 with one in each), a missed breakdown costs a
+// product an iteration (equal points, rank 16, which breaks down at the second:
+// 14.3 ms and 4.5 ms).
+constexpr int64_t kLanczosLookMin = 65536;
+
 // Lanczos on K + noise I from the deterministic +-1 start vector
 // (compute_lanczos_inv_root_jit, jit_prediction.mojo:974-1177), one iteration
 // per step() after the caller has formed w = A v_j (w may live in a caller's
@@ -1221,7 +1228,7 @@ struct LanczosSolve {
   Provider& pv;
   int64_t n;
   hipStream_t st;
-  int r, nb, nbd;
+  int r, nb, nbd, look;
   DevBuf<float> Q, wbuf, ab;
   DevBuf<double> part, coef;
   DevBuf<int> stop;
@@ -1233,7 +1240,7 @@ struct LanczosSolve {
 
   LanczosSolve(Provider& pv_, int r_, float* w_ext = nullptr, float* v_ext = nullptr)
       : pv(pv_), n(pv_.n), st(pv_.st), r(r_), nb(cg_chunks(pv_.n)), nbd(reduction_chunks(pv_.n)),
-        vnext(v_ext) {
+        look(pv_.n >= kLanczosLookMin ? 3 : 15), vnext(v_ext) {
     MGP_REQUIRE(r >= 1 && r <= 1000, "Lanczos rank must be in [1, 1000]");
     Q.ensure((size_t)r * n);
     w = w_ext ? w_ext : wbuf.ensure(n);
@@ -1290,9 +1297,9 @@ struct LanczosSolve {
     hipLaunchKernelGGL(k_lz_next, g1(n), blk, 0, st, w, part.ptr, nb, j, r, ab.ptr, stop.ptr,
                        j + 1 < r ? Q.ptr + (size_t)(j + 1) * n : nullptr, vnext, n);
     MGP_HIP_CHECK(hipGetLastError());
-    // a breakdown leaves the remaining Q columns zero; looked for now and
-    // then, its later iterations do nothing
-    if ((j & 15) == 15) {
+    // a breakdown leaves the remaining Q columns zero and its later iterations
+    // do nothing but form the caller's product
+    if ((j & look) == look) {
       int sh = 0;
       MGP_HIP_CHECK(hipMemcpyAsync(&sh, stop.ptr, sizeof(int), hipMemcpyDeviceToHost, st));
       MGP_HIP_CHECK(hipStreamSynchronize(st));

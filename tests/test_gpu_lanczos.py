@@ -13,7 +13,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [600, 2000, 5100, 8000, 30000])
+@pytest.mark.parametrize("n", [600, 2000, 5100, 8000, 30000, 65536])
 def test_lanczos_breakdown(n):
     from mojogp_amd._engine import load_engine, load_kernel_module
     X = np.full((n, 2), 0.5, np.float32)
