@@ -357,12 +357,26 @@ double tree_diag(const KernelTree& t, const float* params) {
 }
 
 namespace {
-// Square products with 5 to 16 right-hand sides from this many points on run
-// on the symmetric kernel (RBF x periodic + RQ, d = 6, 16 columns, us
-// one-sided / symmetric: 61 / 66 at n = 4096, 85 / 73 at 5000, 226 / 172 at
-// 10000, 738 / 522 at 20000; below, too few block pairs fill the chip); a model
-// of this size repays its compilation, as for the gradient kernel.
-constexpr int64_t kTreeSymMin = 5000;
+// Cost of one pair's value in units of a dimension's part of it: a leaf's
+// exponential and the like weigh about five.
+int tree_cost(const KernelTree& t) {
+  int c = 0;
+  for (int l = 0; l < t.nleaves; ++l) c += 5 + t.leaf[l].ndim;
+  return c;
+}
+
+// Square products with 5 to 16 right-hand sides run on the symmetric kernel
+// where n + 100 tree_cost >= 8600: below, the blocks fill too few rounds of the
+// chip, the dearer a value the earlier half of them pays (11 columns, one-sided
+// / symmetric us: RQ in 1 dimension, cost 6, n = 7500 77 / 75, 8000 85 / 74,
+// 16000 206 / 173; RBF + Matern-5/2 in 1, cost 12, 7000 95 / 89, 8000 113 / 92;
+// RBF x periodic + RQ in 4, cost 24, 5500 83 / 81, 6000 89 / 87, 6500 102 / 88,
+// 20000 600 / 458; four leaves in 4, cost 33, 5000 103 / 85).
+// Compilation takes 0.14 s the first time (later processes read the runtime's
+// disk cache, ~5 ms), in place of the one-sided kernels' 0.21 s for a fit (11
+// columns throughout), beside it once predictions need those too; a fit of 100
+// steps of up to 100 iterations saves that from about this line on.
+constexpr int64_t kTreeSymBase = 8600, kTreeSymPerCost = 100;
 constexpr int kTreeSymMinCols = 5;
 constexpr double kTreeSymMaxBytes = 8e9;
 
@@ -412,7 +426,7 @@ bool tree_sym_route(const KernelTree& t, int64_t m, int64_t n, int nc, bool squa
   if ((double)n * (double)n * 16 * 4 / 512 > kTreeSymMaxBytes) return false;
   const int mode = sym_switch();
   if (mode >= 0) return mode == 1;
-  return n >= kTreeSymMin && nc >= kTreeSymMinCols;
+  return n + kTreeSymPerCost * tree_cost(t) >= kTreeSymBase && nc >= kTreeSymMinCols;
 }
 }  // namespace
 
@@ -490,13 +504,16 @@ int64_t grad_splits(int64_t n) {
   return std::max<int64_t>(1, std::min<int64_t>(ceil_div(2048, rows), ceil_div(n, 64)));
 }
 
-// Points from which the trace runs on the tree's generated kernel (RBF x
-// periodic + RQ, 11 factor columns: 0.13 ms generated and 0.78 ms interpreted
-// at n = 4096, 0.22 and 7.5 ms at n = 10007, where the interpreted one was
-// measured with the old splits): a model of this size trains for seconds, in
-// which one compilation (~0.5 s per tree and process) is repaid.  Below, and
-// for trees whose leaves share parameter slots, the interpreted kernel.
-constexpr int64_t kTreeGradJitMin = 4096;
+// The trace runs on the tree's generated kernel where n^2 tree_cost reaches
+// this: its compilation takes 0.15 s the first time, and a trace is
+// ~0.165 ms (n / 10000)^2 tree_cost shorter than the interpreted one, so from
+// here on a fit of 100 steps (the default) in a fresh process repays it (11
+// factor columns, interpreted / generated ms: RQ in 1 dimension, cost 6, n =
+// 12000 1.48 / 0.18; RBF + Matern-5/2 in 1, cost 12, 8000 1.27 / 0.13, 9000 1.67
+// / 0.15; RBF x periodic + RQ in 4, cost 24, 6000 1.90 / 0.13, 10000 4.41 /
+// 0.22; four leaves in 4, cost 33, 5000 1.62 / 0.14).  Below, and for trees
+// whose leaves share parameter slots, the interpreted kernel.
+constexpr double kTreeGradJitWork = 9e8;
 }  // namespace
 
 void tree_cat_grad_tables(const KernelTree& t, const float* p_dev, const float* X, int64_t n,
@@ -525,7 +542,7 @@ void tree_grad_traces(const KernelTree& t, const float* p_dev, const float* X, i
                       DevBuf<double>& work, hipStream_t st) {
   const int P = t.nparams;
   TreeGradJitKernel jk;
-  if (n >= kTreeGradJitMin) jk = tree_grad_jit_kernel(t);
+  if ((double)n * (double)n * tree_cost(t) >= kTreeGradJitWork) jk = tree_grad_jit_kernel(t);
   int64_t rows = ceil_div(n, 256), splits = grad_splits(n), dps = 0;
   if (jk.fn) {
     rows = ceil_div(n, (int64_t)jk.block);

@@ -1,5 +1,5 @@
-"""Gradient traces of kernel trees on their generated kernel (n >= 4096) and
-on the interpreted one just below, against the float64 tree restatement:
+"""Gradient traces of kernel trees on their generated kernel (from 5500 to 7500
+points on for these trees) and on the interpreted one below, against the float64 tree restatement:
 every leaf kind, isotropic and ARD, shared subtrees' adjoints, a categorical
 leaf (tables need not be symmetric, so no pair is folded), ragged last blocks
 and 1 .. 17 factor columns.
@@ -42,7 +42,7 @@ def _check(T, X, params, L, R, got):
 
 
 @pytest.mark.parametrize("name", list(TREES))
-@pytest.mark.parametrize("n,t", [(700, 17), (4095, 3), (4096, 1), (4227, 17)])
+@pytest.mark.parametrize("n,t", [(700, 17), (4095, 3), (4096, 1), (4227, 17), (7555, 17)])
 def test_traces_match_oracle(name, n, t):
     mk, d = TREES[name]
     node = mk()
@@ -62,11 +62,12 @@ def test_traces_match_oracle(name, n, t):
     _check(T, X, params, L, R, got)
 
 
-def test_categorical_tree_is_not_folded():
+@pytest.mark.parametrize("n", [4100, 8700])
+def test_categorical_tree_is_not_folded(n):
     import ctypes as C
     from mojogp_amd import _lib
     rng = np.random.default_rng(5)
-    n, t, levels = 4100, 6, 4
+    t, levels = 6, 4
     X = np.stack([rng.uniform(-2, 2, n), rng.integers(0, levels, n)], axis=1).astype(np.float32)
     node = RBF(active_dims=[0]) * GD(levels, active_dims=[1])
     table = rng.uniform(0.2, 1.0, size=(levels, levels)).astype(np.float32)  # not symmetric

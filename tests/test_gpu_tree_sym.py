@@ -1,7 +1,8 @@
 """Symmetric generated products of kernel trees (square, 5 .. 16 right-hand
-sides, n >= 5000) at the edges of their 256-point blocks and 64-column stages
-(even and odd block counts, ragged last block), beside column chunks that stay
-on the one-sided kernel, against the float64 tree restatement on sampled rows;
+sides, from 5800 to 6500 points on for these trees) at the edges of their
+256-point blocks and 64-column stages (even and odd block counts, ragged last
+block), beside column chunks and sizes that stay on the one-sided kernel,
+against the float64 tree restatement on sampled rows;
 a tree with a correlation table keeps the one-sided kernel.
 
 Bound: a value carries the hardware exp / sin / log error and an exponent
@@ -44,7 +45,8 @@ def _run(node, T, d, X, V, params, tables=None):
 
 
 @pytest.mark.parametrize("name", list(TREES))
-@pytest.mark.parametrize("n,t", [(4999, 11), (5000, 5), (5121, 16), (5376, 21), (5503, 17)])
+@pytest.mark.parametrize("n,t", [(4999, 11), (5000, 5), (5121, 16), (5376, 21), (5503, 17), (6500, 5),
+                                 (6657, 11), (6912, 16), (7039, 21)])
 def test_products_match_oracle(name, n, t):
     mk, d = TREES[name]
     node = mk()
