@@ -85,3 +85,39 @@ def test_converged_quadratic_form():
     yc = y.astype(np.float64) - np.float32(0.1)
     want = yc @ np.linalg.solve(K, yc)
     assert abs(a[1] - want) <= 2e-5 * want
+
+
+@pytest.mark.parametrize("n", [777, 4500])
+def test_column_without_a_direction(n):
+    """Targets equal to the mean leave the first column zero: p.Ap = 0, so it
+    keeps x = 0 (no step, no NaN) while the probes go on, as on the general path."""
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(n, 2)).astype(np.float32)
+    y = np.full(n, np.float32(0.1))
+    p = NativeProvider(ok.RBF, False, X, np.array([0.8, 1.1], np.float32), 0.4)
+    try:
+        a, ga, ia = _bbmm(p, y, 6, 4, False)
+        b, gb, ib = _bbmm(p, y, 6, 4, True)
+    finally:
+        p.close()
+    assert ia == ib and a[1] == 0.0 and b[1] == 0.0
+    assert np.isfinite(a).all() and np.isfinite(ga).all()
+    assert np.allclose(a, b, rtol=2e-5)
+    assert np.linalg.norm(ga - gb) <= 1e-3 * np.linalg.norm(gb)
+
+
+def test_columns_that_stop_moving():
+    """A system solved to rounding long before the last iteration: residuals reach
+    the noise floor, where steps are skipped or shrink, and the solution stays."""
+    rng = np.random.default_rng(8)
+    n = 900
+    X = rng.normal(size=(n, 1)).astype(np.float32)
+    y = rng.normal(size=n).astype(np.float32)
+    p = NativeProvider(ok.RBF, False, X, np.array([0.6, 1.0], np.float32), 2.0)
+    try:
+        a, ga, _ = _bbmm(p, y, 5, 40, False)
+        b, gb, _ = _bbmm(p, y, 5, 400, False)
+    finally:
+        p.close()
+    assert np.isfinite(b).all() and np.isfinite(gb).all()
+    assert abs(a[1] - b[1]) <= 2e-5 * abs(a[1])

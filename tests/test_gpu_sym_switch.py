@@ -95,3 +95,31 @@ def test_off_above_the_automatic_line(monkeypatch, kind):
         p.close()
     assert np.array_equal(sym, auto) and not np.array_equal(one, sym)
     assert _rms(sym, one) <= 2e-6
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("route,n,t", [("difference", 700, 7), ("tree", 700, 16), ("one", 700, 1),
+                                       ("two", 5003, 2)])
+def test_one_bad_entry_stays_in_its_column(monkeypatch, route, n, t, bad):
+    """An infinity or NaN in a right-hand side: its column is not finite where the
+    one-sided kernel's is not, the other columns keep their bits."""
+    rng = np.random.default_rng(n + t)
+    X = rng.uniform(-1, 1, size=(n, 2)).astype(np.float32)
+    V = rng.normal(size=(t, n)).astype(np.float32)
+    if route == "tree":
+        node = RBF() * Periodic(active_dims=[0]) + RQ()
+        p = NativeProvider(None, False, X, np.linspace(0.9, 1.4, 8).astype(np.float32), 0.1,
+                           tree_spec=node.to_tree_spec(2))
+    else:
+        kind = ok.MATERN12 if route == "difference" else ok.MATERN52
+        p = NativeProvider(kind, False, X, np.array([1.0, 1.0], np.float32), 0.1)
+    W = V.copy()
+    W[t - 1, n // 3] = bad
+    try:
+        _, clean, _ = _both(monkeypatch, p, V)
+        one, sym, _ = _both(monkeypatch, p, W)
+    finally:
+        p.close()
+    assert np.array_equal(clean[:t - 1], sym[:t - 1])
+    assert np.array_equal(np.isfinite(one[t - 1]), np.isfinite(sym[t - 1]))
+    assert not np.isfinite(sym[t - 1]).any()

@@ -31,14 +31,22 @@ TREES = {
 
 def _check(T, X, params, L, R, got):
     ref, mag = np.zeros(T.nparams), np.zeros(T.nparams)
-    for i in range(0, len(X), 256):
-        G = T.gradients(X[i:i + 256], X, params)
-        W = L[:, i:i + 256].astype(np.float64).T @ R.astype(np.float64)
+    rows = np.flatnonzero(L.any(axis=0))  # the others' terms are zero
+    for i in range(0, len(rows), 256):
+        at = rows[i:i + 256]
+        G = T.gradients(X[at], X, params)
+        W = L[:, at].astype(np.float64).T @ R.astype(np.float64)
         ref += (G * W).sum(axis=(1, 2))
         mag += np.abs(G * W).sum(axis=(1, 2))
     err = np.abs(got - ref)
     print("  error / bound", np.round(err / np.maximum(80 * 2.0**-24 * mag, 1e-300), 4), flush=True)
     assert np.all(err <= 80 * 2.0**-24 * mag)
+
+
+def _unused(rng, n):
+    """Rows left without weight where the restatement of all would take long:
+    all but 400 and the last 40."""
+    return np.setdiff1d(np.arange(n - 40), rng.choice(n - 40, 400, replace=False))
 
 
 @pytest.mark.parametrize("name", list(TREES))
@@ -53,6 +61,8 @@ def test_traces_match_oracle(name, n, t):
     if "poly" in name:
         params = node.to_engine_params(node.get_initial_params()).astype(np.float32)
     L, R = (rng.normal(size=(t, n)).astype(np.float32) for _ in range(2))
+    if n > 5000:
+        L[:, _unused(rng, n)] = 0.0
     print(f"tree trace {name} n={n} t={t}", flush=True)
     p = NativeProvider(None, False, X, params, 0.2, tree_spec=node.to_tree_spec(d))
     try:
@@ -105,3 +115,50 @@ def test_parameter_factors_are_not_rounded(n):
         assert np.all(np.abs(got[[1, 4]] - want) <= 1e-12 * want)
     else:
         assert np.all(np.abs(got[[1, 4]] - want) <= 16 * 2.0**-24 * want)
+
+
+def test_many_parameters():
+    """46 parameters: the generated kernel keeps two sums of each per lane, some
+    of them in scratch memory."""
+    d, n, t = 10, 4001, 5
+    node = make_ard_kernel((RBF(ard=True) + RQ(ard=True)) * Periodic(period=2.0, ard=True)
+                           + Matern52(ard=True), d)
+    rng = np.random.default_rng(7)
+    X = rng.uniform(-2, 2, size=(n, d)).astype(np.float32)
+    T = ok.TreeKernel(node.to_dict(), d)
+    assert T.nparams == 46
+    params = rng.uniform(2.0, 5.0, T.nparams).astype(np.float32)
+    L, R = (rng.normal(size=(t, n)).astype(np.float32) for _ in range(2))
+    L[:, _unused(rng, n)] = 0.0
+    p = NativeProvider(None, False, X, params, 0.2, tree_spec=node.to_tree_spec(d))
+    try:
+        got = p.gradient_trace(L, R)
+    finally:
+        p.close()
+    _check(T, X, params, L, R, got)
+
+
+def test_shared_parameter_slots():
+    """Two leaves that read the same lengthscale and outputscale: no generated
+    kernel, and the trace is the sum of the leaves' own."""
+    n, t = 7200, 4
+    rng = np.random.default_rng(11)
+    X = rng.uniform(-2, 2, size=(n, 4)).astype(np.float32)
+    L, R = (rng.normal(size=(t, n)).astype(np.float32) for _ in range(2))
+    spec = list((RBF() + Matern52()).to_tree_spec(4))
+    both = np.array([0.9, 1.3], np.float32)
+    got = []
+    for shared in (True, False):
+        s = list(spec)
+        if shared:
+            assert s[1] == 4 and s[15] == 2  # parameters; the second leaf's first one
+            s[1], s[15] = 2, 0
+        p = NativeProvider(None, False, X, both if shared else np.tile(both, 2), 0.2, tree_spec=s)
+        try:
+            got.append(p.gradient_trace(L, R))
+        finally:
+            p.close()
+    want = got[1][:2] + got[1][2:]
+    mag = np.abs(L).sum() * np.abs(R).sum() / n**2  # mean |w|, up to the columns' signs
+    print(got[0], want, flush=True)
+    assert np.all(np.abs(got[0] - want) <= 80 * 2.0**-24 * mag * n * n)
