@@ -2601,16 +2601,18 @@ SymFn pick_sym(int kb) {
   return nullptr;
 }
 
-// Delta splits of the symmetric kernels (k_sym_tile, k_grad_sym).  They run
-// one workgroup per CU; item L of the grid goes to XCD L / per (launch order
-// deals workgroups to the XCDs in turn), and each XCD's CUs take its items in
-// order as they free up.  A partly filled last round of items leaves CUs idle
+// Delta splits of the symmetric kernels (k_sym_tile, k_grad_sym, k_sym_vec).
+// Item L of the grid goes to XCD L / per (launch order deals workgroups to the
+// XCDs in turn), and each XCD's CUs, with as many workgroups as fit, take its
+// items in order as they free up.  A partly filled last round of items leaves CUs idle
 // for up to one item, so the split count is chosen by simulating that
 // dispatch: an item costs `stages` per delta plus about one stage of set-up
 // (fitted to measured k_sym_tile launches at nb = 489: 5, 9, 12 and 35
 // splits gave 3.81 to 3.87 us per simulated stage), and each split's partial
 // sums (`split_bytes`) cost their extra read in the reduction (priced at 2 us
-// per stage, a short stage, so the choice leans towards fewer splits).
+// per stage, a short stage, so the choice leans towards fewer splits; not
+// fitted for k_sym_vec, one of whose splits is priced below 1/100 of a stage up
+// to 30000 points whatever a stage takes).
 // Cached per kernel, block count and device.
 // granule: pieces into which a delta may be cut (1: whole deltas); the count
 // returned is for ranges of ceil((hmax + 1) granule / splits) pieces.
