@@ -187,7 +187,12 @@ void fused_matvec(const MatvecArgs& a, const PackedPoints& rows,
                   MatvecWorkspace& ws, hipStream_t st, int force_splits = 0);
 constexpr int64_t kSymMinBlocks = 48;
 // One and two right-hand sides run on the symmetric VALU product (k_sym_vec)
-// from this many points on.
+// from this many points on: below, the CG of small systems (SmallCg) needs the
+// one-sided form and the two are within 3 us of each other (us a call, one-sided
+// / symmetric, one column: Matern-5/2 in 6 dimensions n = 2000 22.6 / 22.3, 4000
+// 28.0 / 26.1, 5000 30.6 / 28.0, 10000 50.9 / 43.9, 20000 135 / 101, 40000 445 /
+// 308; RBF in 2 5000 28.0 / 27.0, 20000 99 / 81; two columns, Matern-5/2 5000
+// 37.7 / 30.5, 20000 170 / 124).
 constexpr int kSymVecCols = 2;
 constexpr int64_t kSymVecMinPoints = 5000;
 // True when a square product of the packed points with ncols right-hand
