@@ -366,7 +366,8 @@ int tree_cost(const KernelTree& t) {
 }
 
 // Square products with 5 to 16 right-hand sides run on the symmetric kernel
-// where n + 100 tree_cost >= 8600: below, the blocks fill too few rounds of the
+// where n + 100 tree_cost >= 8600 (and n >= 5000, the smallest size at which a
+// costly tree gained clearly): below, the blocks fill too few rounds of the
 // chip, the dearer a value the earlier half of them pays (11 columns, one-sided
 // / symmetric us: RQ in 1 dimension, cost 6, n = 7500 77 / 75, 8000 85 / 74,
 // 16000 206 / 173; RBF + Matern-5/2 in 1, cost 12, 7000 95 / 89, 8000 113 / 92;
@@ -376,7 +377,7 @@ int tree_cost(const KernelTree& t) {
 // disk cache, ~5 ms), in place of the one-sided kernels' 0.21 s for a fit (11
 // columns throughout), beside it once predictions need those too; a fit of 100
 // steps of up to 100 iterations saves that from about this line on.
-constexpr int64_t kTreeSymBase = 8600, kTreeSymPerCost = 100;
+constexpr int64_t kTreeSymMin = 5000, kTreeSymBase = 8600, kTreeSymPerCost = 100;
 constexpr int kTreeSymMinCols = 5;
 constexpr double kTreeSymMaxBytes = 8e9;
 
@@ -426,7 +427,8 @@ bool tree_sym_route(const KernelTree& t, int64_t m, int64_t n, int nc, bool squa
   if ((double)n * (double)n * 16 * 4 / 512 > kTreeSymMaxBytes) return false;
   const int mode = sym_switch();
   if (mode >= 0) return mode == 1;
-  return n + kTreeSymPerCost * tree_cost(t) >= kTreeSymBase && nc >= kTreeSymMinCols;
+  return n >= kTreeSymMin && n + kTreeSymPerCost * tree_cost(t) >= kTreeSymBase &&
+         nc >= kTreeSymMinCols;
 }
 }  // namespace
 

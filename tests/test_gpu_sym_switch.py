@@ -12,7 +12,7 @@ of the partial sums, at most a few per entry.  Trees: fp32 sums over at most
 import numpy as np
 import pytest
 
-from mojogp_amd import RBF, RQ, Linear, Periodic, Polynomial
+from mojogp_amd import RBF, RQ, Linear, Matern52, Periodic, Polynomial, make_ard_kernel
 from mojogp_amd._provider import NativeProvider
 from oracle import kernels as ok
 
@@ -95,6 +95,24 @@ def test_off_above_the_automatic_line(monkeypatch, kind):
         p.close()
     assert np.array_equal(sym, auto) and not np.array_equal(one, sym)
     assert _rms(sym, one) <= 2e-6
+
+
+@pytest.mark.parametrize("n", [900, 4999, 5000])
+def test_costly_trees_have_a_smallest_size(monkeypatch, n):
+    """The dearer a tree's values the earlier it goes symmetric, but not below 5000
+    points, where blocks are too few."""
+    d = 10
+    node = make_ard_kernel((RBF(ard=True) + RQ(ard=True)) * Periodic(period=2.0, ard=True)
+                           + Matern52(ard=True), d)
+    rng = np.random.default_rng(n)
+    X = rng.uniform(-1, 1, size=(n, d)).astype(np.float32)
+    params = rng.uniform(2.0, 5.0, 46).astype(np.float32)
+    p = NativeProvider(None, False, X, params, 0.1, tree_spec=node.to_tree_spec(d))
+    try:
+        one, sym, auto = _both(monkeypatch, p, rng.normal(size=(6, n)).astype(np.float32))
+    finally:
+        p.close()
+    assert np.array_equal(auto, one if n < 5000 else sym)
 
 
 @pytest.mark.parametrize("bad", [np.inf, np.nan])
